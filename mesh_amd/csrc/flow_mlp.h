@@ -207,6 +207,209 @@ template <int NI, bool FAST = false, bool SY = true> __device__ void mlp_forward
 	wave_sync();
 }
 
+// ---- the MLP on one wavefront with the activations in registers -----------
+//
+// A 16-row tile is computed transposed, Y^T = W^T X^T: the weights are the
+// MFMA's A operand (lane l: output column l % 16 of a block), the activations
+// its B operand (lane l: row l % 16).  The product leaves row l % 16's columns
+// 16 b + 4 (l / 16) + j in acc[b][j] of lane l, and the next layer takes its
+// contraction index in just that order -- step (b, j) contracts the columns
+// 16 b + 4 q + j, q = 0..3, one per quarter of the wavefront -- so every lane
+// already holds the B operand of the next product and no activation goes
+// through LDS.  (With the tile's activations in LDS, rows 64 floats apart,
+// the 16 rows of an A operand fell on one bank and each product read them
+// again for each block of columns.)  Only the weights are read from LDS, each
+// once per tile: rows padded to WS (W3S) floats, 4 WS = 16 (mod 64), put the
+// four quarters of a read on different banks.
+constexpr int WS = NH + 4;  // row stride of W1 and W2
+constexpr int W3S = 20;     // row stride of W3 (columns NO..15 zero)
+constexpr int YS = 20;      // row stride of a tile's outputs
+
+// LDS image of one layer's weights
+template <int NI> struct alignas(16) LWP
+{
+	float w1[NI * WS], b1[NH], w2[NH * WS], b2[NH], w3[NH * W3S], b3[16];
+};
+
+// One layer's parameters held in registers (two floats a lane per chunk) so
+// that the next layer's global loads overlap the current layer's work; NP is
+// even for every NI, so each layer starts 8-byte aligned.  store() writes the
+// LDS image (the pad columns of W3/b3 stay as zero_pad() left them).
+template <int NI, int THREADS> struct WeightRegsP
+{
+	using Y = Layout<NI>;
+	static_assert(Y::NP % 2 == 0 && Y::OB1 % 2 == 0 && Y::OW2 % 2 == 0 && Y::OB2 % 2 == 0 && Y::OW3 % 2 == 0 &&
+	                  Y::OB3 % 2 == 0 && NO % 2 == 0,
+	              "pairs of parameters");
+	static constexpr int NC = Y::NP / 2;
+	static constexpr int PER = (NC + THREADS - 1) / THREADS;
+	float2 v[PER];
+
+	__device__ void load(const float *__restrict__ p)
+	{
+		const float2 *q = reinterpret_cast<const float2 *>(p);
+#pragma unroll
+		for (int i = 0; i < PER; ++i)
+		{
+			const int c = threadIdx.x + i * THREADS;
+			if (c < NC)
+				v[i] = q[c];
+		}
+	}
+	__device__ void store(LWP<NI> &lw) const
+	{
+#pragma unroll
+		for (int i = 0; i < PER; ++i)
+		{
+			const int c = threadIdx.x + i * THREADS, x = 2 * c;
+			if (c >= NC)
+				break;
+			float *dst;
+			if (x < Y::OB1)
+				dst = lw.w1 + (x / NH) * WS + x % NH;
+			else if (x < Y::OW2)
+				dst = lw.b1 + (x - Y::OB1);
+			else if (x < Y::OB2)
+				dst = lw.w2 + ((x - Y::OW2) / NH) * WS + (x - Y::OW2) % NH;
+			else if (x < Y::OW3)
+				dst = lw.b2 + (x - Y::OB2);
+			else if (x < Y::OB3)
+				dst = lw.w3 + ((x - Y::OW3) / NO) * W3S + (x - Y::OW3) % NO;
+			else
+				dst = lw.b3 + (x - Y::OB3);
+			*reinterpret_cast<float2 *>(dst) = v[i];
+		}
+	}
+};
+
+// zero the W3/b3 padding columns NO..15 once per kernel (store() never writes them)
+template <int NI> __device__ void zero_pad(LWP<NI> &lw)
+{
+	for (int i = threadIdx.x; i < NH * 16; i += blockDim.x)
+		if (i % 16 >= NO)
+			lw.w3[(i / 16) * W3S + i % 16] = 0.f;
+	if (threadIdx.x < 16 && threadIdx.x >= NO)
+		lw.b3[threadIdx.x] = 0.f;
+}
+
+// act() of one block of pre-activations
+template <bool FAST> __device__ __forceinline__ f4 act4(f4 a)
+{
+	return f4{act<FAST>(a[0]), act<FAST>(a[1]), act<FAST>(a[2]), act<FAST>(a[3])};
+}
+
+// MLP forward of one tile: lane l holds row l % 16; x[s] is its feature
+// row(s), the four lanes of a row holding NI / 4 different features each.
+// h1[b][j], h2[b][j]: hidden columns 16 b + 4 (l / 16) + j; the return value:
+// outputs 4 (l / 16) + j.
+//
+// AHEAD (kernels with one wavefront a SIMD): the weights come a chunk of 16
+// ahead of their products; the scheduling barriers keep the loads there, which
+// left alone are placed two products before their use, so that each pair of
+// products waits out the LDS.  16^2 sample, 256 chains: 47.2 -> 43.7 us; with
+// more wavefronts its registers cost more (32^2 propose 210 -> 228 us).
+template <int NI, bool FAST, bool AHEAD, class ROW>
+__device__ __forceinline__ f4 mlp_rows(LWP<NI> const &lw, const float (&x)[NI / 4], ROW row, f4 (&h1)[4], f4 (&h2)[4])
+{
+	constexpr int NS = NI / 4, C1 = (NS + 3) / 4; // steps and chunks of the first layer
+	const int l = threadIdx.x & 63, i = l & 15, q4 = (l >> 4) * 4;
+	const float *w2 = lw.w2 + q4 * WS + i, *w3 = lw.w3 + q4 * W3S + i;
+	float w[2][16];
+	// chunk c of the weights: C1 of W1, four of W2 (one for each block of 16 of h1's columns), W3
+	auto load = [&](int c, float (&d)[16]) {
+#pragma unroll
+		for (int s = 0; s < 4; ++s)
+			if (c < C1)
+			{
+				if (4 * c + s < NS)
+#pragma unroll
+					for (int b = 0; b < 4; ++b)
+						d[4 * s + b] = lw.w1[row(4 * c + s) * WS + i + 16 * b];
+			}
+			else if (c < C1 + 4)
+#pragma unroll
+				for (int b = 0; b < 4; ++b)
+					d[4 * s + b] = w2[(16 * (c - C1) + s) * WS + 16 * b];
+			else
+#pragma unroll
+				for (int b = 0; b < 4; ++b)
+					d[4 * s + b] = w3[(16 * b + s) * W3S];
+	};
+	auto mm = [](float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); };
+#pragma unroll
+	for (int b = 0; b < 4; ++b)
+	{
+		h1[b] = *reinterpret_cast<const f4 *>(lw.b1 + 16 * b + q4);
+		h2[b] = *reinterpret_cast<const f4 *>(lw.b2 + 16 * b + q4);
+	}
+	// two chains: the products of one block of columns are each other's input
+	f4 y0 = *reinterpret_cast<const f4 *>(lw.b3 + q4), y1 = {0.f, 0.f, 0.f, 0.f};
+	if (AHEAD)
+		load(0, w[0]);
+#pragma unroll
+	for (int c = 0; c < C1 + 5; ++c)
+	{
+		if (!AHEAD)
+			load(c, w[c & 1]);
+		else if (c < C1 + 4)
+			load(c + 1, w[(c + 1) & 1]);
+		if (AHEAD)
+			__builtin_amdgcn_sched_barrier(0);
+		float (&d)[16] = w[c & 1];
+		const int k = c - C1;
+		if (k < 0)
+		{
+#pragma unroll
+			for (int s = 0; s < 4; ++s)
+				if (4 * c + s < NS)
+#pragma unroll
+					for (int b = 0; b < 4; ++b)
+						h1[b] = mm(d[4 * s + b], x[4 * c + s], h1[b]);
+			if (k == -1)
+				h1[0] = act4<FAST>(h1[0]);
+		}
+		else if (k < 3)
+		{
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+#pragma unroll
+				for (int b = 0; b < 4; ++b)
+					h2[b] = mm(d[4 * j + b], h1[k][j], h2[b]);
+			h1[k + 1] = act4<FAST>(h1[k + 1]);
+		}
+		else if (k == 3)
+		{
+#pragma unroll
+			for (int b = 0; b < 4; ++b)
+			{
+#pragma unroll
+				for (int j = 0; j < 4; ++j)
+					h2[b] = mm(d[4 * j + b], h1[3][j], h2[b]);
+				h2[b] = act4<FAST>(h2[b]);
+			}
+		}
+		else
+		{
+#pragma unroll
+			for (int b = 0; b < 4; b += 2)
+#pragma unroll
+				for (int j = 0; j < 4; ++j)
+				{
+					y0 = mm(d[4 * j + b], h2[b][j], y0);
+					y1 = mm(d[4 * j + b + 1], h2[b + 1][j], y1);
+				}
+		}
+	}
+	return y0 + y1;
+}
+
+// outputs of mlp_rows to y[row * YS + column] (one wavefront's scratch, 16 YS floats)
+__device__ __forceinline__ void put_outputs(float *y, f4 v)
+{
+	const int l = threadIdx.x & 63;
+	*reinterpret_cast<f4 *>(y + (l & 15) * YS + (l >> 4) * 4) = v;
+}
+
 // transform parameters from the MLP outputs
 struct NCP
 {
@@ -284,6 +487,62 @@ __device__ __forceinline__ float ncp_inverse(NCP const &p, float target, float &
 	return u;
 }
 
+// ---- elementary functions of the quad maps below, for the ranges they meet.
+// The maps were held by these: the library's sincosf and atan2f carry the
+// reduction of huge arguments, infinities and zeros, about 90 and 60 VALU
+// instructions a call against 24 and 27 here.  Coefficients: minimax fits
+// (reweighted least squares) of (sin r - r) / r^3 and (cos r - 1 + r^2 / 2) /
+// r^4 over |r| <= pi / 4 and of (atan q - q) / q^3 over [0, 1]; largest errors
+// in FP32 0.66 ulp (sin), 1.22 ulp (cos), 0.88 ulp (atan).
+
+// n / d to within an ulp, for d and 1 / d in the normal range
+__device__ __forceinline__ float div1(float n, float d)
+{
+	const float r = __builtin_amdgcn_rcpf(d), q = n * r;
+	return fmaf(fmaf(-q, d, n), r, q);
+}
+
+constexpr float HALF_PI_HI = 1.57079637050628662109f, HALF_PI_LO = -4.37113900018624283e-8f;
+
+// sin and cos for |x| up to a few turns (NaN gives NaN)
+__device__ __forceinline__ void sincos1(float x, float &sn, float &cs)
+{
+	const float q = rintf(x * 0.63661977236758134f);
+	float r = fmaf(-q, HALF_PI_HI, x);
+	r = fmaf(-q, HALF_PI_LO, r);
+	const float r2 = r * r;
+	const float s = fmaf(r * r2, fmaf(fmaf(-0.00019516977772582322f, r2, 0.008332176133990288f), r2,
+	                                  -0.16666655242443085f), r);
+	const float c = fmaf(r2 * r2, fmaf(fmaf(2.443809171381872e-05f, r2, -0.0013887364184483886f), r2,
+	                                   0.04166664555668831f), fmaf(-0.5f, r2, 1.f));
+	const int i = (int)q;
+	const bool odd = i & 1;
+	sn = __int_as_float(__float_as_int(odd ? c : s) ^ ((i & 2) << 30));
+	cs = __int_as_float(__float_as_int(odd ? s : c) ^ (((i + 1) & 2) << 30));
+}
+
+// atan2(y, x) for finite arguments, the larger of them a normal number whose
+// reciprocal is one too
+__device__ __forceinline__ float atan2_1(float y, float x)
+{
+	const float ax = fabsf(x), ay = fabsf(y);
+	const float q = div1(fminf(ax, ay), fmaxf(ax, ay)), q2 = q * q;
+	float p = fmaf(-0.0018272141460329294f, q2, 0.011064446531236172f);
+	p = fmaf(p, q2, -0.031455714255571365f);
+	p = fmaf(p, q2, 0.0582345649600029f);
+	p = fmaf(p, q2, -0.0841946005821228f);
+	p = fmaf(p, q2, 0.10957576334476471f);
+	p = fmaf(p, q2, -0.1426524519920349f);
+	p = fmaf(p, q2, 0.19998638331890106f);
+	p = fmaf(p, q2, -0.33333301544189453f);
+	const float a = fmaf(q * q2, p, q);
+	// pi/2 -+ a where |y| > |x|, pi - a for x < 0 below that
+	const bool steep = ay > ax, neg = x < 0.f;
+	const float k = steep ? HALF_PI_HI : (neg ? 2.f * HALF_PI_HI : 0.f);
+	const float t = fmaf(k, HALF_PI_LO / HALF_PI_HI, steep != neg ? -a : a);
+	return copysignf(k + t, y);
+}
+
 // ---- the mixture on a quad of lanes: lane k (= lane % 4) of a quad holds
 // component k; sums over the quad pair lanes (0,1)(2,3) and then the pairs,
 // with commutative adds, so that every lane of the quad holds the same bits.
@@ -322,10 +581,10 @@ __device__ __forceinline__ NCPq ncpq_params(const float *y)
 __device__ __forceinline__ void ncpq_eval(NCPq const &p, float u, float &G, float &Gp)
 {
 	float sn, c;
-	sincosf(0.5f * u, &sn, &c);
-	const float d = fmaf(c, c, p.s * p.s * sn * sn);
-	G = quad_sum(p.w * (2.f * atan2f(p.s * sn, c)));
-	Gp = quad_sum(p.w * (p.s / d));
+	sincos1(0.5f * u, sn, c);
+	const float d = fmaf(c, c, p.s * p.s * sn * sn); // e^-16 .. e^16
+	G = quad_sum(p.w * (2.f * atan2_1(p.s * sn, c)));
+	Gp = quad_sum(p.w * div1(p.s, d));
 }
 
 __device__ __forceinline__ float quad_min(float v)
@@ -351,8 +610,8 @@ __device__ __forceinline__ float quad_max(float v)
 __device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float &Gp)
 {
 	float st, ct;
-	sincosf(0.5f * target, &st, &ct);
-	const float uk = fminf(fmaxf(2.f * atan2f(st, p.s * ct), -PI_F), PI_F);
+	sincos1(0.5f * target, st, ct);
+	const float uk = fminf(fmaxf(2.f * atan2_1(st, p.s * ct), -PI_F), PI_F);
 	float lo = quad_min(uk), hi = quad_max(uk), u = quad_sum(p.w * uk), G;
 	lo = fmaxf(-PI_F, lo - 5e-7f * fmaxf(1.f, fabsf(lo)));
 	hi = fminf(PI_F, hi + 5e-7f * fmaxf(1.f, fabsf(hi)));
@@ -371,7 +630,7 @@ __device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float
 			hi = u;
 		if (hi - lo <= 2e-7f * fmaxf(1.f, fabsf(u)))
 			break;
-		float un = u - f / Gp;
+		float un = u - f * __builtin_amdgcn_rcpf(Gp);
 		fresh = false;
 		if (un > lo && un < hi)
 		{

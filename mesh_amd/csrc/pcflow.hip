@@ -36,17 +36,26 @@
 using namespace mesh_dev;
 namespace FM = flow_mlp;
 using u1_plaq::block_sum;
-using u1_plaq::PGeo;
 using u1_plaq::plaqp;
 using u1_plaq::wrapd;
 
 namespace {
 
+struct PCGeo : u1_plaq::PGeo
+{
+	unsigned hm; // ceil(2^20 / (L1 / 2)), see active_xy
+};
+
 constexpr int NI = 40; // features: 20 loops, (cos, sin) each
 constexpr int XS = FM::Layout<NI>::XS;
 constexpr int NP_LAYER = FM::Layout<NI>::NP;
 constexpr int MAX_LAYERS = 64;
-constexpr int THREADS = 256;
+constexpr int THREADS = 256; // of the backward kernel
+// smallest volume on 512 threads (forward and inverse): every one of the eight
+// wavefronts has a tile in a layer from V / 4 = 8 * 16 on.  32^2, 256 chains:
+// sample 126.5 us on 256 threads, 117.6 on 512; propose 217 and 209; 64^2
+// propose 1003 and 876
+constexpr int WIDE_V = 512;
 constexpr bool FAST = true; // tanh_fast in every kernel of this flow
 constexpr uint32_t TAG_PCFZ = 0x5043465au; // prior, holonomies, gauge
 constexpr uint32_t TAG_PCFI = 0x50434649u; // initial weights
@@ -61,7 +70,7 @@ __device__ __forceinline__ void ring(int k, int &d0, int &d1)
 }
 
 // site (x0, x1) with one periodic step either way
-__device__ __forceinline__ int sitew(PGeo const &g, int x0, int x1)
+__device__ __forceinline__ int sitew(PCGeo const &g, int x0, int x1)
 {
 	x0 = x0 < 0 ? x0 + g.L0 : (x0 >= g.L0 ? x0 - g.L0 : x0);
 	x1 = x1 < 0 ? x1 + g.L1 : (x1 >= g.L1 ? x1 - g.L1 : x1);
@@ -69,15 +78,17 @@ __device__ __forceinline__ int sitew(PGeo const &g, int x0, int x1)
 }
 
 // active plaquette r of mask class m
-__device__ __forceinline__ void active_xy(PGeo const &g, int m, int r, int &x0, int &x1)
+__device__ __forceinline__ void active_xy(PCGeo const &g, int m, int r, int &x0, int &x1)
 {
-	const int h = g.L1 >> 1, i = r / h, j = r - i * h;
+	// r < 1024 and h <= 512: r / h = r ceil(2^20 / h) >> 20 exactly, since
+	// r (h ceil(2^20 / h) - 2^20) < 2^20
+	const int h = g.L1 >> 1, i = (int)(((unsigned)r * g.hm) >> 20), j = r - i * h;
 	x0 = (m & 1) + 2 * i;
 	x1 = (m >> 1) + 2 * j;
 }
-__device__ __forceinline__ int n_active(PGeo const &g, int m) { return (g.V >> 2) - (m == 3 ? 1 : 0); }
-__device__ __forceinline__ int class_of(PGeo const &g, int x) { return ((x / g.L1) & 1) | (((x % g.L1) & 1) << 1); }
-__device__ __forceinline__ int active_index(PGeo const &g, int x)
+__device__ __forceinline__ int n_active(PCGeo const &g, int m) { return (g.V >> 2) - (m == 3 ? 1 : 0); }
+__device__ __forceinline__ int class_of(PCGeo const &g, int x) { return ((x / g.L1) & 1) | (((x % g.L1) & 1) << 1); }
+__device__ __forceinline__ int active_index(PCGeo const &g, int x)
 {
 	return ((x / g.L1) >> 1) * (g.L1 >> 1) + ((x % g.L1) >> 1);
 }
@@ -88,7 +99,7 @@ __device__ __forceinline__ int active_index(PGeo const &g, int x)
 // 2j + 1 (mod 8), j = k - 16 (the 2x2 square at corner 2j without its
 // centre); by angle addition.  cs holds (cos, sin) of every plaquette, (1, 0)
 // for the last, which enters the context as the angle 0.
-__device__ __forceinline__ float2 ring_cs(PGeo const &g, const float2 *cs, int x0, int x1, int k)
+__device__ __forceinline__ float2 ring_cs(PCGeo const &g, const float2 *cs, int x0, int x1, int k)
 {
 	int d0, d1;
 	ring(k & 7, d0, d1);
@@ -98,7 +109,7 @@ __device__ __forceinline__ float2 cs_add(float2 a, float2 b)
 {
 	return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.y, b.x, a.x * b.y));
 }
-__device__ __forceinline__ float2 loop_cs(PGeo const &g, const float2 *cs, int x0, int x1, int k)
+__device__ __forceinline__ float2 loop_cs(PCGeo const &g, const float2 *cs, int x0, int x1, int k)
 {
 	if (k < 8)
 		return ring_cs(g, cs, x0, x1, k);
@@ -114,7 +125,7 @@ __device__ __forceinline__ float2 loop_cs(PGeo const &g, const float2 *cs, int x
 // from NI on zero.  First the 8 ring plaquettes of every row (the only
 // gathers from the configuration), then the 1x2 and L-shaped loops from those
 // columns, by the angle additions of loop_cs in its order (the same bits).
-template <class TILE> __device__ void features(PGeo const &g, const float2 *cs, int m, int r0, int NA, TILE &T)
+template <class TILE> __device__ void features(PCGeo const &g, const float2 *cs, int m, int r0, int NA, TILE &T)
 {
 	const int l = threadIdx.x & 63;
 	for (int e = l; e < 16 * 8; e += 64)
@@ -151,44 +162,85 @@ template <class TILE> __device__ void features(PGeo const &g, const float2 *cs, 
 __device__ __forceinline__ float2 sincos2(float a)
 {
 	float s, c;
-	sincosf(a, &s, &c);
+	FM::sincos1(a, s, c);
 	return make_float2(c, s);
 }
 
-// LDS of the forward and inverse kernels (MLP outputs over the features) and
-// of the backward kernel (outputs apart: they carry dL/dy)
-template <bool SEP_Y> struct PCSharedT
+// LDS of the forward and inverse kernels of NT threads
+template <int NT> struct PCSharedF
+{
+	FM::LWP<NI> lw;
+	float y[NT / 64][16 * FM::YS];
+	double red[4][NT / 64];
+};
+// LDS of the backward kernel (outputs apart from the features: they carry dL/dy)
+struct PCSharedB
 {
 	FM::LW<NI> lw;
-	FM::Tile<NI, SEP_Y> tile[4];
+	FM::Tile<NI> tile[4];
 	double red[4][4];
 };
-using PCShared = PCSharedT<false>;
-using PCSharedB = PCSharedT<true>;
 
-// One layer on the workgroup: wavefront w takes tiles w, w + 4, ... of the
-// NA active plaquettes: features, MLP, then the circle map on quads (lane
-// 4i + k: row i of the tile, mixture component k).  Features read only
-// frozen plaquettes, so a wavefront may move its active ones while the others
-// still read theirs.  INV: apply g^-1 (the inverse pass).  Adds log g' to ld.
-template <bool INV>
-__device__ void layer_apply(PGeo const &g, float *phi, float2 *cs, int m, PCShared &sh, double &ld)
+// A lane's share of the 20 context loops of its row's plaquette: quarter q of
+// the wavefront takes ring plaquettes 2q and 2q + 1, the 1x2 loops (2q, 2q + 1)
+// and (2q - 1, 2q) and the L-shaped loop (2q - 1, 2q, 2q + 1), so three gathers
+// give its ten features.  rg: the loops' (cos, sin), in that order; row(s): the
+// feature index of x[s].
+struct LaneLoops
 {
-	const int w = threadIdx.x >> 6, l = threadIdx.x & 63, NA = n_active(g, m), NT = (NA + 15) / 16;
-	auto &T = sh.tile[w];
-	for (int tix = w; tix < NT; tix += 4)
+	int q, d0[3], d1[3]; // quarter; offsets of ring plaquettes 2q - 1, 2q, 2q + 1
+	__device__ LaneLoops()
 	{
-		features(g, cs, m, tix * 16, NA, T);
+		q = (threadIdx.x >> 4) & 3;
+		ring((2 * q + 7) & 7, d0[0], d1[0]);
+		ring(2 * q, d0[1], d1[1]);
+		ring(2 * q + 1, d0[2], d1[2]);
+	}
+	__device__ __forceinline__ int row(int s) const
+	{
+		return s < 4 ? 4 * q + s : (s < 6 ? 12 + 4 * q + s : (s < 8 ? 10 + 2 * ((2 * q + 7) & 7) + s : 24 + 2 * q + s));
+	}
+	// the additions of loop_cs, in its order
+	__device__ __forceinline__ void features(PCGeo const &g, const float2 *cs, int x0, int x1, float (&x)[NI / 4]) const
+	{
+		const float2 a = cs[sitew(g, x0 + d0[0], x1 + d1[0])], b = cs[sitew(g, x0 + d0[1], x1 + d1[1])],
+		             c = cs[sitew(g, x0 + d0[2], x1 + d1[2])];
+		const float2 p = cs_add(b, c), m = cs_add(a, b), t = cs_add(m, c);
+		x[0] = b.x, x[1] = b.y, x[2] = c.x, x[3] = c.y, x[4] = p.x, x[5] = p.y, x[6] = m.x, x[7] = m.y, x[8] = t.x,
+		x[9] = t.y;
+	}
+};
+
+// One layer on the workgroup: wavefront w takes tiles w, w + NT / 64, ... of
+// the NA active plaquettes: features and MLP in registers (mlp_rows), then the
+// circle map on quads (lane 4i + k: row i of the tile, mixture component k),
+// to which the outputs go through 1.25 KB of LDS.  Features read only frozen
+// plaquettes, so a wavefront may move its active ones while the others still
+// read theirs.  INV: apply g^-1 (the inverse pass).  Adds log g' to ld.
+template <bool INV, int NT>
+__device__ __forceinline__ void layer_apply(PCGeo const &g, LaneLoops const &ll, float *phi, float2 *cs, int m,
+                                            PCSharedF<NT> &sh, double &ld)
+{
+	const int w = threadIdx.x >> 6, l = threadIdx.x & 63, NA = n_active(g, m), ntile = (NA + 15) / 16;
+	float *y = sh.y[w];
+	for (int tix = w; tix < ntile; tix += NT / 64)
+	{
+		int x0, x1;
+		// rows beyond NA repeat the last one; nothing reads their outputs
+		active_xy(g, m, min(tix * 16 + (l & 15), NA - 1), x0, x1);
+		float x[NI / 4];
+		ll.features(g, cs, x0, x1, x);
+		FM::f4 h1[4], h2[4];
+		const FM::f4 out = FM::mlp_rows<NI, FAST, NT == 256>(sh.lw, x, [&](int s) { return ll.row(s); }, h1, h2);
+		FM::put_outputs(y, out);
 		FM::wave_sync();
-		FM::mlp_forward<NI, FAST>(sh.lw, T);
 		const int row = l >> 2, r = tix * 16 + row;
 		if (r < NA)
 		{
-			int x0, x1;
 			active_xy(g, m, r, x0, x1);
-			const int x = x0 * g.L1 + x1;
-			const FM::NCPq p = FM::ncpq_params(&T.y()[row * 16]);
-			const float a = FM::wrapf(phi[x] - p.t);
+			const int xs = x0 * g.L1 + x1;
+			const FM::NCPq p = FM::ncpq_params(&y[row * FM::YS]);
+			const float a = FM::wrapf(phi[xs] - p.t);
 			float v, Gp;
 			if (INV)
 				v = FM::ncpq_inverse(p, a, Gp);
@@ -197,8 +249,8 @@ __device__ void layer_apply(PGeo const &g, float *phi, float2 *cs, int m, PCShar
 			if ((l & 3) == 0)
 			{
 				const float nx = FM::wrapf(v + p.t);
-				phi[x] = nx;
-				cs[x] = sincos2(nx);
+				phi[xs] = nx;
+				cs[xs] = sincos2(nx);
 				ld += (double)logf(Gp);
 			}
 		}
@@ -211,18 +263,20 @@ __device__ void layer_apply(PGeo const &g, float *phi, float2 *cs, int m, PCShar
 // links.  out[2c + {0,1}] = {log q, S/beta}, S of the links when they are
 // formed, else of the plaquettes (the last one = -sum of the free ones).
 // LDS: phi[V], cs[V] (then the links' scratch), al[V].
-__device__ void pc_forward(PGeo const &g, int nl, const float *__restrict__ params, uint64_t seed, uint32_t step,
-                           float *theta_out, float *phi_layers, float *phi_final, double *out, int c, float *dyn,
-                           PCShared &sh)
+template <int NT>
+__device__ __forceinline__ void pc_forward(PCGeo const &g, int nl, const float *__restrict__ params, uint64_t seed,
+                                           uint32_t step, float *theta_out, float *phi_layers, float *phi_final,
+                                           double *out, int c, float *dyn, PCSharedF<NT> &sh)
 {
 	float *phi = dyn;
 	float2 *cs = reinterpret_cast<float2 *>(dyn + g.V);
 	float *al = dyn + 3 * g.V;
 	const uint32_t cc = (uint32_t)c << 1;
-	Weights wr;
+	FM::WeightRegsP<NI, NT> wr;
+	const LaneLoops ll;
 	wr.load(params);
 	FM::zero_pad<NI>(sh.lw);
-	for (int x = threadIdx.x; x < g.V; x += THREADS)
+	for (int x = threadIdx.x; x < g.V; x += NT)
 	{
 		const float z = x < g.V - 1 ? u1_plaq::uniform_angle(seed, step, (uint32_t)x, cc, TAG_PCFZ) : 0.f;
 		phi[x] = z;
@@ -235,39 +289,39 @@ __device__ void pc_forward(PGeo const &g, int nl, const float *__restrict__ para
 		__syncthreads(); // the previous layer is done with the weights and the plaquettes
 		wr.store(sh.lw);
 		if (phi_layers)
-			for (int x = threadIdx.x; x < g.V; x += THREADS)
+			for (int x = threadIdx.x; x < g.V; x += NT)
 				phi_layers[((long)c * nl + layer) * g.V + x] = phi[x];
 		__syncthreads();
 		if (layer + 1 < nl)
 			wr.load(params + (long)(layer + 1) * NP_LAYER);
-		layer_apply<false>(g, phi, cs, layer & 3, sh, ld);
+		layer_apply<false, NT>(g, ll, phi, cs, layer & 3, sh, ld);
 	}
 	__syncthreads();
 	if (phi_final)
-		for (int x = threadIdx.x; x < g.V; x += THREADS)
+		for (int x = threadIdx.x; x < g.V; x += NT)
 			phi_final[(long)c * g.V + x] = phi[x];
 	double v[3] = {ld, 0.0, 0.0}; // log det, S of the free plaquettes, their sum
-	for (int x = threadIdx.x; x < g.V - 1; x += THREADS)
+	for (int x = threadIdx.x; x < g.V - 1; x += NT)
 	{
 		v[1] += 1.0 - cos((double)phi[x]);
 		v[2] += (double)phi[x];
 	}
-	block_sum<3>(v, sh.red);
+	block_sum<3, NT / 64>(v, sh.red);
 	double S = v[1] + (1.0 - cos(wrapd(-v[2])));
 	if (theta_out)
 	{
 		float *o = theta_out + (long)c * 2 * g.V;
 		const float h0 = u1_plaq::uniform_angle(seed, step, (uint32_t)g.V, cc, TAG_PCFZ);
 		const float h1 = u1_plaq::uniform_angle(seed, step, (uint32_t)g.V + 1u, cc, TAG_PCFZ);
-		u1_plaq::links_from_plaquettes(g, phi, h0, h1, al, reinterpret_cast<float *>(cs), o, THREADS);
+		u1_plaq::links_from_plaquettes(g, phi, h0, h1, al, reinterpret_cast<float *>(cs), o, NT);
 		__syncthreads();
 		double s[1] = {0.0};
-		for (int x = threadIdx.x; x < g.V; x += THREADS)
+		for (int x = threadIdx.x; x < g.V; x += NT)
 		{
 			const int x0 = x / g.L1, x1 = x - x0 * g.L1;
 			s[0] += 1.0 - cos((double)plaqp(g, o, x0, x1));
 		}
-		block_sum<1>(s, sh.red);
+		block_sum<1, NT / 64>(s, sh.red);
 		S = s[0];
 	}
 	if (threadIdx.x == 0)
@@ -280,20 +334,23 @@ __device__ void pc_forward(PGeo const &g, int nl, const float *__restrict__ para
 // log q of given links: plaquettes, then the layers in reverse with g^-1.
 // out[2c + {0,1}] = {log q(U), S(U)/beta}; z_out (optional): the prior draws,
 // V per configuration (the last 0).  LDS: the links (then cs[V]), phi[V].
-__device__ void pc_inverse(PGeo const &g, int nl, const float *__restrict__ params, const float *__restrict__ theta,
-                           float *z_out, double *out, int c, float *dyn, PCShared &sh)
+template <int NT>
+__device__ __forceinline__ void pc_inverse(PCGeo const &g, int nl, const float *__restrict__ params,
+                                           const float *__restrict__ theta, float *z_out, double *out, int c,
+                                           float *dyn, PCSharedF<NT> &sh)
 {
 	float *th = dyn;
 	float2 *cs = reinterpret_cast<float2 *>(dyn);
 	float *phi = dyn + 2 * g.V;
-	Weights wr;
+	FM::WeightRegsP<NI, NT> wr;
+	const LaneLoops ll;
 	wr.load(params + (long)(nl - 1) * NP_LAYER);
 	FM::zero_pad<NI>(sh.lw);
-	for (int i = threadIdx.x; i < 2 * g.V; i += THREADS)
+	for (int i = threadIdx.x; i < 2 * g.V; i += NT)
 		th[i] = theta[(long)c * 2 * g.V + i];
 	__syncthreads();
 	double v[2] = {0.0, 0.0}; // log det, S
-	for (int x = threadIdx.x; x < g.V; x += THREADS)
+	for (int x = threadIdx.x; x < g.V; x += NT)
 	{
 		const int x0 = x / g.L1, x1 = x - x0 * g.L1;
 		const float tp = plaqp(g, th, x0, x1);
@@ -301,7 +358,7 @@ __device__ void pc_inverse(PGeo const &g, int nl, const float *__restrict__ para
 		phi[x] = x < g.V - 1 ? FM::wrapf(tp) : 0.f;
 	}
 	__syncthreads(); // the links are read; cs takes their place
-	for (int x = threadIdx.x; x < g.V; x += THREADS)
+	for (int x = threadIdx.x; x < g.V; x += NT)
 		cs[x] = sincos2(phi[x]);
 	for (int layer = nl - 1; layer >= 0; --layer)
 	{
@@ -310,47 +367,50 @@ __device__ void pc_inverse(PGeo const &g, int nl, const float *__restrict__ para
 		__syncthreads();
 		if (layer > 0)
 			wr.load(params + (long)(layer - 1) * NP_LAYER);
-		layer_apply<true>(g, phi, cs, layer & 3, sh, v[0]);
+		layer_apply<true, NT>(g, ll, phi, cs, layer & 3, sh, v[0]);
 	}
 	__syncthreads();
-	block_sum<2>(v, sh.red);
+	block_sum<2, NT / 64>(v, sh.red);
 	if (threadIdx.x == 0)
 	{
 		out[2 * c + 0] = -v[0] - 2.0 * g.V * LOG_2PI;
 		out[2 * c + 1] = v[1];
 	}
 	if (z_out)
-		for (int x = threadIdx.x; x < g.V; x += THREADS)
+		for (int x = threadIdx.x; x < g.V; x += NT)
 			z_out[(long)c * g.V + x] = phi[x];
 }
 
-__global__ __launch_bounds__(THREADS) void k_pc_forward(PGeo g, int nl, const float *__restrict__ params,
-                                                        uint64_t seed, uint32_t step, float *theta_out,
-                                                        float *phi_layers, float *phi_final, double *out)
+// The kernels run on 256 or 512 threads (by_width()).
+template <int NT>
+__global__ __launch_bounds__(NT) void k_pc_forward(PCGeo g, int nl, const float *__restrict__ params, uint64_t seed,
+                                                   uint32_t step, float *theta_out, float *phi_layers,
+                                                   float *phi_final, double *out)
 {
 	extern __shared__ float dyn[];
-	__shared__ PCShared sh;
+	__shared__ PCSharedF<NT> sh;
 	pc_forward(g, nl, params, seed, step, theta_out, phi_layers, phi_final, out, blockIdx.x, dyn, sh);
 }
 
-__global__ __launch_bounds__(THREADS) void k_pc_inverse(PGeo g, int nl, const float *__restrict__ params,
-                                                        const float *__restrict__ theta, float *z_out, double *out)
+template <int NT>
+__global__ __launch_bounds__(NT) void k_pc_inverse(PCGeo g, int nl, const float *__restrict__ params,
+                                                   const float *__restrict__ theta, float *z_out, double *out)
 {
 	extern __shared__ float dyn[];
-	__shared__ PCShared sh;
+	__shared__ PCSharedF<NT> sh;
 	pc_inverse(g, nl, params, theta, z_out, out, blockIdx.x, dyn, sh);
 }
 
 // one MH proposal round in one launch: workgroups 0..batch-1 take log q of
 // the current configurations, batch..2 batch-1 draw the proposals, so that on
 // small lattices (two workgroups' LDS per CU) the two passes share the CUs
-__global__ __launch_bounds__(THREADS) void k_pc_propose(PGeo g, int nl, const float *__restrict__ params, int batch,
-                                                        const float *__restrict__ theta, double *state,
-                                                        uint64_t seed, uint32_t step, float *theta_prop,
-                                                        double *prop_out)
+template <int NT>
+__global__ __launch_bounds__(NT) void k_pc_propose(PCGeo g, int nl, const float *__restrict__ params, int batch,
+                                                   const float *__restrict__ theta, double *state, uint64_t seed,
+                                                   uint32_t step, float *theta_prop, double *prop_out)
 {
 	extern __shared__ float dyn[];
-	__shared__ PCShared sh;
+	__shared__ PCSharedF<NT> sh;
 	if ((int)blockIdx.x < batch)
 		pc_inverse(g, nl, params, theta, nullptr, state, blockIdx.x, dyn, sh);
 	else
@@ -362,7 +422,7 @@ __global__ __launch_bounds__(THREADS) void k_pc_propose(PGeo g, int nl, const fl
 // partial[c][layer * NP_LAYER + i].  phi_layers / phi_final from k_pc_forward;
 // dxs: scratch of (V/4) * NI floats per configuration.
 // LDS: cs[V] (of the current layer's input), phi[V], a[V], gact[V/4].
-__global__ __launch_bounds__(THREADS) void k_pc_backward(PGeo g, int nl, const float *__restrict__ params,
+__global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const float *__restrict__ params,
                                                          const float *__restrict__ phi_layers,
                                                          const float *__restrict__ phi_final, float beta,
                                                          float *__restrict__ dxs, float *__restrict__ partial)
@@ -498,7 +558,7 @@ __global__ void k_pc_init(int n, float *p, uint64_t seed)
 		FM::init_param<NI>(i, p, seed, TAG_PCFI);
 }
 
-int pc_setup(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers, PGeo *pg, const float *params = nullptr)
+int pc_setup(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers, PCGeo *pg, const float *params = nullptr)
 {
 	if (layers < 1 || layers > MAX_LAYERS)
 		return mesh_fail(ctx, MESH_E_ARG, "the plaquette coupling flow has 1 to 64 layers");
@@ -514,12 +574,35 @@ int pc_setup(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers, PGeo *pg,
 	pg->L0 = g->dims[0];
 	pg->L1 = g->dims[1];
 	pg->V = (int)V;
+	const unsigned h = (unsigned)pg->L1 >> 1;
+	pg->hm = ((1u << 20) + h - 1) / h;
 	return MESH_OK;
 }
 
 template <class K> int set_lds(mesh_ctx *ctx, K kernel, size_t bytes)
 {
 	MESH_HIP(ctx, hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+	return MESH_OK;
+}
+
+// kernel(std::integral_constant<int, threads>) on 512 threads from WIDE_V on
+template <class F> int by_width(PCGeo const &g, F &&kernel)
+{
+	if (g.V >= WIDE_V)
+		return kernel(std::integral_constant<int, 512>{});
+	return kernel(std::integral_constant<int, 256>{});
+}
+
+template <int NT> int launch_forward(mesh_ctx *ctx, PCGeo const &g, int batch, int layers, const float *params,
+                                     uint64_t seed, uint32_t step, float *theta_out, float *phi_layers,
+                                     float *phi_final, double *out)
+{
+	const size_t lds = 4 * (size_t)g.V * sizeof(float);
+	if (int rc = set_lds(ctx, k_pc_forward<NT>, lds))
+		return rc;
+	k_pc_forward<NT><<<batch, NT, lds, ctx->stream>>>(g, layers, params, seed, step, theta_out, phi_layers, phi_final,
+	                                                  out);
+	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }
 
@@ -544,35 +627,35 @@ int mesh_pcflow_sample(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers,
                        uint32_t step, float *theta_out, double *out_dev)
 {
 	MESH_CHECK_CTX(ctx);
-	PGeo pg;
+	PCGeo pg;
 	if (int rc = pc_setup(ctx, g, batch, layers, &pg, params))
 		return rc;
 	if (!params || !theta_out || !out_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_sample");
-	const size_t lds = 4 * (size_t)pg.V * sizeof(float);
-	if (int rc = set_lds(ctx, k_pc_forward, lds))
-		return rc;
-	k_pc_forward<<<batch, THREADS, lds, ctx->stream>>>(pg, layers, params, seed, step, theta_out, nullptr, nullptr,
-	                                                   out_dev);
-	MESH_LAUNCHED(ctx);
-	return MESH_OK;
+	return by_width(pg, [&](auto nt) {
+		return launch_forward<decltype(nt)::value>(ctx, pg, batch, layers, params, seed, step, theta_out, nullptr,
+		                                           nullptr, out_dev);
+	});
 }
 
 int mesh_pcflow_logq(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers, const float *params,
                      const float *theta, float *z_out, double *out_dev)
 {
 	MESH_CHECK_CTX(ctx);
-	PGeo pg;
+	PCGeo pg;
 	if (int rc = pc_setup(ctx, g, batch, layers, &pg, params))
 		return rc;
 	if (!params || !theta || !out_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_logq");
-	const size_t lds = 3 * (size_t)pg.V * sizeof(float);
-	if (int rc = set_lds(ctx, k_pc_inverse, lds))
-		return rc;
-	k_pc_inverse<<<batch, THREADS, lds, ctx->stream>>>(pg, layers, params, theta, z_out, out_dev);
-	MESH_LAUNCHED(ctx);
-	return MESH_OK;
+	return by_width(pg, [&](auto nt) -> int {
+		constexpr int NT = decltype(nt)::value;
+		const size_t lds = 3 * (size_t)pg.V * sizeof(float);
+		if (int rc = set_lds(ctx, k_pc_inverse<NT>, lds))
+			return rc;
+		k_pc_inverse<NT><<<batch, NT, lds, ctx->stream>>>(pg, layers, params, theta, z_out, out_dev);
+		MESH_LAUNCHED(ctx);
+		return MESH_OK;
+	});
 }
 
 int mesh_pcflow_propose(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers, const float *params,
@@ -580,25 +663,28 @@ int mesh_pcflow_propose(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers
                         double *prop_dev)
 {
 	MESH_CHECK_CTX(ctx);
-	PGeo pg;
+	PCGeo pg;
 	if (int rc = pc_setup(ctx, g, batch, layers, &pg, params))
 		return rc;
 	if (!params || !theta || !state_dev || !theta_prop || !prop_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_propose");
 	if (theta == theta_prop || state_dev == prop_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "pcflow_propose: the proposals and their log q need their own buffers");
-	const size_t lds = 4 * (size_t)pg.V * sizeof(float);
-	if (int rc = set_lds(ctx, k_pc_propose, lds))
-		return rc;
-	k_pc_propose<<<2 * batch, THREADS, lds, ctx->stream>>>(pg, layers, params, batch, theta, state_dev, seed, step,
-	                                                       theta_prop, prop_dev);
-	MESH_LAUNCHED(ctx);
-	return MESH_OK;
+	return by_width(pg, [&](auto nt) -> int {
+		constexpr int NT = decltype(nt)::value;
+		const size_t lds = 4 * (size_t)pg.V * sizeof(float);
+		if (int rc = set_lds(ctx, k_pc_propose<NT>, lds))
+			return rc;
+		k_pc_propose<NT><<<2 * batch, NT, lds, ctx->stream>>>(pg, layers, params, batch, theta, state_dev, seed, step,
+		                                                      theta_prop, prop_dev);
+		MESH_LAUNCHED(ctx);
+		return MESH_OK;
+	});
 }
 
 size_t mesh_pcflow_workspace_bytes(const mesh_grid *g, int batch, int layers)
 {
-	PGeo pg;
+	PCGeo pg;
 	if (pc_setup(nullptr, g, batch, layers, &pg))
 		return 0;
 	size_t n = (size_t)batch * layers * pg.V           // plaquettes per layer
@@ -612,7 +698,7 @@ int mesh_pcflow_gradient(mesh_ctx *ctx, const mesh_grid *g, int batch, int layer
                          uint32_t step, double beta, void *workspace, float *grad, double *out_dev)
 {
 	MESH_CHECK_CTX(ctx);
-	PGeo pg;
+	PCGeo pg;
 	if (int rc = pc_setup(ctx, g, batch, layers, &pg, params))
 		return rc;
 	if (!params || !workspace || !grad || !out_dev)
@@ -621,11 +707,11 @@ int mesh_pcflow_gradient(mesh_ctx *ctx, const mesh_grid *g, int batch, int layer
 	float *pf = pl + (size_t)batch * layers * pg.V;
 	float *dxs = pf + (size_t)batch * pg.V;
 	float *part = dxs + (size_t)batch * (pg.V / 4) * NI;
-	const size_t lds_f = 4 * (size_t)pg.V * sizeof(float);
-	if (int rc = set_lds(ctx, k_pc_forward, lds_f))
+	if (int rc = by_width(pg, [&](auto nt) {
+		    return launch_forward<decltype(nt)::value>(ctx, pg, batch, layers, params, seed, step, nullptr, pl, pf,
+		                                               out_dev);
+	    }))
 		return rc;
-	k_pc_forward<<<batch, THREADS, lds_f, ctx->stream>>>(pg, layers, params, seed, step, nullptr, pl, pf, out_dev);
-	MESH_LAUNCHED(ctx);
 	const size_t lds_b = (4 * (size_t)pg.V + pg.V / 4) * sizeof(float);
 	if (int rc = set_lds(ctx, k_pc_backward, lds_b))
 		return rc;

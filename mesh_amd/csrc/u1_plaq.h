@@ -56,8 +56,8 @@ __device__ __forceinline__ float uniform_angle(uint64_t seed, uint32_t step, uin
 	return (float)(6.283185307179586477 * u - 3.141592653589793238);
 }
 
-// sums over the 256 threads of a workgroup, in a fixed order
-template <int NQ> __device__ __forceinline__ void block_sum(double (&v)[NQ], double (*red)[4])
+// sums over the NW wavefronts of a workgroup, in a fixed order
+template <int NQ, int NW = 4> __device__ __forceinline__ void block_sum(double (&v)[NQ], double (*red)[NW])
 {
 	int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 	for (int q = 0; q < NQ; ++q)
@@ -70,7 +70,11 @@ template <int NQ> __device__ __forceinline__ void block_sum(double (&v)[NQ], dou
 	}
 	__syncthreads();
 	for (int q = 0; q < NQ; ++q)
-		v[q] = ((red[q][0] + red[q][1]) + red[q][2]) + red[q][3];
+	{
+		v[q] = red[q][0];
+		for (int i = 1; i < NW; ++i)
+			v[q] += red[q][i];
+	}
 	__syncthreads();
 }
 

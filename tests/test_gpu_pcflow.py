@@ -93,6 +93,31 @@ def test_pcflow_sample_against_oracle(ctx, L0, L1):
     np.testing.assert_allclose(out[:, 1], U.action_over_beta(th.astype(np.float64)), rtol=1e-4)
 
 
+@pytest.mark.parametrize("L0,L1", [(4, 4), (10, 50), (4, 128), (6, 86), (64, 64), (4, 1024)])
+def test_pcflow_tile_edges(ctx, L0, L1):
+    """both widths of the kernels (512 threads from 512 plaquettes on), tiles
+    with 3, 13, 16 and 1 rows, the largest volume and the longest row: the
+    forward map against the oracle, and the inverse back to the draws (bounds
+    of the tests above: FP32 steps through 8 layers, log q a sum over V)"""
+    torch = pytest.importorskip("torch")
+    B, seed, step = 2, 17, 3
+    V = L0 * L1
+    p = _params(18, 0.2)
+    f = U1.PlaqCouplingFlow(L0, L1, ctx)
+    f.set_params(p)
+    ens = U1.U1Ensemble(L0, L1, B, ctx)
+    out = f.sample(ens, seed, step).download().reshape(B, 2)
+    z = np.stack([U.pcflow_draws(seed, step, c, L0, L1)[0] for c in range(B)]).astype(np.float64)
+    phi, ld = U.pcflow_forward(torch.tensor(p.astype(np.float64)), torch.tensor(z), L0, L1)
+    tol = 2e-3 * max(1.0, V / 64)
+    assert _wrapdiff(_free_plaquettes(ens.angles()), phi.numpy()).max() < 1e-3
+    np.testing.assert_allclose(out[:, 0], U.log_prior(L0, L1) - ld.numpy(), atol=tol)
+    z_out = U1.Buffer(B * V, np.float32, ctx)
+    inv = f.logq(ens, z_out=z_out).download().reshape(B, 2)
+    assert _wrapdiff(z_out.download().reshape(B, V)[:, :-1], z).max() < 2e-3
+    np.testing.assert_allclose(inv[:, 0], out[:, 0], atol=tol)
+
+
 def test_pcflow_inverse_roundtrip(ctx):
     """log q by the inverse of a sample equals the sampler's log q and
     recovers its prior draws"""
