@@ -21,8 +21,7 @@
 // gauge-equivariant (it moves links by gauge-invariant amounts).
 //
 // Kernels: one workgroup (256 threads) per configuration, angles in LDS;
-// the dense layers of the MLP run on FP32 MFMA (v_mfma_f32_16x16x4_f32) in
-// 16-row tiles, one tile per wavefront.
+// the dense layers of the MLP run on FP32 MFMA (flow_mlp.h).
 #include "flow_mlp.h"
 #include "mesh_internal.h"
 #include "rng_dev.h"
@@ -96,27 +95,23 @@ __device__ __forceinline__ int updated_link(FGeo const &g, int mu, int y0, int y
 	return mu == 0 ? site(g, y0, y1) : g.V + site(g, y0 + 1, y1);
 }
 
-using LWF = LW<NI>;
-using TileF = Tile<NI>;
+// Quarter q of a wavefront takes the features 4 s + q, s < 3, of its lanes'
+// rows: the cosine (q even) or sine of frozen neighbour 2 s + q / 2.
+__device__ __forceinline__ int feature_row(int q, int s) { return 4 * s + q; }
 
-// features of the 16 active plaquettes r0..r0+15 (rows beyond NA are zero)
-__device__ void features(FGeo const &g, const float *t, int mu, int a, int r0, TileF &T)
+__device__ __forceinline__ void features(FGeo const &g, const float *t, int mu, int a, int r, float (&x)[NI / 4])
 {
-	int l = threadIdx.x & 63;
-	for (int e = l; e < 16 * 16; e += 64)
+	const int q = (threadIdx.x >> 4) & 3;
+	int y0, y1;
+	active_corner(g, mu, a, r, y0, y1);
+#pragma unroll
+	for (int s = 0; s < NI / 4; ++s)
 	{
-		int row = e / 16, col = e % 16;
-		float v = 0.f;
-		int r = r0 + row;
-		if (r < g.NA && col < NI)
-		{
-			int y0, y1, z0, z1;
-			active_corner(g, mu, a, r, y0, y1);
-			frozen_corner(mu, col / 2, y0, y1, z0, z1);
-			float p = plaqf(g, t, z0, z1);
-			v = (col & 1) ? sinf(p) : cosf(p);
-		}
-		T.x[e] = v;
+		int z0, z1;
+		frozen_corner(mu, 2 * s + (q >> 1), y0, y1, z0, z1);
+		float sn, cs;
+		sincos1(plaqf(g, t, z0, z1), sn, cs);
+		x[s] = (q & 1) ? sn : cs;
 	}
 }
 
@@ -124,27 +119,52 @@ __device__ void features(FGeo const &g, const float *t, int mu, int a, int r0, T
 
 struct FlowShared
 {
-	LWF lw;
-	TileF tile[4];
+	LWP<NI> lw;
+	float y[THREADS / 64][16 * YS];
 	double red[4][4];
 };
-
-// MLP outputs of tiles it .. it+15 (four per wavefront) into Ys[tile][row*16+k]
-__device__ void mlp_round(FGeo const &g, const float *th, int mu, int a, int it, int NT, FlowShared &sh,
-                          float (*Ys)[256])
+struct FlowSharedB
 {
-	const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-	TileF &T = sh.tile[w];
-	for (int q = 0; q < 4; ++q)
+	LWP<NI> lw;
+	BackBuf<NI> buf;
+};
+
+// One layer on the workgroup: wavefront w takes tiles w, w + 4, ... of the NA
+// active plaquettes: features, MLP, then the circle map on quads (lane 4i + k:
+// row i of the tile, component k).  Frozen plaquettes hold no updated link and
+// an active one only its own, so a wavefront may move its links while the
+// others still read theirs.  INV: apply g^-1.  Adds log g' to ld.
+template <bool INV>
+__device__ __forceinline__ void layer_apply(FGeo const &g, float *th, int mu, int a, FlowShared &sh, double &ld)
+{
+	const int w = threadIdx.x >> 6, l = threadIdx.x & 63, q = l >> 4, ntile = (g.NA + 15) / 16;
+	float *y = sh.y[w];
+	for (int tix = w; tix < ntile; tix += THREADS / 64)
 	{
-		const int tl = q * 4 + w, tix = it + tl;
-		if (tix >= NT)
-			break;
-		features(g, th, mu, a, tix * 16, T);
+		float x[NI / 4];
+		features(g, th, mu, a, min(tix * 16 + (l & 15), g.NA - 1), x);
+		f4 h1[4], h2[4];
+		put_outputs(y, mlp_rows<NI, false, true>(sh.lw, x, [&](int s) { return feature_row(q, s); }, h1, h2));
 		wave_sync();
-		mlp_forward<NI>(sh.lw, T);
-		for (int e = l; e < 256; e += 64)
-			Ys[tl][e] = T.y()[e];
+		const int r = tix * 16 + (l >> 2);
+		if (r < g.NA)
+		{
+			int y0, y1;
+			active_corner(g, mu, a, r, y0, y1);
+			const NCPq p = ncpq_params(&y[(l >> 2) * YS]);
+			const float tp = plaqf(g, th, y0, y1), u = wrapf(tp - p.t);
+			float v, Gp;
+			if (INV)
+				v = ncpq_inverse(p, u, Gp);
+			else
+				ncpq_eval(p, u, v, Gp);
+			if ((l & 3) == 0)
+			{
+				const int ul = updated_link(g, mu, y0, y1);
+				th[ul] = wrapf(INV ? th[ul] - tp + v + p.t : th[ul] + (v + p.t - tp));
+				ld += (double)logf(Gp);
+			}
+		}
 		wave_sync();
 	}
 }
@@ -157,7 +177,6 @@ __global__ __launch_bounds__(THREADS) void k_flow_forward(FGeo g, int nl, const 
 {
 	extern __shared__ float th[]; // 2V
 	__shared__ FlowShared sh;
-	__shared__ float Ys[16][256];
 	const int c = blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
 	for (int i = threadIdx.x; i < 2 * g.V; i += THREADS)
 	{
@@ -168,37 +187,20 @@ __global__ __launch_bounds__(THREADS) void k_flow_forward(FGeo g, int nl, const 
 		th[i] = (float)(6.283185307179586477 * u - 3.141592653589793238);
 	}
 	double logdet = 0.0;
-	const int NT = (g.NA + 15) / 16;
+	WeightRegsP<NI, THREADS> wr;
+	wr.load(params);
+	zero_pad<NI>(sh.lw);
 	for (int layer = 0; layer < nl; ++layer)
 	{
-		const int mu = layer & 1, a = (layer >> 1) & 3;
 		__syncthreads();
 		if (theta_layers)
 			for (int i = threadIdx.x; i < 2 * g.V; i += THREADS)
 				theta_layers[((long)c * nl + layer) * 2 * g.V + i] = th[i];
-		load_weights<NI>(sh.lw, params + layer * NP_LAYER);
+		wr.store(sh.lw);
 		__syncthreads();
-		// within a layer the MLP inputs (frozen plaquettes) never change, so
-		// all MLPs of a round run first and then every thread moves one link
-		for (int it = 0; it < NT; it += 16)
-		{
-			mlp_round(g, th, mu, a, it, NT, sh, Ys);
-			__syncthreads();
-			const int r = it * 16 + threadIdx.x;
-			if (r < g.NA)
-			{
-				int y0, y1;
-				active_corner(g, mu, a, r, y0, y1);
-				NCP p = ncp_params(&Ys[threadIdx.x >> 4][(threadIdx.x & 15) * 16]);
-				float tp = plaqf(g, th, y0, y1);
-				float u = wrapf(tp - p.t), G, Gp;
-				ncp_eval(p, u, G, Gp);
-				int ul = updated_link(g, mu, y0, y1);
-				th[ul] = wrapf(th[ul] + (G + p.t - tp));
-				logdet += (double)logf(Gp);
-			}
-			__syncthreads();
-		}
+		if (layer + 1 < nl)
+			wr.load(params + (long)(layer + 1) * NP_LAYER);
+		layer_apply<false>(g, th, layer & 1, (layer >> 1) & 3, sh, logdet);
 	}
 	__syncthreads();
 	double v[2] = {logdet, 0.0};
@@ -231,7 +233,6 @@ __global__ __launch_bounds__(THREADS) void k_flow_inverse(FGeo g, int nl, const 
 {
 	extern __shared__ float th[];
 	__shared__ FlowShared sh;
-	__shared__ float Ys[16][256];
 	const int c = blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
 	for (int i = threadIdx.x; i < 2 * g.V; i += THREADS)
 		th[i] = theta_in[(long)c * 2 * g.V + i];
@@ -239,32 +240,17 @@ __global__ __launch_bounds__(THREADS) void k_flow_inverse(FGeo g, int nl, const 
 	__syncthreads();
 	for (int x = threadIdx.x; x < g.V; x += THREADS)
 		v[1] += 1.0 - cos((double)plaqf(g, th, x / g.L1, x % g.L1));
-	const int NT = (g.NA + 15) / 16;
+	WeightRegsP<NI, THREADS> wr;
+	wr.load(params + (long)(nl - 1) * NP_LAYER);
+	zero_pad<NI>(sh.lw);
 	for (int layer = nl - 1; layer >= 0; --layer)
 	{
-		const int mu = layer & 1, a = (layer >> 1) & 3;
 		__syncthreads();
-		load_weights<NI>(sh.lw, params + layer * NP_LAYER);
+		wr.store(sh.lw);
 		__syncthreads();
-		for (int it = 0; it < NT; it += 16)
-		{
-			mlp_round(g, th, mu, a, it, NT, sh, Ys);
-			__syncthreads();
-			const int r = it * 16 + threadIdx.x;
-			if (r < g.NA)
-			{
-				int y0, y1;
-				active_corner(g, mu, a, r, y0, y1);
-				NCP p = ncp_params(&Ys[threadIdx.x >> 4][(threadIdx.x & 15) * 16]);
-				float tpn = plaqf(g, th, y0, y1);
-				float Gp;
-				float u = ncp_inverse(p, wrapf(tpn - p.t), Gp);
-				int ul = updated_link(g, mu, y0, y1);
-				th[ul] = wrapf(th[ul] - tpn + u + p.t);
-				v[0] += (double)logf(Gp);
-			}
-			__syncthreads();
-		}
+		if (layer > 0)
+			wr.load(params + (long)(layer - 1) * NP_LAYER);
+		layer_apply<true>(g, th, layer & 1, (layer >> 1) & 3, sh, v[0]);
 	}
 	__syncthreads();
 	for (int q = 0; q < 2; ++q)
@@ -302,7 +288,7 @@ __global__ __launch_bounds__(THREADS) void k_flow_backward(FGeo g, int nl, const
 	float *ab = dyn + 2 * g.V;      // 2V: adjoint w.r.t. the current layer's output
 	float *gp = dyn + 4 * g.V;      // V: plaquette gradients of the layer
 	float *gact = dyn + 5 * g.V;    // NA: dL/dtheta_P of the active plaquettes
-	__shared__ FlowShared sh;
+	__shared__ FlowSharedB sh;
 	const int c = blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
 	float *dx = dxs + (long)c * g.NA * NI;
 	float *part = partial + (long)c * nl * NP_LAYER;
@@ -319,54 +305,56 @@ __global__ __launch_bounds__(THREADS) void k_flow_backward(FGeo g, int nl, const
 		ab[x] = beta * (gp[x] - gp[site(g, x0, x1 - 1)]);
 		ab[g.V + x] = beta * (gp[site(g, x0 - 1, x1)] - gp[x]);
 	}
-	const int NT = (g.NA + 15) / 16;
+	const int ntile = (g.NA + 15) / 16;
+	WeightRegsP<NI, THREADS> wr;
+	wr.load(params + (long)(nl - 1) * NP_LAYER);
+	zero_pad<NI>(sh.lw);
 	for (int layer = nl - 1; layer >= 0; --layer)
 	{
 		const int mu = layer & 1, a = (layer >> 1) & 3;
 		__syncthreads();
 		for (int i = threadIdx.x; i < 2 * g.V; i += THREADS)
 			th[i] = theta_layers[((long)c * nl + layer) * 2 * g.V + i];
-		load_weights<NI>(sh.lw, params + layer * NP_LAYER);
+		wr.store(sh.lw);
 		__syncthreads();
-		Grad<NI> gr;
+		if (layer > 0)
+			wr.load(params + (long)(layer - 1) * NP_LAYER);
+		GradP<NI> gr;
 		gr.zero();
-		for (int it = 0; it < (NT + 3) / 4; ++it)
+		// four tiles a round; a wavefront past the last tile repeats the last
+		// row with dL/dy = 0
+		for (int t0 = 0; t0 < ntile; t0 += 4)
 		{
-			const int tix = it * 4 + w;
-			TileF &T = sh.tile[w];
-			if (tix < NT)
+			const int r = (t0 + w) * 16 + (l & 15); // this lane's row in the MLP
+			float x[NI / 4], *y = sh.buf.y[w];
+			features(g, th, mu, a, min(r, g.NA - 1), x);
+			f4 h1[4], h2[4], dxr[GradP<NI>::NB];
+			put_outputs(y, mlp_rows<NI, false, true>(sh.lw, x, [&](int s) { return feature_row(l >> 4, s); }, h1, h2));
+			wave_sync();
 			{
-				features(g, th, mu, a, tix * 16, T);
-				wave_sync();
-				mlp_forward<NI>(sh.lw, T);
-				// output adjoints of the 16 rows (lanes 0..15 own one row each):
 				// the updated link moves by g(u) + t - theta_P, so its adjoint A
 				// reaches theta_P as A (g' - 1) plus the log-det term
-				if (l < 16)
-				{
-					float dy[16];
-					for (int k = 0; k < 16; ++k)
-						dy[k] = 0.f;
-					int r = tix * 16 + l;
-					if (r < g.NA)
-					{
-						int y0, y1;
-						active_corner(g, mu, a, r, y0, y1);
-						const float *y = T.y() + l * 16;
-						float tp = plaqf(g, th, y0, y1);
-						float A = ab[updated_link(g, mu, y0, y1)];
-						gact[r] = ncp_adjoint(y, wrapf(tp - ncp_params(y).t), A, dy) - A;
-					}
-					for (int k = 0; k < 16; ++k)
-						T.y()[l * 16 + k] = dy[k];
-				}
-				wave_sync();
-				mlp_backward<NI>(sh.lw, T, gr, dx, tix * 16, g.NA);
+				const int rq = (t0 + w) * 16 + (l >> 2); // the quad's row in the map
+				const bool live = rq < g.NA;
+				int y0, y1;
+				active_corner(g, mu, a, min(rq, g.NA - 1), y0, y1);
+				float *yr = y + (l >> 2) * YS;
+				const NCPq p = ncpq_params(yr);
+				const float A = ab[updated_link(g, mu, y0, y1)];
+				const float da = ncpq_adjoint(p, yr, wrapf(plaqf(g, th, y0, y1) - p.t), A, live);
+				if (live && (l & 3) == 0)
+					gact[rq] = da - A;
 			}
-			__syncthreads();
+			wave_sync();
+			mlp_rows_backward<NI>(sh.lw, sh.buf, x, feature_row, h1, h2, gr, dxr);
+			if (r < g.NA)
+#pragma unroll
+				for (int s = 0; s < NI / 4; ++s)
+					dx[(long)r * NI + feature_row(l >> 4, s)] = dxr[s / 4][s & 3];
 		}
-		// per-configuration weight gradients of this layer, waves in order
-		store_grad<NI>(gr, part + layer * NP_LAYER);
+		__syncthreads();
+		// per-configuration weight gradients of this layer
+		store_grad<NI>(gr, feature_row, part + (long)layer * NP_LAYER);
 		// plaquette gradients: active from gact, frozen from the feature adjoints
 		for (int x = threadIdx.x; x < g.V; x += THREADS)
 		{
@@ -416,19 +404,6 @@ __global__ __launch_bounds__(THREADS) void k_flow_backward(FGeo g, int nl, const
 			ab[g.V + x] += gp[site(g, x0 - 1, x1)] - gp[x];
 		}
 	}
-}
-
-// grad[i] = scale * sum_c partial[c][i] (fixed order)
-__global__ void k_flow_reduce(int n, const float *__restrict__ partial, int batch, float scale,
-                              float *__restrict__ grad)
-{
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	double s = 0.0;
-	for (int c = 0; c < batch; ++c)
-		s += partial[(long)c * n + i];
-	grad[i] = (float)(s * scale);
 }
 
 // Adam (Kingma & Ba 2015)
@@ -591,7 +566,7 @@ int mesh_flow_gradient(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers,
 	k_flow_backward<<<batch, THREADS, lds, ctx->stream>>>(fg, layers, params, tl, samp, (float)beta, dxs, part);
 	MESH_LAUNCHED(ctx);
 	int n = layers * NP_LAYER;
-	k_flow_reduce<<<(n + 255) / 256, 256, 0, ctx->stream>>>(n, part, batch, 1.0f / batch, grad);
+	k_grad_reduce<<<(n + 63) / 64, 256, 0, ctx->stream>>>(n, part, batch, 1.0f / batch, grad);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }

@@ -6,8 +6,9 @@
 //   h(a) = g(wrap(a - t)) + t,  g(u) = sum_k w_k 2 atan(s_k tan(u / 2))
 // (a mixture of NK = 4 non-compact projections; s_k = exp(clamp(y_k, -8, 8)),
 // w = softmax(y_{4..7}), t = atan2(y_9, y_8)).  The dense layers run on FP32
-// MFMA (v_mfma_f32_16x16x4_f32) in 16-row tiles, one tile per wavefront; the
-// backward pass forms the weight gradients as MFMA tile products.
+// MFMA (v_mfma_f32_16x16x4_f32) in 16-row tiles, one tile per wavefront, with
+// the activations in registers; the backward pass forms the weight gradients
+// as MFMA products over the rows of four tiles.
 //
 // Parameters of one layer, in order: W1 [NI][64], b1 [64], W2 [64][64],
 // b2 [64], W3 [64][10], b3 [10].
@@ -31,7 +32,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 template <int NI> struct Layout
 {
 	static_assert(NI % 4 == 0 && NI <= 48, "features: a multiple of 4, at most 48");
-	static constexpr int XS = (NI + 15) / 16 * 16; // feature row stride of a tile
 	static constexpr int OW1 = 0, OB1 = OW1 + NI * NH, OW2 = OB1 + NH, OB2 = OW2 + NH * NH, OW3 = OB2 + NH,
 	                     OB3 = OW3 + NH * NO, NP = OB3 + NO;
 };
@@ -50,115 +50,6 @@ __device__ __forceinline__ float wrapf(float a)
 	return a >= PI_F ? a - TWO_PI_F : (a < -PI_F ? a + TWO_PI_F : a);
 }
 
-// D(16x16) = sum_k A(i,k) B(k,n), A(i,k) = A[i*sai + k*sak], B(k,n) = B[k*sbk + n*sbn],
-// k < K (multiple of 4).  Lane l supplies A(l%16, k0 + l/16) and
-// B(k0 + l/16, l%16); it receives D(4*(l/16) + j, l%16), j < 4.
-__device__ __forceinline__ f4 tile_mm(const float *A, int sai, int sak, const float *B, int sbk, int sbn, int K)
-{
-	int l = threadIdx.x & 63, i = l & 15, kk = l >> 4;
-	f4 acc = {0.f, 0.f, 0.f, 0.f};
-	for (int k0 = 0; k0 < K; k0 += 4)
-		acc = __builtin_amdgcn_mfma_f32_16x16x4f32(A[i * sai + (k0 + kk) * sak], B[(k0 + kk) * sbk + i * sbn], acc,
-		                                           0, 0, 0);
-	return acc;
-}
-
-// LDS image of one layer's weights (W3/b3 padded to 16 columns)
-template <int NI> struct LW
-{
-	float w1[NI * NH], b1[NH], w2[NH * NH], b2[NH], w3[NH * 16], b3[16];
-};
-
-template <int NI> __device__ void load_weights(LW<NI> &lw, const float *__restrict__ p)
-{
-	using Y = Layout<NI>;
-	for (int i = threadIdx.x; i < NI * NH; i += blockDim.x)
-		lw.w1[i] = p[Y::OW1 + i];
-	for (int i = threadIdx.x; i < NH * NH; i += blockDim.x)
-		lw.w2[i] = p[Y::OW2 + i];
-	for (int i = threadIdx.x; i < NH * 16; i += blockDim.x)
-	{
-		int k = i / 16, n = i % 16;
-		lw.w3[i] = n < NO ? p[Y::OW3 + k * NO + n] : 0.f;
-	}
-	for (int i = threadIdx.x; i < NH; i += blockDim.x)
-	{
-		lw.b1[i] = p[Y::OB1 + i];
-		lw.b2[i] = p[Y::OB2 + i];
-	}
-	for (int i = threadIdx.x; i < 16; i += blockDim.x)
-		lw.b3[i] = i < NO ? p[Y::OB3 + i] : 0.f;
-}
-
-// per-wavefront tile scratch: features (row stride XS; the columns from NI on
-// must be finite), two hidden layers h1, h2() and the outputs y().  SEP = false
-// (kernels without a backward pass, which needs every layer's values) puts h2
-// over h1 and the outputs over the features, each consumed by then: 5 KB less
-// LDS per tile.
-template <int NI, bool SEP = true> struct Tile
-{
-	float x[16 * Layout<NI>::XS], h1[16 * NH];
-	float h2s[SEP ? 16 * NH : 1];
-	float ys[SEP ? 16 * 16 : 1];
-	__device__ float *h2() { return SEP ? h2s : h1; }
-	__device__ float *y() { return SEP ? ys : x; }
-};
-
-// One layer's parameters held in registers (two floats a lane per chunk) so
-// that the next layer's global loads overlap the current layer's work; NP is
-// even for every NI, so each layer starts 8-byte aligned.  store() writes the
-// LDS image: w1, b1, w2, b2 in the parameters' own order, W3/b3 into their
-// 16-column padding (the pad stays as zero_pad() left it).
-template <int NI, int THREADS> struct WeightRegs
-{
-	using Y = Layout<NI>;
-	static_assert(Y::NP % 2 == 0 && Y::OW3 % 2 == 0 && Y::OB3 % 2 == 0 && NO % 2 == 0, "pairs of parameters");
-	static constexpr int NC = Y::NP / 2;
-	static constexpr int PER = (NC + THREADS - 1) / THREADS;
-	float2 v[PER];
-
-	__device__ void load(const float *__restrict__ p)
-	{
-		const float2 *q = reinterpret_cast<const float2 *>(p);
-		for (int i = 0; i < PER; ++i)
-		{
-			const int c = threadIdx.x + i * THREADS;
-			if (c < NC)
-				v[i] = q[c];
-		}
-	}
-	__device__ void store(LW<NI> &lw) const
-	{
-		static_assert(offsetof(LW<NI>, w3) == Y::OW3 * sizeof(float), "w1, b1, w2, b2 as in the parameters");
-		float2 *head = reinterpret_cast<float2 *>(&lw);
-		for (int i = 0; i < PER; ++i)
-		{
-			const int c = threadIdx.x + i * THREADS, idx = 2 * c;
-			if (c >= NC)
-				break;
-			if (idx < Y::OW3)
-				head[c] = v[i];
-			else if (idx < Y::OB3)
-			{
-				const int k = (idx - Y::OW3) / NO, n = idx - Y::OW3 - k * NO;
-				*reinterpret_cast<float2 *>(&lw.w3[k * 16 + n]) = v[i];
-			}
-			else
-				*reinterpret_cast<float2 *>(&lw.b3[idx - Y::OB3]) = v[i];
-		}
-	}
-};
-
-// zero the W3/b3 padding columns NO..15 once per kernel (store() never writes them)
-template <int NI> __device__ void zero_pad(LW<NI> &lw)
-{
-	for (int i = threadIdx.x; i < NH * 16; i += blockDim.x)
-		if (i % 16 >= NO)
-			lw.w3[i] = 0.f;
-	if (threadIdx.x < 16 && threadIdx.x >= NO)
-		lw.b3[threadIdx.x] = 0.f;
-}
-
 // tanh from the hardware exponential and reciprocal: absolute error a few
 // 1e-7, saturating to +-1 (e = inf or 0)
 __device__ __forceinline__ float tanh_fast(float x)
@@ -168,44 +59,6 @@ __device__ __forceinline__ float tanh_fast(float x)
 }
 
 template <bool FAST> __device__ __forceinline__ float act(float x) { return FAST ? tanh_fast(x) : tanhf(x); }
-
-// MLP forward of one tile: h1 = tanh(x W1 + b1), h2 = tanh(h1 W2 + b2), y = h2 W3 + b3
-// (FAST: tanh_fast; a flow uses one choice in all of its kernels)
-template <int NI, bool FAST = false, bool SY = true> __device__ void mlp_forward(LW<NI> const &lw, Tile<NI, SY> &T)
-{
-	constexpr int XS = Layout<NI>::XS;
-	int l = threadIdx.x & 63, c = l & 15, rq = (l >> 4) * 4;
-	for (int n0 = 0; n0 < NH; n0 += 16)
-	{
-		f4 d = tile_mm(T.x, XS, 1, lw.w1 + n0, NH, 1, NI);
-		for (int j = 0; j < 4; ++j)
-			T.h1[(rq + j) * NH + n0 + c] = act<FAST>(d[j] + lw.b1[n0 + c]);
-	}
-	wave_sync();
-	if constexpr (SY)
-		for (int n0 = 0; n0 < NH; n0 += 16)
-		{
-			f4 d = tile_mm(T.h1, NH, 1, lw.w2 + n0, NH, 1, NH);
-			for (int j = 0; j < 4; ++j)
-				T.h2()[(rq + j) * NH + n0 + c] = act<FAST>(d[j] + lw.b2[n0 + c]);
-		}
-	else
-	{
-		// h2() is h1's storage: all four column blocks of h1 W2 first
-		f4 d2[NH / 16];
-		for (int n0 = 0; n0 < NH; n0 += 16)
-			d2[n0 / 16] = tile_mm(T.h1, NH, 1, lw.w2 + n0, NH, 1, NH);
-		wave_sync();
-		for (int n0 = 0; n0 < NH; n0 += 16)
-			for (int j = 0; j < 4; ++j)
-				T.h2()[(rq + j) * NH + n0 + c] = act<FAST>(d2[n0 / 16][j] + lw.b2[n0 + c]);
-	}
-	wave_sync();
-	f4 d = tile_mm(T.h2(), NH, 1, lw.w3, 16, 1, NH);
-	for (int j = 0; j < 4; ++j)
-		T.y()[(rq + j) * 16 + c] = d[j] + lw.b3[c];
-	wave_sync();
-}
 
 // ---- the MLP on one wavefront with the activations in registers -----------
 //
@@ -231,10 +84,10 @@ template <int NI> struct alignas(16) LWP
 	float w1[NI * WS], b1[NH], w2[NH * WS], b2[NH], w3[NH * W3S], b3[16];
 };
 
-// One layer's parameters held in registers (two floats a lane per chunk) so
-// that the next layer's global loads overlap the current layer's work; NP is
-// even for every NI, so each layer starts 8-byte aligned.  store() writes the
-// LDS image (the pad columns of W3/b3 stay as zero_pad() left them).
+// One layer's parameters held in registers (two floats a lane per chunk, from
+// 4-byte aligned memory) so that the next layer's global loads overlap the
+// current layer's work.  store() writes the LDS image (the pad columns of
+// W3/b3 stay as zero_pad() left them).
 template <int NI, int THREADS> struct WeightRegsP
 {
 	using Y = Layout<NI>;
@@ -243,11 +96,15 @@ template <int NI, int THREADS> struct WeightRegsP
 	              "pairs of parameters");
 	static constexpr int NC = Y::NP / 2;
 	static constexpr int PER = (NC + THREADS - 1) / THREADS;
-	float2 v[PER];
+	struct __attribute__((packed, aligned(4))) Pair
+	{
+		float x, y;
+	};
+	Pair v[PER];
 
 	__device__ void load(const float *__restrict__ p)
 	{
-		const float2 *q = reinterpret_cast<const float2 *>(p);
+		const Pair *q = reinterpret_cast<const Pair *>(p);
 #pragma unroll
 		for (int i = 0; i < PER; ++i)
 		{
@@ -277,7 +134,7 @@ template <int NI, int THREADS> struct WeightRegsP
 				dst = lw.w3 + ((x - Y::OW3) / NO) * W3S + (x - Y::OW3) % NO;
 			else
 				dst = lw.b3 + (x - Y::OB3);
-			*reinterpret_cast<float2 *>(dst) = v[i];
+			*reinterpret_cast<float2 *>(dst) = make_float2(v[i].x, v[i].y);
 		}
 	}
 };
@@ -408,83 +265,6 @@ __device__ __forceinline__ void put_outputs(float *y, f4 v)
 {
 	const int l = threadIdx.x & 63;
 	*reinterpret_cast<f4 *>(y + (l & 15) * YS + (l >> 4) * 4) = v;
-}
-
-// transform parameters from the MLP outputs
-struct NCP
-{
-	float s[NK], w[NK], t, ta, tb;
-};
-
-__device__ __forceinline__ NCP ncp_params(const float *y)
-{
-	NCP p;
-	float m = y[NK];
-	for (int k = 1; k < NK; ++k)
-		m = fmaxf(m, y[NK + k]);
-	float z = 0.f;
-	for (int k = 0; k < NK; ++k)
-	{
-		p.s[k] = expf(fminf(fmaxf(y[k], -8.f), 8.f));
-		p.w[k] = expf(y[NK + k] - m);
-		z += p.w[k];
-	}
-	for (int k = 0; k < NK; ++k)
-		p.w[k] /= z;
-	p.ta = y[2 * NK];
-	p.tb = y[2 * NK + 1];
-	p.t = atan2f(p.tb, p.ta);
-	return p;
-}
-
-// g(u), g'(u) of the mixture
-__device__ __forceinline__ void ncp_eval(NCP const &p, float u, float &G, float &Gp)
-{
-	float c = cosf(0.5f * u), sn = sinf(0.5f * u);
-	G = 0.f;
-	Gp = 0.f;
-	for (int k = 0; k < NK; ++k)
-	{
-		float d = fmaf(c, c, p.s[k] * p.s[k] * sn * sn);
-		G = fmaf(p.w[k], 2.f * atan2f(p.s[k] * sn, c), G);
-		Gp = fmaf(p.w[k], p.s[k] / d, Gp);
-	}
-}
-
-// u = g^-1(target): g is increasing on [-pi, pi] with g(+-pi) = +-pi, so
-// Newton steps inside a bracket that every evaluation narrows, bisection when
-// a step leaves it, until a step or the bracket is below 2e-7 max(1, |u|)
-// (an FP32 ulp of u is up to 2.4e-7 here, so an absolute bound could not stop
-// an iterate that alternates between neighbouring floats; at most 40
-// evaluations).  Returns u, and g'(u) in Gp.
-__device__ __forceinline__ float ncp_inverse(NCP const &p, float target, float &Gp)
-{
-	float lo = -PI_F, hi = PI_F, u = target, G;
-	for (int b = 0; b < 40; ++b)
-	{
-		ncp_eval(p, u, G, Gp);
-		float f = G - target;
-		if (f == 0.f)
-			break;
-		if (f < 0.f)
-			lo = u;
-		else
-			hi = u;
-		if (hi - lo <= 2e-7f * fmaxf(1.f, fabsf(u)))
-			break;
-		float un = u - f / Gp;
-		if (un > lo && un < hi)
-		{
-			bool done = fabsf(un - u) <= 2e-7f * fmaxf(1.f, fabsf(un));
-			u = un;
-			if (done)
-				break;
-		}
-		else
-			u = 0.5f * (lo + hi);
-	}
-	ncp_eval(p, u, G, Gp);
-	return u;
 }
 
 // ---- elementary functions of the quad maps below, for the ranges they meet.
@@ -648,169 +428,242 @@ __device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float
 }
 
 // Adjoints of L = A (g(u) + t) - log g'(u), u = wrap(a - t), for one active
-// variable a with MLP outputs y: dy[16] = dL/dy (through s, w and t), and
-// the return value dL/da.
-__device__ __forceinline__ float ncp_adjoint(const float *y, float u, float A, float (&dy)[16])
+// variable a with MLP outputs y[16] on its quad: overwrites y with dL/dy
+// (through s, w and t; the columns from NO on zero) and returns dL/da in every
+// lane of the quad.  live = false: a row without a variable, dL/dy = 0.
+__device__ __forceinline__ float ncpq_adjoint(NCPq const &p, float *y, float u, float A, bool live)
 {
-	NCP p = ncp_params(y);
-	float cc = cosf(0.5f * u), sn = sinf(0.5f * u);
-	float Gp = 0.f, Gpp = 0.f, gk[NK], gpk[NK], dgs[NK], dgps[NK];
-	for (int k = 0; k < NK; ++k)
-	{
-		float s2 = p.s[k] * p.s[k];
-		float d = fmaf(cc, cc, s2 * sn * sn);
-		gk[k] = 2.f * atan2f(p.s[k] * sn, cc);
-		gpk[k] = p.s[k] / d;
-		dgs[k] = 2.f * sn * cc / d;
-		dgps[k] = (cc * cc - s2 * sn * sn) / (d * d);
-		Gp = fmaf(p.w[k], gpk[k], Gp);
-		Gpp = fmaf(p.w[k], -p.s[k] * (s2 - 1.f) * sn * cc / (d * d), Gpp);
-	}
-	float iG = 1.f / Gp;
-	float dLdt = A * (1.f - Gp) + Gpp * iG;
-	float dLdw[NK], sw = 0.f;
-	for (int k = 0; k < 16; ++k)
-		dy[k] = 0.f;
-	for (int k = 0; k < NK; ++k)
-	{
-		dLdw[k] = A * gk[k] - gpk[k] * iG;
-		sw = fmaf(p.w[k], dLdw[k], sw);
-		float dLds = p.w[k] * (A * dgs[k] - dgps[k] * iG);
-		dy[k] = (y[k] > -8.f && y[k] < 8.f) ? p.s[k] * dLds : 0.f;
-	}
-	for (int k = 0; k < NK; ++k)
-		dy[NK + k] = p.w[k] * (dLdw[k] - sw);
-	float r2 = fmaf(p.ta, p.ta, p.tb * p.tb) + 1e-20f;
-	dy[2 * NK] = dLdt * (-p.tb / r2);
-	dy[2 * NK + 1] = dLdt * (p.ta / r2);
+	const int k = threadIdx.x & 3;
+	float sn, c;
+	sincos1(0.5f * u, sn, c);
+	const float s2 = p.s * p.s, d = fmaf(c, c, s2 * sn * sn), id = div1(1.f, d);
+	const float g = 2.f * atan2_1(p.s * sn, c), gp = p.s * id;
+	const float dgs = 2.f * sn * c * id, dgps = (c * c - s2 * sn * sn) * (id * id);
+	const float Gp = quad_sum(p.w * gp), Gpp = quad_sum(p.w * (-p.s * (s2 - 1.f) * sn * c * (id * id)));
+	const float iG = div1(1.f, Gp);
+	const float dLdt = A * (1.f - Gp) + Gpp * iG;
+	const float dLdw = A * g - gp * iG, sw = quad_sum(p.w * dLdw);
+	const float yk = y[k], ta = y[2 * NK], tb = y[2 * NK + 1];
+	const float r2 = fmaf(ta, ta, tb * tb) + 1e-20f;
+	wave_sync(); // every lane of the quad has read y
+	y[k] = live && yk > -8.f && yk < 8.f ? p.s * (p.w * (A * dgs - dgps * iG)) : 0.f;
+	y[NK + k] = live ? p.w * (dLdw - sw) : 0.f;
+	y[2 * NK + k] = live && k < 2 ? dLdt * ((k ? ta : -tb) / r2) : 0.f;
+	y[2 * NK + 4 + k] = 0.f;
 	return A * Gp - Gpp * iG;
 }
 
-// Weight-gradient accumulators of one wavefront (lane-owned tile fragments)
-template <int NI> struct Grad
+// ---- backward of four tiles, one on each of a workgroup's four wavefronts
+//
+// The adjoints run back through the layers in registers just as the
+// activations ran forward (mlp_rows).  The weight gradients contract over the
+// rows: the tiles' activations and adjoints go to LDS transposed, [column]
+// [row], and wavefront w forms block w of the gradient's columns (of W3: of its
+// rows) over the 64 rows of all four tiles, so that no sum over the wavefronts
+// is left and a wavefront's accumulators are a quarter of the gradient.  Row
+// stride TS: 16 consecutive columns are read from 16 different groups of four
+// banks, and a column's 16 rows written to 16 banks.
+constexpr int TS = 20;
+
+template <int NI> struct BackBuf
 {
-	static constexpr int NX = Layout<NI>::XS / 16;
-	f4 w1[NX * 4], w2[16], w3[4];
+	alignas(16) float a[4][NH * TS], b[4][NH * TS];
+	alignas(16) float y[4][16 * TS]; // outputs of mlp_rows, then dL/dy, then its transpose (YS = TS)
+	static_assert(YS == TS && NI <= NH, "the outputs and their transpose share their storage");
+};
+
+// gradient accumulators of wavefront w: columns 16 w + l % 16 of W1 (rows: the
+// features row(4 b + j) of the lane's quarter) and W2 (rows 16 b + 4 q + j),
+// rows 16 w + 4 q + j of W3, and the biases' sums over the lane's rows
+template <int NI> struct GradP
+{
+	static constexpr int NB = (NI / 4 + 3) / 4; // blocks of four features of a quarter
+	f4 w1[NB], w2[4], w3;
 	float b1, b2, b3;
 	__device__ void zero()
 	{
-		for (int q = 0; q < NX * 4; ++q)
-			w1[q] = f4{0.f, 0.f, 0.f, 0.f};
-		for (int q = 0; q < 16; ++q)
-			w2[q] = f4{0.f, 0.f, 0.f, 0.f};
-		for (int q = 0; q < 4; ++q)
-			w3[q] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+		for (int b = 0; b < NB; ++b)
+			w1[b] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+		for (int b = 0; b < 4; ++b)
+			w2[b] = f4{0.f, 0.f, 0.f, 0.f};
+		w3 = f4{0.f, 0.f, 0.f, 0.f};
 		b1 = b2 = b3 = 0.f;
 	}
 };
 
-// MLP backward of one tile whose T.y() holds dL/dy (and T.x, T.h1, T.h2() the
-// forward values): accumulates the weight gradients into G and writes
-// dL/dx of rows r0 .. r0+15 (r < nrows) to dx[r * NI + feature]
-template <int NI>
-__device__ void mlp_backward(LW<NI> const &lw, Tile<NI> &T, Grad<NI> &G, float *__restrict__ dx, int r0, int nrows)
+__device__ __forceinline__ f4 mm4(f4 a, f4 b, f4 c)
 {
-	constexpr int XS = Layout<NI>::XS;
-	const int l = threadIdx.x & 63, lc = l & 15, rq = (l >> 4) * 4;
-	// dW3 += H2^T dY, db3
-	for (int i0 = 0; i0 < NH; i0 += 16)
-		G.w3[i0 / 16] += tile_mm(T.h2() + i0, 1, NH, T.y(), 16, 1, 16);
-	if (l < 16)
-		for (int rr = 0; rr < 16; ++rr)
-			G.b3 += T.y()[rr * 16 + l];
-	// dA2 = (dY W3^T) * (1 - h2^2), into h2
-	f4 dh2[4];
-	for (int n0 = 0; n0 < NH; n0 += 16)
-		dh2[n0 / 16] = tile_mm(T.y(), 16, 1, lw.w3 + n0 * 16, 1, 16, 16);
-	wave_sync();
-	for (int n0 = 0; n0 < NH; n0 += 16)
-		for (int j = 0; j < 4; ++j)
-		{
-			float hv = T.h2()[(rq + j) * NH + n0 + lc];
-			T.h2()[(rq + j) * NH + n0 + lc] = dh2[n0 / 16][j] * (1.f - hv * hv);
-		}
-	wave_sync();
-	// dW2 += H1^T dA2, db2
-	for (int i0 = 0; i0 < NH; i0 += 16)
-		for (int n0 = 0; n0 < NH; n0 += 16)
-			G.w2[(i0 / 16) * 4 + n0 / 16] += tile_mm(T.h1 + i0, 1, NH, T.h2() + n0, NH, 1, 16);
-	for (int rr = 0; rr < 16; ++rr)
-		G.b2 += T.h2()[rr * NH + l];
-	// dA1 = (dA2 W2^T) * (1 - h1^2), into h1
-	f4 dh1[4];
-	for (int n0 = 0; n0 < NH; n0 += 16)
-		dh1[n0 / 16] = tile_mm(T.h2(), NH, 1, lw.w2 + n0 * NH, 1, NH, NH);
-	wave_sync();
-	for (int n0 = 0; n0 < NH; n0 += 16)
-		for (int j = 0; j < 4; ++j)
-		{
-			float hv = T.h1[(rq + j) * NH + n0 + lc];
-			T.h1[(rq + j) * NH + n0 + lc] = dh1[n0 / 16][j] * (1.f - hv * hv);
-		}
-	wave_sync();
-	// dW1 += X^T dA1, db1
-	for (int i0 = 0; i0 < XS; i0 += 16)
-		for (int n0 = 0; n0 < NH; n0 += 16)
-			G.w1[(i0 / 16) * 4 + n0 / 16] += tile_mm(T.x + i0, 1, XS, T.h1 + n0, NH, 1, 16);
-	for (int rr = 0; rr < 16; ++rr)
-		G.b1 += T.h1[rr * NH + l];
-	// dX = dA1 W1^T (feature columns < NI)
-	for (int n0 = 0; n0 < XS; n0 += 16)
-	{
-		f4 dxt = tile_mm(T.h1, NH, 1, lw.w1 + n0 * NH, 1, NH, NH);
-		for (int j = 0; j < 4; ++j)
-		{
-			int r = r0 + rq + j, f = n0 + lc;
-			if (f < NI && r < nrows)
-				dx[(long)r * NI + f] = dxt[j];
-		}
-	}
-	wave_sync();
+#pragma unroll
+	for (int j = 0; j < 4; ++j)
+		c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+	return c;
 }
 
-// the four wavefronts' accumulators, added in wavefront order, into the
-// layer's per-configuration gradient pl[0 .. NP)
-template <int NI> __device__ void store_grad(Grad<NI> const &G, float *__restrict__ pl)
+// a lane's columns 16 b + 4 q + j of its row to t[column * TS + row]
+template <int NB> __device__ __forceinline__ void put_columns(float *t, f4 const (&v)[NB])
+{
+	const int l = threadIdx.x & 63, q4 = (l >> 4) * 4;
+#pragma unroll
+	for (int b = 0; b < NB; ++b)
+#pragma unroll
+		for (int j = 0; j < 4; ++j)
+			t[(16 * b + q4 + j) * TS + (l & 15)] = v[b][j];
+}
+
+// One round: x, h1, h2 from mlp_rows on this wavefront's tile; B.y[w] holds
+// its dL/dy (ncpq_adjoint).  Adds to G and returns in dx[b][j] the adjoint of
+// feature row(q, 4 b + j), q the lane's quarter.  Called by all 256 threads.
+template <int NI, class ROW>
+__device__ __forceinline__ void mlp_rows_backward(LWP<NI> const &lw, BackBuf<NI> &B, const float (&x)[NI / 4], ROW row,
+                                                  f4 const (&h1)[4], f4 const (&h2)[4], GradP<NI> &G,
+                                                  f4 (&dx)[GradP<NI>::NB])
+{
+	constexpr int NS = NI / 4, NB = GradP<NI>::NB;
+	const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, q4 = (l >> 4) * 4;
+	const f4 zero = {0.f, 0.f, 0.f, 0.f};
+	auto sum = [](f4 v) { return (v[0] + v[1]) + (v[2] + v[3]); };
+	auto at = [&](const float *t, int c) { return *reinterpret_cast<const f4 *>(t + (c + i) * TS + q4); };
+	f4 dy[1] = {*reinterpret_cast<const f4 *>(B.y[w] + i * TS + q4)};
+	wave_sync();
+	put_columns(B.y[w], dy);
+	put_columns(B.a[w], h2);
+	__syncthreads();
+	// dW3 = H2^T dY, dA2 = (dY W3^T) (1 - h2^2)
+	f4 d2[4], d1[4];
+#pragma unroll
+	for (int t = 0; t < 4; ++t)
+	{
+		const f4 v = at(B.y[t], 0);
+		G.w3 = mm4(at(B.a[t], 16 * w), v, G.w3);
+		G.b3 += sum(v);
+	}
+#pragma unroll
+	for (int b = 0; b < 4; ++b)
+		d2[b] = mm4(*reinterpret_cast<const f4 *>(lw.w3 + (16 * b + i) * W3S + q4), dy[0], zero) * (1.f - h2[b] * h2[b]);
+	__syncthreads();
+	put_columns(B.a[w], h1);
+	put_columns(B.b[w], d2);
+	__syncthreads();
+	// dW2 = H1^T dA2, dA1 = (dA2 W2^T) (1 - h1^2)
+#pragma unroll
+	for (int t = 0; t < 4; ++t)
+	{
+		const f4 v = at(B.b[t], 16 * w);
+		G.b2 += sum(v);
+#pragma unroll
+		for (int b = 0; b < 4; ++b)
+			G.w2[b] = mm4(at(B.a[t], 16 * b), v, G.w2[b]);
+	}
+#pragma unroll
+	for (int b = 0; b < 4; ++b)
+	{
+		f4 acc = zero;
+#pragma unroll
+		for (int k = 0; k < 4; ++k)
+			acc = mm4(*reinterpret_cast<const f4 *>(lw.w2 + (16 * b + i) * WS + 16 * k + q4), d2[k], acc);
+		d1[b] = acc * (1.f - h1[b] * h1[b]);
+	}
+	__syncthreads();
+	f4 xb[NB];
+#pragma unroll
+	for (int b = 0; b < NB; ++b)
+#pragma unroll
+		for (int j = 0; j < 4; ++j)
+			xb[b][j] = 4 * b + j < NS ? x[4 * b + j] : 0.f;
+	put_columns(B.a[w], xb);
+	put_columns(B.b[w], d1);
+	__syncthreads();
+	// dW1 = X^T dA1, dX = dA1 W1^T
+#pragma unroll
+	for (int t = 0; t < 4; ++t)
+	{
+		const f4 v = at(B.b[t], 16 * w);
+		G.b1 += sum(v);
+#pragma unroll
+		for (int b = 0; b < NB; ++b)
+			G.w1[b] = mm4(at(B.a[t], 16 * b), v, G.w1[b]);
+	}
+#pragma unroll
+	for (int b = 0; b < NB; ++b)
+	{
+		// row i of the product: feature 4 b + i % 4 of quarter i / 4 (past NS: any, not used)
+		const int s = 4 * b + (i & 3), f = row(i >> 2, s < NS ? s : 0);
+		f4 acc = zero;
+#pragma unroll
+		for (int k = 0; k < 4; ++k)
+			acc = mm4(*reinterpret_cast<const f4 *>(lw.w1 + f * WS + 16 * k + q4), d1[k], acc);
+		dx[b] = acc;
+	}
+	__syncthreads(); // the buffers are free for the next round
+}
+
+// a layer's gradient of one configuration, pl[0 .. NP)
+template <int NI, class ROW> __device__ __forceinline__ void store_grad(GradP<NI> const &G, ROW row, float *__restrict__ pl)
 {
 	using Y = Layout<NI>;
-	constexpr int XS = Y::XS;
-	const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lc = l & 15, rq = (l >> 4) * 4;
-	for (int ww = 0; ww < 4; ++ww)
+	const int w = threadIdx.x >> 6, l = threadIdx.x & 63, i = l & 15, q = l >> 4, n = 16 * w + i;
+#pragma unroll
+	for (int b = 0; b < GradP<NI>::NB; ++b)
+#pragma unroll
+		for (int j = 0; j < 4; ++j)
+			if (4 * b + j < NI / 4)
+				pl[Y::OW1 + row(q, 4 * b + j) * NH + n] = G.w1[b][j];
+#pragma unroll
+	for (int b = 0; b < 4; ++b)
+#pragma unroll
+		for (int j = 0; j < 4; ++j)
+			pl[Y::OW2 + (16 * b + 4 * q + j) * NH + n] = G.w2[b][j];
+	if (i < NO)
+#pragma unroll
+		for (int j = 0; j < 4; ++j)
+			pl[Y::OW3 + (16 * w + 4 * q + j) * NO + i] = G.w3[j];
+	// the biases' sums over the quarters
+	auto quarters = [](float v) {
+		v += __shfl_xor(v, 16, 64);
+		return v + __shfl_xor(v, 32, 64);
+	};
+	const float b1 = quarters(G.b1), b2 = quarters(G.b2), b3 = quarters(G.b3);
+	if (q == 0)
 	{
-		if (w == ww)
-		{
-			for (int i0 = 0; i0 < XS; i0 += 16)
-				for (int n0 = 0; n0 < NH; n0 += 16)
-					for (int j = 0; j < 4; ++j)
-					{
-						int k = i0 + rq + j, n = n0 + lc;
-						if (k < NI)
-						{
-							float *dst = pl + Y::OW1 + k * NH + n;
-							*dst = (ww ? *dst : 0.f) + G.w1[(i0 / 16) * 4 + n0 / 16][j];
-						}
-					}
-			for (int i0 = 0; i0 < NH; i0 += 16)
-				for (int n0 = 0; n0 < NH; n0 += 16)
-					for (int j = 0; j < 4; ++j)
-					{
-						float *dst = pl + Y::OW2 + (i0 + rq + j) * NH + n0 + lc;
-						*dst = (ww ? *dst : 0.f) + G.w2[(i0 / 16) * 4 + n0 / 16][j];
-					}
-			for (int i0 = 0; i0 < NH; i0 += 16)
-				for (int j = 0; j < 4; ++j)
-					if (lc < NO)
-					{
-						float *dst = pl + Y::OW3 + (i0 + rq + j) * NO + lc;
-						*dst = (ww ? *dst : 0.f) + G.w3[i0 / 16][j];
-					}
-			pl[Y::OB1 + l] = (ww ? pl[Y::OB1 + l] : 0.f) + G.b1;
-			pl[Y::OB2 + l] = (ww ? pl[Y::OB2 + l] : 0.f) + G.b2;
-			if (l < NO)
-				pl[Y::OB3 + l] = (ww ? pl[Y::OB3 + l] : 0.f) + G.b3;
-		}
-		__syncthreads();
+		pl[Y::OB1 + n] = b1;
+		pl[Y::OB2 + n] = b2;
+		if (w == 0 && i < NO)
+			pl[Y::OB3 + i] = b3;
 	}
+}
+
+// grad[i] = scale * sum_c partial[c][i], in a fixed order: thread group g of
+// four takes the configurations c = g (mod 4), so that four times the loads are
+// in flight (one thread an entry left 930 wavefronts of serial loads on the
+// chip: 62 us for 256 configurations of 8 layers)
+__global__ __launch_bounds__(256) static void k_grad_reduce(int n, const float *__restrict__ partial, int batch,
+                                                            float scale, float *__restrict__ grad)
+{
+	__shared__ double part[4][64];
+	const int g = threadIdx.x >> 6, l = threadIdx.x & 63, i = blockIdx.x * 64 + l;
+	double s = 0.0;
+	if (i < n)
+	{
+		int c = g;
+		for (; c + 28 < batch; c += 32)
+		{
+			float v[8];
+#pragma unroll
+			for (int k = 0; k < 8; ++k)
+				v[k] = partial[(long)(c + 4 * k) * n + i];
+#pragma unroll
+			for (int k = 0; k < 8; ++k)
+				s += v[k];
+		}
+		for (; c < batch; c += 4)
+			s += partial[(long)c * n + i];
+	}
+	part[g][l] = s;
+	__syncthreads();
+	if (g == 0 && i < n)
+		grad[i] = (float)((((part[0][l] + part[1][l]) + part[2][l]) + part[3][l]) * scale);
 }
 
 // initial weights of n parameters (layers of NP each): W ~ N(0, 1/fan_in) for

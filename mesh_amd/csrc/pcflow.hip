@@ -47,7 +47,6 @@ struct PCGeo : u1_plaq::PGeo
 };
 
 constexpr int NI = 40; // features: 20 loops, (cos, sin) each
-constexpr int XS = FM::Layout<NI>::XS;
 constexpr int NP_LAYER = FM::Layout<NI>::NP;
 constexpr int MAX_LAYERS = 64;
 constexpr int THREADS = 256; // of the backward kernel
@@ -60,7 +59,6 @@ constexpr bool FAST = true; // tanh_fast in every kernel of this flow
 constexpr uint32_t TAG_PCFZ = 0x5043465au; // prior, holonomies, gauge
 constexpr uint32_t TAG_PCFI = 0x50434649u; // initial weights
 constexpr double LOG_2PI = 1.8378770664093454836;
-using Weights = FM::WeightRegs<NI, THREADS>;
 
 // offset of ring position k = 0..7 around a plaquette, in order around it
 __device__ __forceinline__ void ring(int k, int &d0, int &d1)
@@ -87,76 +85,10 @@ __device__ __forceinline__ void active_xy(PCGeo const &g, int m, int r, int &x0,
 	x1 = (m >> 1) + 2 * j;
 }
 __device__ __forceinline__ int n_active(PCGeo const &g, int m) { return (g.V >> 2) - (m == 3 ? 1 : 0); }
-__device__ __forceinline__ int class_of(PCGeo const &g, int x) { return ((x / g.L1) & 1) | (((x % g.L1) & 1) << 1); }
-__device__ __forceinline__ int active_index(PCGeo const &g, int x)
-{
-	return ((x / g.L1) >> 1) * (g.L1 >> 1) + ((x % g.L1) >> 1);
-}
-
-// (cos, sin) of context loop k of the plaquette at (x0, x1): k < 8 ring
-// plaquette k; 8 <= k < 16 the 1x2 loop of ring plaquettes k - 8 and k - 7
-// (mod 8); 16 <= k < 20 the L-shaped loop of ring plaquettes 2j - 1, 2j and
-// 2j + 1 (mod 8), j = k - 16 (the 2x2 square at corner 2j without its
-// centre); by angle addition.  cs holds (cos, sin) of every plaquette, (1, 0)
-// for the last, which enters the context as the angle 0.
-__device__ __forceinline__ float2 ring_cs(PCGeo const &g, const float2 *cs, int x0, int x1, int k)
-{
-	int d0, d1;
-	ring(k & 7, d0, d1);
-	return cs[sitew(g, x0 + d0, x1 + d1)];
-}
+// (cos, sin) of the sum of two angles
 __device__ __forceinline__ float2 cs_add(float2 a, float2 b)
 {
 	return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.y, b.x, a.x * b.y));
-}
-__device__ __forceinline__ float2 loop_cs(PCGeo const &g, const float2 *cs, int x0, int x1, int k)
-{
-	if (k < 8)
-		return ring_cs(g, cs, x0, x1, k);
-	if (k < 16)
-		return cs_add(ring_cs(g, cs, x0, x1, k - 8), ring_cs(g, cs, x0, x1, k - 7));
-	const int j = k - 16;
-	return cs_add(cs_add(ring_cs(g, cs, x0, x1, 2 * j + 7), ring_cs(g, cs, x0, x1, 2 * j)),
-	              ring_cs(g, cs, x0, x1, 2 * j + 1));
-}
-
-// features of the 16 active plaquettes r0..r0+15 of class m (rows beyond NA
-// zero): columns 2k, 2k+1 = (cos, sin) of context loop k, the row's columns
-// from NI on zero.  First the 8 ring plaquettes of every row (the only
-// gathers from the configuration), then the 1x2 and L-shaped loops from those
-// columns, by the angle additions of loop_cs in its order (the same bits).
-template <class TILE> __device__ void features(PCGeo const &g, const float2 *cs, int m, int r0, int NA, TILE &T)
-{
-	const int l = threadIdx.x & 63;
-	for (int e = l; e < 16 * 8; e += 64)
-	{
-		const int row = e >> 3, k = e & 7, r = r0 + row;
-		float2 v = make_float2(0.f, 0.f);
-		if (r < NA)
-		{
-			int x0, x1;
-			active_xy(g, m, r, x0, x1);
-			v = ring_cs(g, cs, x0, x1, k);
-		}
-		*reinterpret_cast<float2 *>(&T.x[row * XS + 2 * k]) = v;
-	}
-	FM::wave_sync();
-	for (int e = l; e < 16 * 12; e += 64)
-	{
-		const int row = e / 12, q = e - row * 12;
-		const float2 *rg = reinterpret_cast<const float2 *>(&T.x[row * XS]);
-		float2 v;
-		if (q < 8)
-			v = cs_add(rg[q], rg[(q + 1) & 7]);
-		else
-		{
-			const int j = q - 8;
-			v = cs_add(cs_add(rg[(2 * j + 7) & 7], rg[2 * j]), rg[2 * j + 1]);
-		}
-		*reinterpret_cast<float2 *>(&T.x[row * XS + 16 + 2 * q]) = v;
-	}
-	for (int e = l; e < 16 * (XS - NI); e += 64)
-		T.x[(e / (XS - NI)) * XS + NI + e % (XS - NI)] = 0.f;
 }
 
 __device__ __forceinline__ float2 sincos2(float a)
@@ -173,11 +105,11 @@ template <int NT> struct PCSharedF
 	float y[NT / 64][16 * FM::YS];
 	double red[4][NT / 64];
 };
-// LDS of the backward kernel (outputs apart from the features: they carry dL/dy)
+// LDS of the backward kernel
 struct PCSharedB
 {
-	FM::LW<NI> lw;
-	FM::Tile<NI> tile[4];
+	FM::LWP<NI> lw;
+	FM::BackBuf<NI> buf;
 	double red[4][4];
 };
 
@@ -196,11 +128,11 @@ struct LaneLoops
 		ring(2 * q, d0[1], d1[1]);
 		ring(2 * q + 1, d0[2], d1[2]);
 	}
-	__device__ __forceinline__ int row(int s) const
+	// index of the parameters' feature that is x[s] of quarter q
+	static __device__ __forceinline__ int row(int q, int s)
 	{
 		return s < 4 ? 4 * q + s : (s < 6 ? 12 + 4 * q + s : (s < 8 ? 10 + 2 * ((2 * q + 7) & 7) + s : 24 + 2 * q + s));
 	}
-	// the additions of loop_cs, in its order
 	__device__ __forceinline__ void features(PCGeo const &g, const float2 *cs, int x0, int x1, float (&x)[NI / 4]) const
 	{
 		const float2 a = cs[sitew(g, x0 + d0[0], x1 + d1[0])], b = cs[sitew(g, x0 + d0[1], x1 + d1[1])],
@@ -231,7 +163,7 @@ __device__ __forceinline__ void layer_apply(PCGeo const &g, LaneLoops const &ll,
 		float x[NI / 4];
 		ll.features(g, cs, x0, x1, x);
 		FM::f4 h1[4], h2[4];
-		const FM::f4 out = FM::mlp_rows<NI, FAST, NT == 256>(sh.lw, x, [&](int s) { return ll.row(s); }, h1, h2);
+		const FM::f4 out = FM::mlp_rows<NI, FAST, NT == 256>(sh.lw, x, [&](int s) { return LaneLoops::row(ll.q, s); }, h1, h2);
 		FM::put_outputs(y, out);
 		FM::wave_sync();
 		const int row = l >> 2, r = tix * 16 + row;
@@ -420,12 +352,13 @@ __global__ __launch_bounds__(NT) void k_pc_propose(PCGeo g, int nl, const float 
 // gradient of the per-configuration loss beta S - log det (S with the last
 // plaquette = -sum of the free ones) with respect to every weight:
 // partial[c][layer * NP_LAYER + i].  phi_layers / phi_final from k_pc_forward;
-// dxs: scratch of (V/4) * NI floats per configuration.
+// drs: scratch of (V/4) * 8 floats per configuration, the adjoints of every
+// active plaquette's ring.
 // LDS: cs[V] (of the current layer's input), phi[V], a[V], gact[V/4].
 __global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const float *__restrict__ params,
                                                          const float *__restrict__ phi_layers,
                                                          const float *__restrict__ phi_final, float beta,
-                                                         float *__restrict__ dxs, float *__restrict__ partial)
+                                                         float *__restrict__ drs, float *__restrict__ partial)
 {
 	extern __shared__ float dyn[];
 	float2 *cs = reinterpret_cast<float2 *>(dyn);
@@ -434,8 +367,12 @@ __global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const 
 	float *gact = dyn + 4 * g.V; // adjoint w.r.t. the active plaquettes' input
 	__shared__ PCSharedB sh;
 	const int c = blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
-	float *dx = dxs + (long)c * (g.V >> 2) * NI;
+	float *dr = drs + (long)c * (g.V >> 2) * 8;
 	float *part = partial + (long)c * nl * NP_LAYER;
+	FM::WeightRegsP<NI, THREADS> wr;
+	const LaneLoops ll;
+	auto row = [](int q, int s) { return LaneLoops::row(q, s); };
+	wr.load(params + (long)(nl - 1) * NP_LAYER);
 	FM::zero_pad<NI>(sh.lw);
 	for (int x = threadIdx.x; x < g.V; x += THREADS)
 		phi[x] = phi_final[(long)c * g.V + x];
@@ -448,7 +385,7 @@ __global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const 
 		a[x] = x < g.V - 1 ? beta * (sinf(phi[x]) - sin_last) : 0.f;
 	for (int layer = nl - 1; layer >= 0; --layer)
 	{
-		const int m = layer & 3, NA = n_active(g, m), NT = (NA + 15) / 16;
+		const int m = layer & 3, NA = n_active(g, m), ntile = (NA + 15) / 16;
 		__syncthreads();
 		for (int x = threadIdx.x; x < g.V; x += THREADS)
 		{
@@ -456,99 +393,81 @@ __global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const 
 			phi[x] = p;
 			cs[x] = sincos2(p);
 		}
-		{
-			// no prefetch here: the gradient accumulators need the registers
-			Weights wr;
-			wr.load(params + (long)layer * NP_LAYER);
-			wr.store(sh.lw);
-		}
+		wr.store(sh.lw);
 		__syncthreads();
-		FM::Grad<NI> gr;
+		if (layer > 0)
+			wr.load(params + (long)(layer - 1) * NP_LAYER);
+		FM::GradP<NI> gr;
 		gr.zero();
-		auto &T = sh.tile[w];
-		for (int tix = w; tix < NT; tix += 4)
+		// four tiles a round; a wavefront past the last tile repeats the last
+		// row with dL/dy = 0
+		for (int t0 = 0; t0 < ntile; t0 += 4)
 		{
-			features(g, cs, m, tix * 16, NA, T);
+			const int r = (t0 + w) * 16 + (l & 15); // this lane's row in the MLP
+			int x0, x1;
+			active_xy(g, m, min(r, NA - 1), x0, x1);
+			float x[NI / 4], *y = sh.buf.y[w];
+			ll.features(g, cs, x0, x1, x);
+			FM::f4 h1[4], h2[4], dx[FM::GradP<NI>::NB];
+			const FM::f4 out = FM::mlp_rows<NI, FAST, true>(sh.lw, x, [&](int k) { return row(ll.q, k); }, h1, h2);
+			FM::put_outputs(y, out);
 			FM::wave_sync();
-			FM::mlp_forward<NI, FAST>(sh.lw, T);
-			if (l < 16)
 			{
-				float dy[16];
-				for (int k = 0; k < 16; ++k)
-					dy[k] = 0.f;
-				const int r = tix * 16 + l;
-				if (r < NA)
-				{
-					int x0, x1;
-					active_xy(g, m, r, x0, x1);
-					const int x = x0 * g.L1 + x1;
-					const float *y = T.y() + l * 16;
-					gact[r] = FM::ncp_adjoint(y, FM::wrapf(phi[x] - FM::ncp_params(y).t), a[x], dy);
-				}
-				for (int k = 0; k < 16; ++k)
-					T.y()[l * 16 + k] = dy[k];
+				const int rq = (t0 + w) * 16 + (l >> 2); // its quad's row in the map
+				const bool live = rq < NA;
+				active_xy(g, m, min(rq, NA - 1), x0, x1);
+				const int xs = x0 * g.L1 + x1;
+				float *yr = y + (l >> 2) * FM::YS;
+				const FM::NCPq p = FM::ncpq_params(yr);
+				const float da = FM::ncpq_adjoint(p, yr, FM::wrapf(phi[xs] - p.t), a[xs], live);
+				if (live && (l & 3) == 0)
+					gact[rq] = da;
 			}
 			FM::wave_sync();
-			FM::mlp_backward<NI>(sh.lw, T, gr, dx, tix * 16, NA);
+			FM::mlp_rows_backward<NI>(sh.lw, sh.buf, x, row, h1, h2, gr, dx);
+			// the adjoints of the lane's loops' angles, then of ring plaquettes
+			// 2q and 2q + 1 (that of 2q - 1 goes to the quarter which holds it)
+			float e[5];
+#pragma unroll
+			for (int k = 0; k < 5; ++k)
+				e[k] = fmaf(x[2 * k], dx[(2 * k + 1) / 4][(2 * k + 1) & 3], -x[2 * k + 1] * dx[2 * k / 4][(2 * k) & 3]);
+			const float from_next = __shfl(e[3] + e[4], (l + 16) & 63, 64);
+			if (r < NA)
+				*reinterpret_cast<float2 *>(dr + r * 8 + 2 * ll.q) =
+				    make_float2(e[0] + e[2] + e[3] + e[4], e[1] + e[2] + e[4] + from_next);
 		}
 		__syncthreads();
-		FM::store_grad<NI>(gr, part + (long)layer * NP_LAYER);
+		FM::store_grad<NI>(gr, row, part + (long)layer * NP_LAYER);
 		// adjoints w.r.t. the layer's input: the active plaquettes from gact,
-		// the frozen ones gain their features' adjoints
+		// the frozen ones gain theirs as ring plaquettes of the active ones,
+		// which lie one step along x0, x1 or both (class bits that differ)
+		const int h = g.L1 >> 1;
 		for (int y = threadIdx.x; y < g.V - 1; y += THREADS)
 		{
-			if (class_of(g, y) == m)
+			const int y0 = y / g.L1, y1 = y - y0 * g.L1;
+			const int s0 = (y0 ^ m) & 1, s1 = (y1 ^ (m >> 1)) & 1;
+			if (!s0 && !s1)
 			{
-				a[y] = gact[active_index(g, y)];
+				a[y] = gact[(y0 >> 1) * h + (y1 >> 1)];
 				continue;
 			}
-			const int y0 = y / g.L1, y1 = y - y0 * g.L1;
-			const float2 cy = cs[y];
 			float acc = 0.f;
+#pragma unroll
 			for (int k = 0; k < 8; ++k)
 			{
 				int d0, d1;
 				ring(k, d0, d1);
+				if ((d0 != 0) != (s0 != 0) || (d1 != 0) != (s1 != 0))
+					continue;
 				const int x = sitew(g, y0 - d0, y1 - d1);
-				if (x == g.V - 1 || class_of(g, x) != m)
+				if (x == g.V - 1)
 					continue;
 				const int x0 = x / g.L1, x1 = x - x0 * g.L1;
-				const float *dr = dx + (long)active_index(g, x) * NI;
-				acc = fmaf(-cy.y, dr[2 * k], acc);
-				acc = fmaf(cy.x, dr[2 * k + 1], acc);
-				// the two 1x2 loops that contain ring position k
-				for (int j : {(k + 7) & 7, k})
-				{
-					const float2 ps = loop_cs(g, cs, x0, x1, 8 + j);
-					acc = fmaf(-ps.y, dr[16 + 2 * j], acc);
-					acc = fmaf(ps.x, dr[16 + 2 * j + 1], acc);
-				}
-				// the L-shaped loops (ring positions 2j - 1, 2j, 2j + 1) that
-				// contain ring position k: one for a corner, two for an edge
-				for (int j : {(k & 1) ? (k - 1) >> 1 : k >> 1, (k & 1) ? ((k + 1) >> 1) & 3 : -1})
-				{
-					if (j < 0)
-						continue;
-					const float2 ps = loop_cs(g, cs, x0, x1, 16 + j);
-					acc = fmaf(-ps.y, dr[32 + 2 * j], acc);
-					acc = fmaf(ps.x, dr[32 + 2 * j + 1], acc);
-				}
+				acc += dr[((x0 >> 1) * h + (x1 >> 1)) * 8 + k];
 			}
 			a[y] += acc;
 		}
 	}
-}
-
-// grad[i] = scale * sum_c partial[c][i] (fixed order)
-__global__ void k_pc_reduce(int n, const float *__restrict__ partial, int batch, float scale, float *__restrict__ grad)
-{
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	double s = 0.0;
-	for (int c = 0; c < batch; ++c)
-		s += partial[(long)c * n + i];
-	grad[i] = (float)(s * scale);
 }
 
 __global__ void k_pc_init(int n, float *p, uint64_t seed)
@@ -689,7 +608,7 @@ size_t mesh_pcflow_workspace_bytes(const mesh_grid *g, int batch, int layers)
 		return 0;
 	size_t n = (size_t)batch * layers * pg.V           // plaquettes per layer
 	           + (size_t)batch * pg.V                  // final plaquettes
-	           + (size_t)batch * (pg.V / 4) * NI       // feature adjoints
+	           + (size_t)batch * (pg.V / 4) * 8        // adjoints of the active plaquettes' rings
 	           + (size_t)batch * layers * NP_LAYER;    // per-configuration gradients
 	return n * sizeof(float);
 }
@@ -705,8 +624,8 @@ int mesh_pcflow_gradient(mesh_ctx *ctx, const mesh_grid *g, int batch, int layer
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_gradient");
 	float *pl = (float *)workspace;
 	float *pf = pl + (size_t)batch * layers * pg.V;
-	float *dxs = pf + (size_t)batch * pg.V;
-	float *part = dxs + (size_t)batch * (pg.V / 4) * NI;
+	float *drs = pf + (size_t)batch * pg.V;
+	float *part = drs + (size_t)batch * (pg.V / 4) * 8;
 	if (int rc = by_width(pg, [&](auto nt) {
 		    return launch_forward<decltype(nt)::value>(ctx, pg, batch, layers, params, seed, step, nullptr, pl, pf,
 		                                               out_dev);
@@ -715,10 +634,10 @@ int mesh_pcflow_gradient(mesh_ctx *ctx, const mesh_grid *g, int batch, int layer
 	const size_t lds_b = (4 * (size_t)pg.V + pg.V / 4) * sizeof(float);
 	if (int rc = set_lds(ctx, k_pc_backward, lds_b))
 		return rc;
-	k_pc_backward<<<batch, THREADS, lds_b, ctx->stream>>>(pg, layers, params, pl, pf, (float)beta, dxs, part);
+	k_pc_backward<<<batch, THREADS, lds_b, ctx->stream>>>(pg, layers, params, pl, pf, (float)beta, drs, part);
 	MESH_LAUNCHED(ctx);
 	const int n = layers * NP_LAYER;
-	k_pc_reduce<<<(n + 255) / 256, 256, 0, ctx->stream>>>(n, part, batch, 1.0f / batch, grad);
+	FM::k_grad_reduce<<<(n + 63) / 64, 256, 0, ctx->stream>>>(n, part, batch, 1.0f / batch, grad);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }

@@ -211,6 +211,29 @@ def test_pcflow_gradient_against_autograd(ctx):
         assert np.linalg.norm(g[sl] - gr[sl]) <= 2e-3 * np.linalg.norm(gr[sl]) + 1e-6, layer
 
 
+@pytest.mark.parametrize("L0,L1,B,nl", [(4, 4, 1, 4), (6, 10, 5, 4), (8, 32, 33, 2), (6, 44, 2, 4), (4, 66, 3, 3),
+                                        (64, 64, 2, 4)])
+def test_pcflow_gradient_tile_edges(ctx, L0, L1, B, nl):
+    """the backward pass takes four tiles of 16 active plaquettes a round:
+    rounds of one to four tiles, last tiles with 1 to 16 rows, the largest
+    volume; batches around the reduction's groups of configurations.  Bound:
+    that of the test above, per layer."""
+    torch = pytest.importorskip("torch")
+    beta, seed, step = 2.0, 31, 2
+    p = _params(32, 0.2, nl)
+    f = U1.PlaqCouplingFlow(L0, L1, ctx, layers=nl)
+    f.set_params(p)
+    f.gradient(B, beta, seed, step)
+    g = f.grad.download().astype(np.float64)
+    pt = torch.tensor(p.astype(np.float64), requires_grad=True)
+    z = torch.tensor(np.stack([U.pcflow_draws(seed, step, c, L0, L1)[0] for c in range(B)]).astype(np.float64))
+    U.pcflow_loss(pt, z, L0, L1, beta)[0].mean().backward()
+    gr = pt.grad.numpy()
+    for layer in range(nl):
+        sl = slice(layer * U.PC_NP_LAYER, (layer + 1) * U.PC_NP_LAYER)
+        assert np.linalg.norm(g[sl] - gr[sl]) <= 2e-3 * np.linalg.norm(gr[sl]) + 1e-6, layer
+
+
 def test_pcflow_deeper_stack(ctx):
     """a 12-layer stack: samples, inverse log q and gradient against the oracle"""
     torch = pytest.importorskip("torch")

@@ -267,6 +267,35 @@ def test_flow_gradient_against_autograd(ctx):
         assert np.linalg.norm(g[sl] - gr[sl]) <= 2e-3 * np.linalg.norm(gr[sl]) + 1e-6, layer
 
 
+@pytest.mark.parametrize("L0,L1,B", [(4, 4, 1), (12, 8, 5), (4, 68, 2), (64, 64, 2)])
+def test_flow_tile_edges(ctx, L0, L1, B):
+    """tiles of 16 active plaquettes, four a round in the backward pass: last
+    tiles with 4, 8 and 16 rows, the largest volume; forward, inverse and
+    gradient against the oracle (bounds of the tests above: log q sums one
+    FP32 log g' per active plaquette and layer)"""
+    torch = pytest.importorskip("torch")
+    seed, step, beta, nl, V = 61, 2, 2.0, 4, L0 * L1
+    p = _params(62, 0.2, nl)
+    f = U1.Flow(L0, L1, ctx, layers=nl)
+    f.set_params(p)
+    ens = U1.U1Ensemble(L0, L1, B, ctx)
+    out = f.sample(ens, seed, step).download().reshape(B, 2)
+    zn = np.stack([U.flow_z(seed, step, c, L0, L1) for c in range(B)]).astype(np.float64)
+    z = torch.tensor(zn)
+    pt = torch.tensor(p.astype(np.float64), requires_grad=True)
+    loss, th, ld, _ = U.flow_loss(pt, z, beta)
+    loss.backward()
+    assert _wrapdiff(ens.angles(), th.detach().numpy()).max() < 2e-3
+    np.testing.assert_allclose(out[:, 0], U.log_prior(L0, L1) - ld.detach().numpy(), atol=1e-2 * max(1.0, V / 64))
+    z_out = U1.Buffer(B * 2 * V, np.float32, ctx)
+    inv = f.logq(ens, z_out=z_out).download().reshape(B, 2)
+    assert _wrapdiff(z_out.download().reshape(zn.shape), zn).max() < 2e-3
+    np.testing.assert_allclose(inv[:, 0], out[:, 0], atol=3e-3 * max(1.0, V / 64))
+    f.gradient(B, beta, seed, step)
+    g, gr = f.grad.download().astype(np.float64), pt.grad.numpy()
+    assert np.linalg.norm(g - gr) / np.linalg.norm(gr) < 2e-3
+
+
 def test_flow_training_respects_free_energy_bound(ctx):
     """Adam on the reverse KL lowers E[log q + beta S] from its identity value
     and never below -log Z (the KL is non-negative)."""
