@@ -18,8 +18,13 @@
 
 #include "mesh_internal.h"
 #include "rng_dev.h"
+#include "trig_dev.h"
 
 namespace flow_mlp {
+
+using mesh_dev::atan2_1;
+using mesh_dev::div1;
+using mesh_dev::sincos1;
 
 constexpr int NK = 4;          // mixture components
 constexpr int NH = 64;         // hidden width
@@ -265,62 +270,6 @@ __device__ __forceinline__ void put_outputs(float *y, f4 v)
 {
 	const int l = threadIdx.x & 63;
 	*reinterpret_cast<f4 *>(y + (l & 15) * YS + (l >> 4) * 4) = v;
-}
-
-// ---- elementary functions of the quad maps below, for the ranges they meet.
-// The maps were held by these: the library's sincosf and atan2f carry the
-// reduction of huge arguments, infinities and zeros, about 90 and 60 VALU
-// instructions a call against 24 and 27 here.  Coefficients: minimax fits
-// (reweighted least squares) of (sin r - r) / r^3 and (cos r - 1 + r^2 / 2) /
-// r^4 over |r| <= pi / 4 and of (atan q - q) / q^3 over [0, 1]; largest errors
-// in FP32 0.66 ulp (sin), 1.22 ulp (cos), 0.88 ulp (atan).
-
-// n / d to within an ulp, for d and 1 / d in the normal range
-__device__ __forceinline__ float div1(float n, float d)
-{
-	const float r = __builtin_amdgcn_rcpf(d), q = n * r;
-	return fmaf(fmaf(-q, d, n), r, q);
-}
-
-constexpr float HALF_PI_HI = 1.57079637050628662109f, HALF_PI_LO = -4.37113900018624283e-8f;
-
-// sin and cos for |x| up to a few turns (NaN gives NaN)
-__device__ __forceinline__ void sincos1(float x, float &sn, float &cs)
-{
-	const float q = rintf(x * 0.63661977236758134f);
-	float r = fmaf(-q, HALF_PI_HI, x);
-	r = fmaf(-q, HALF_PI_LO, r);
-	const float r2 = r * r;
-	const float s = fmaf(r * r2, fmaf(fmaf(-0.00019516977772582322f, r2, 0.008332176133990288f), r2,
-	                                  -0.16666655242443085f), r);
-	const float c = fmaf(r2 * r2, fmaf(fmaf(2.443809171381872e-05f, r2, -0.0013887364184483886f), r2,
-	                                   0.04166664555668831f), fmaf(-0.5f, r2, 1.f));
-	const int i = (int)q;
-	const bool odd = i & 1;
-	sn = __int_as_float(__float_as_int(odd ? c : s) ^ ((i & 2) << 30));
-	cs = __int_as_float(__float_as_int(odd ? s : c) ^ (((i + 1) & 2) << 30));
-}
-
-// atan2(y, x) for finite arguments, the larger of them a normal number whose
-// reciprocal is one too
-__device__ __forceinline__ float atan2_1(float y, float x)
-{
-	const float ax = fabsf(x), ay = fabsf(y);
-	const float q = div1(fminf(ax, ay), fmaxf(ax, ay)), q2 = q * q;
-	float p = fmaf(-0.0018272141460329294f, q2, 0.011064446531236172f);
-	p = fmaf(p, q2, -0.031455714255571365f);
-	p = fmaf(p, q2, 0.0582345649600029f);
-	p = fmaf(p, q2, -0.0841946005821228f);
-	p = fmaf(p, q2, 0.10957576334476471f);
-	p = fmaf(p, q2, -0.1426524519920349f);
-	p = fmaf(p, q2, 0.19998638331890106f);
-	p = fmaf(p, q2, -0.33333301544189453f);
-	const float a = fmaf(q * q2, p, q);
-	// pi/2 -+ a where |y| > |x|, pi - a for x < 0 below that
-	const bool steep = ay > ax, neg = x < 0.f;
-	const float k = steep ? HALF_PI_HI : (neg ? 2.f * HALF_PI_HI : 0.f);
-	const float t = fmaf(k, HALF_PI_LO / HALF_PI_HI, steep != neg ? -a : a);
-	return copysignf(k + t, y);
 }
 
 // ---- the mixture on a quad of lanes: lane k (= lane % 4) of a quad holds

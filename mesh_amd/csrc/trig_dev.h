@@ -1,0 +1,105 @@
+// Sine, cosine, arctangent and quotient for the ranges that the U(1) kernels
+// meet: angles of a few turns at most and finite, non-zero quotients.
+//
+// These kernels are held by vector instructions, and the library's functions
+// carry the reduction of huge arguments, infinities and zeros: sincosf and
+// atan2f are about 90 and 60 instructions a call against 24 and 27 here, the
+// double cosine about 100 against 35.  Coefficients: minimax fits (reweighted
+// least squares) of (sin r - r) / r^3 and (cos r - 1 + r^2 / 2) / r^4 over
+// |r| <= pi / 4 and of (atan q - q) / q^3 over [0, 1]; largest errors in FP32
+// 0.66 ulp (sin), 1.22 ulp (cos), 0.88 ulp (atan).  FP64: Taylor series to
+// below half an ulp.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace mesh_dev {
+
+#define TD __device__ __forceinline__
+
+// n / d to within an ulp, for d and 1 / d in the normal range
+TD float div1(float n, float d)
+{
+	const float r = __builtin_amdgcn_rcpf(d), q = n * r;
+	return fmaf(fmaf(-q, d, n), r, q);
+}
+
+constexpr float HALF_PI_HI = 1.57079637050628662109f, HALF_PI_LO = -4.37113900018624283e-8f;
+
+TD float sin_quarter(float r, float r2)
+{
+	return fmaf(r * r2,
+	            fmaf(fmaf(-0.00019516977772582322f, r2, 0.008332176133990288f), r2, -0.16666655242443085f), r);
+}
+TD float cos_quarter(float r2)
+{
+	return fmaf(r2 * r2, fmaf(fmaf(2.443809171381872e-05f, r2, -0.0013887364184483886f), r2, 0.04166664555668831f),
+	            fmaf(-0.5f, r2, 1.f));
+}
+// r = x - i pi / 2, |r| <= pi / 4 (the first step is exact for a few turns)
+TD float quarter(float x, int &i)
+{
+	const float q = rintf(x * 0.63661977236758134f);
+	i = (int)q;
+	return fmaf(-q, HALF_PI_LO, fmaf(-q, HALF_PI_HI, x));
+}
+
+// sin and cos for |x| up to a few turns (NaN gives NaN)
+TD void sincos1(float x, float &sn, float &cs)
+{
+	int i;
+	const float r = quarter(x, i), r2 = r * r, s = sin_quarter(r, r2), c = cos_quarter(r2);
+	const bool odd = i & 1;
+	sn = __int_as_float(__float_as_int(odd ? c : s) ^ ((i & 2) << 30));
+	cs = __int_as_float(__float_as_int(odd ? s : c) ^ (((i + 1) & 2) << 30));
+}
+// atan2(y, x) for finite arguments, the larger of them a normal number whose
+// reciprocal is one too
+TD float atan2_1(float y, float x)
+{
+	const float ax = fabsf(x), ay = fabsf(y);
+	const float q = div1(fminf(ax, ay), fmaxf(ax, ay)), q2 = q * q;
+	float p = fmaf(-0.0018272141460329294f, q2, 0.011064446531236172f);
+	p = fmaf(p, q2, -0.031455714255571365f);
+	p = fmaf(p, q2, 0.0582345649600029f);
+	p = fmaf(p, q2, -0.0841946005821228f);
+	p = fmaf(p, q2, 0.10957576334476471f);
+	p = fmaf(p, q2, -0.1426524519920349f);
+	p = fmaf(p, q2, 0.19998638331890106f);
+	p = fmaf(p, q2, -0.33333301544189453f);
+	const float a = fmaf(q * q2, p, q);
+	// pi/2 -+ a where |y| > |x|, pi - a for x < 0 below that
+	const bool steep = ay > ax, neg = x < 0.f;
+	const float k = steep ? HALF_PI_HI : (neg ? 2.f * HALF_PI_HI : 0.f);
+	const float t = fmaf(k, HALF_PI_LO / HALF_PI_HI, steep != neg ? -a : a);
+	return copysignf(k + t, y);
+}
+
+// cos for |x| up to a few turns, FP64
+TD double cos1(double x)
+{
+	const double q = rint(x * 0.63661977236758134308);
+	const double r = fma(-q, 6.123233995736766036e-17, fma(-q, 1.57079632679489655800, x)), r2 = r * r;
+	double ps = -1.0 / 1307674368000.0;
+	ps = fma(ps, r2, 1.0 / 6227020800.0);
+	ps = fma(ps, r2, -1.0 / 39916800.0);
+	ps = fma(ps, r2, 1.0 / 362880.0);
+	ps = fma(ps, r2, -1.0 / 5040.0);
+	ps = fma(ps, r2, 1.0 / 120.0);
+	ps = fma(ps, r2, -1.0 / 6.0);
+	const double s = fma(r * r2, ps, r);
+	double pc = 1.0 / 20922789888000.0;
+	pc = fma(pc, r2, -1.0 / 87178291200.0);
+	pc = fma(pc, r2, 1.0 / 479001600.0);
+	pc = fma(pc, r2, -1.0 / 3628800.0);
+	pc = fma(pc, r2, 1.0 / 40320.0);
+	pc = fma(pc, r2, -1.0 / 720.0);
+	pc = fma(pc, r2, 1.0 / 24.0);
+	const double c = fma(r2 * r2, pc, fma(-0.5, r2, 1.0));
+	const int i = (int)q;
+	const double v = i & 1 ? s : c;
+	return (i + 1) & 2 ? -v : v;
+}
+
+#undef TD
+
+} // namespace mesh_dev

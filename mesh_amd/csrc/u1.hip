@@ -10,11 +10,14 @@
 // theta_P(x) = theta_0(x) + theta_1(x+0) - theta_0(x+1) - theta_1(x);
 // S = beta sum_x (1 - cos theta_P(x)); Q = round(sum_x wrap(theta_P(x)) / 2 pi).
 //
-// Design: a configuration (2 V floats, 8 KB at 32^2) lives in LDS for the
-// whole trajectory; one workgroup of 256 threads owns one configuration, so a
-// trajectory is one launch over the batch with no HBM traffic between steps.
+// Design: a trajectory of a lattice up to 4096 sites is one launch over the
+// batch with no HBM traffic between steps.  One workgroup owns one
+// configuration; a thread keeps its sites' angles and momenta in registers and
+// LDS carries what neighbours read (angles, then sin theta_P).
 #include "mesh_internal.h"
 #include "rng_dev.h"
+#include "trig_dev.h"
+#include <utility>
 
 using namespace mesh_dev;
 
@@ -149,77 +152,131 @@ __global__ __launch_bounds__(U1_THREADS) void k_u1_obs(U1Geo g, const float *__r
 	}
 }
 
-// One HMC trajectory per configuration, entirely in LDS.
-// out[c*4 + {0,1,2,3}] = {Delta H, accepted, u, S_new/beta}
-__global__ __launch_bounds__(U1_THREADS) void k_u1_hmc(U1Geo g, float *th, const double *__restrict__ deltas, int nd,
-                                                      double beta, uint64_t seed, uint32_t traj, int metropolis,
-                                                      double *out)
+// block sum of NQ doubles over the workgroup's wavefronts (at most 16), in a
+// fixed order; result valid in thread 0
+template <int NQ> __device__ __forceinline__ void bsum_wide(double (&v)[NQ], double (*red)[16])
 {
-	extern __shared__ float lds[];
-	float *t = lds;               // angles, 2V
-	float *q = lds + 2 * g.V;     // momenta, 2V
-	float *sp = lds + 4 * g.V;    // sin theta_P, V
-	__shared__ double red[4][4];
-	__shared__ int acc_s;
-	int c = blockIdx.x;
-	float *tg = th + (long)c * 2 * g.V;
-	const float hb = (float)(0.5 * beta);
-	double eold = 0.0;
-	for (int i = threadIdx.x; i < 2 * g.V; i += U1_THREADS)
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+	for (int q = 0; q < NQ; ++q)
 	{
-		t[i] = tg[i];
-		int mu = i >= g.V, x = i - mu * g.V;
-		float qq = (float)(u1_normal(seed, TAG_U1MOM, traj, c, mu, x) * 0.70710678118654752440);
-		q[i] = qq;
+		double s = v[q];
+#pragma unroll
+		for (int o = 32; o >= 1; o >>= 1)
+			s += __shfl_xor(s, o, 64);
+		if (lane == 0)
+			red[q][w] = s;
 	}
 	__syncthreads();
-	// per-site energy before: beta (1 - cos theta_P(x)) + q_0(x)^2 + q_1(x)^2
-	for (int x = threadIdx.x; x < g.V; x += U1_THREADS)
+	if (threadIdx.x == 0)
+#pragma unroll
+		for (int q = 0; q < NQ; ++q)
+		{
+			v[q] = red[q][0];
+			for (int i = 1; i < nw; ++i)
+				v[q] += red[q][i];
+		}
+}
+
+// One HMC trajectory per configuration in one workgroup: thread i owns the
+// sites i, i + blockDim, ... (SPT of them), their angles and momenta in
+// registers.  A step writes the angles to LDS, reads the two that a plaquette
+// takes from its neighbours, writes sin theta_P and reads it at the two
+// backward neighbours: two barriers.  The chain of barriers, LDS reads and one
+// sine bounds it, so a lattice takes as many threads as it has sites, up to
+// 1024 (256 chains of 32^2, 20 steps: 24 us; 256 threads with angles and
+// momenta in LDS and three barriers a step took 63 us).
+// out[c*4 + {0,1,2,3}] = {Delta H, accepted, u, S_new/beta}
+template <int SPT>
+__global__ __launch_bounds__(1024) void k_u1_hmc(U1Geo g, float *th, const double *__restrict__ deltas, int nd,
+                                                 double beta, uint64_t seed, uint32_t traj, int metropolis, double *out)
+{
+	extern __shared__ float lds[];
+	float *T0 = lds, *T1 = lds + g.V, *SP = lds + 2 * g.V;
+	__shared__ double red[3][16];
+	__shared__ int acc_s;
+	const int c = blockIdx.x;
+	float *tg = th + (long)c * 2 * g.V;
+	const float hb = (float)(0.5 * beta);
+	float t0[SPT], t1[SPT], q0[SPT], q1[SPT], sp[SPT];
+	int f0[SPT], f1[SPT], b0[SPT], b1[SPT]; // neighbours
+#pragma unroll
+	for (int k = 0; k < SPT; ++k)
 	{
-		double k = (double)q[x] * q[x] + (double)q[g.V + x] * q[g.V + x];
-		eold += beta * (1.0 - cos((double)plaq(g, t, x))) + k;
+		const int x = threadIdx.x + k * blockDim.x;
+		if (x >= g.V)
+			break;
+		f0[k] = xp0(g, x), f1[k] = xp1(g, x), b0[k] = xm0(g, x), b1[k] = xm1(g, x);
+		T0[x] = t0[k] = tg[x];
+		T1[x] = t1[k] = tg[g.V + x];
+		q0[k] = (float)(u1_normal(seed, TAG_U1MOM, traj, c, 0, x) * 0.70710678118654752440);
+		q1[k] = (float)(u1_normal(seed, TAG_U1MOM, traj, c, 1, x) * 0.70710678118654752440);
+	}
+	// plaquette angle at a thread's k-th site, in plaq()'s order
+	auto angle = [&](int k) { return t0[k] + T1[f0[k]] - T0[f1[k]] - t1[k]; };
+	__syncthreads();
+	// per-site energy before: beta (1 - cos theta_P(x)) + q_0(x)^2 + q_1(x)^2
+	double v[3] = {0.0, 0.0, 0.0}; // H_new, S_new / beta, H_old
+#pragma unroll
+	for (int k = 0; k < SPT; ++k)
+	{
+		if ((int)(threadIdx.x + k * blockDim.x) >= g.V)
+			break;
+		const double kin = (double)q0[k] * q0[k] + (double)q1[k] * q1[k];
+		v[2] += beta * (1.0 - cos1((double)angle(k))) + kin;
 	}
 	// every wave has read the start angles before the first link step moves them
 	__syncthreads();
-	for (int s = 0; s < nd; ++s)
+	for (int s = 0; s < nd; s += 2)
 	{
 		const float d = (float)deltas[s];
-		if (s % 2 == 0)
+#pragma unroll
+		for (int k = 0; k < SPT; ++k)
 		{
-			for (int i = threadIdx.x; i < 2 * g.V; i += U1_THREADS)
-				t[i] = wrap_pi(fmaf(d, q[i], t[i]));
-		}
-		else
-		{
-			for (int x = threadIdx.x; x < g.V; x += U1_THREADS)
-				sp[x] = sinf(plaq(g, t, x));
-			__syncthreads();
-			const float dh = d * hb;
-			for (int x = threadIdx.x; x < g.V; x += U1_THREADS)
-			{
-				float s0 = sp[x] - sp[xm1(g, x)];
-				float s1 = sp[xm0(g, x)] - sp[x];
-				q[x] = fmaf(-dh, s0, q[x]);
-				q[g.V + x] = fmaf(-dh, s1, q[g.V + x]);
-			}
+			const int x = threadIdx.x + k * blockDim.x;
+			if (x >= g.V)
+				break;
+			T0[x] = t0[k] = wrap_pi(fmaf(d, q0[k], t0[k]));
+			T1[x] = t1[k] = wrap_pi(fmaf(d, q1[k], t1[k]));
 		}
 		__syncthreads();
+		if (s + 1 >= nd)
+			break;
+		const float dh = (float)deltas[s + 1] * hb;
+#pragma unroll
+		for (int k = 0; k < SPT; ++k)
+		{
+			const int x = threadIdx.x + k * blockDim.x;
+			if (x >= g.V)
+				break;
+			SP[x] = sp[k] = sinf(angle(k));
+		}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < SPT; ++k)
+		{
+			if ((int)(threadIdx.x + k * blockDim.x) >= g.V)
+				break;
+			const float s0 = sp[k] - SP[b1[k]];
+			const float s1 = SP[b0[k]] - sp[k];
+			q0[k] = fmaf(-dh, s0, q0[k]);
+			q1[k] = fmaf(-dh, s1, q1[k]);
+		}
 	}
-	double v[2] = {0.0, 0.0};
-	for (int x = threadIdx.x; x < g.V; x += U1_THREADS)
+#pragma unroll
+	for (int k = 0; k < SPT; ++k)
 	{
-		double k = (double)q[x] * q[x] + (double)q[g.V + x] * q[g.V + x];
-		double sn = 1.0 - cos((double)plaq(g, t, x));
-		v[0] += beta * sn + k;
+		if ((int)(threadIdx.x + k * blockDim.x) >= g.V)
+			break;
+		const double kin = (double)q0[k] * q0[k] + (double)q1[k] * q1[k];
+		const double sn = 1.0 - cos1((double)angle(k));
+		v[0] += beta * sn + kin;
 		v[1] += sn;
 	}
-	double dd[2] = {v[0], v[1]};
-	double eo[1] = {eold};
-	bsum<2>(dd, red);
-	bsum<1>(eo, red);
+	bsum_wide<3>(v, red);
 	if (threadIdx.x == 0)
 	{
-		double dH = dd[0] - eo[0];
+		const double dH = v[0] - v[2];
 		u4 ctr = {traj, (uint32_t)c, 0u, TAG_U1METRO};
 		u4 r = philox4x32_10(ctr, (uint32_t)seed, (uint32_t)(seed >> 32));
 		double u = u01_from_bits(r.x, r.y);
@@ -228,12 +285,19 @@ __global__ __launch_bounds__(U1_THREADS) void k_u1_hmc(U1Geo g, float *th, const
 		out[4 * c + 0] = dH;
 		out[4 * c + 1] = a;
 		out[4 * c + 2] = u;
-		out[4 * c + 3] = dd[1];
+		out[4 * c + 3] = v[1];
 	}
 	__syncthreads();
 	if (acc_s)
-		for (int i = threadIdx.x; i < 2 * g.V; i += U1_THREADS)
-			tg[i] = t[i];
+#pragma unroll
+		for (int k = 0; k < SPT; ++k)
+		{
+			const int x = threadIdx.x + k * blockDim.x;
+			if (x >= g.V)
+				break;
+			tg[x] = t0[k];
+			tg[g.V + x] = t1[k];
+		}
 }
 
 // ---- any dimension 2 <= nd <= 4, one thread per (configuration, site) -------
@@ -248,7 +312,7 @@ __global__ __launch_bounds__(U1_THREADS) void k_u1_hmc(U1Geo g, float *th, const
 
 struct U1NGeo
 {
-	int nd, V, np;   // dimensions, sites, planes nd (nd - 1) / 2
+	int nd, V;       // dimensions, sites
 	int L[4], st[4]; // extents, row-major strides (dimension 0 slowest)
 };
 
@@ -261,11 +325,6 @@ __device__ __forceinline__ int n_bwd(U1NGeo const &g, int x, int mu)
 {
 	int c = (x / g.st[mu]) % g.L[mu];
 	return c == 0 ? x + (g.L[mu] - 1) * g.st[mu] : x - g.st[mu];
-}
-// plane index of (mu, nu), mu < nu, in the order (0,1), (0,2), ..., (nd-2, nd-1)
-__device__ __forceinline__ int plane_of(U1NGeo const &g, int mu, int nu)
-{
-	return mu * (2 * g.nd - mu - 1) / 2 + (nu - mu - 1);
 }
 // plaquette angle of plane (mu, nu) at x of one configuration t[nd V] (unwrapped)
 __device__ __forceinline__ float plaq_n(U1NGeo const &g, const float *t, int mu, int nu, int x)
@@ -286,95 +345,121 @@ __global__ __launch_bounds__(256) void k_u1n_random(U1NGeo g, long n, float *th,
 	th[i] = (float)(6.283185307179586477 * u - 3.141592653589793238);
 }
 
-// momenta, a copy of the start configuration, per-site energy before
+// neighbours of site x: f[mu] = x + mu, b[mu] = x - mu
+template <int ND> struct Nb
+{
+	int f[ND], b[ND];
+	__device__ __forceinline__ Nb(U1NGeo const &g, int x)
+	{
+		int r = x;
+#pragma unroll
+		for (int mu = ND - 1; mu >= 0; --mu)
+		{
+			const int rest = mu ? (int)((unsigned)r / (unsigned)g.L[mu]) : 0, c = r - rest * g.L[mu], st = g.st[mu];
+			r = rest;
+			f[mu] = c + 1 == g.L[mu] ? x - c * st : x + st;
+			b[mu] = c == 0 ? x + (g.L[mu] - 1) * st : x - st;
+		}
+	}
+};
+
+// momenta, per-site energy before, and the first link step: work = wrap(theta + d q)
+template <int ND>
 __global__ __launch_bounds__(256) void k_u1n_start(U1NGeo g, int batch, const float *__restrict__ th,
-                                                   float *__restrict__ th_old, float *__restrict__ q,
+                                                   float *__restrict__ work, float *__restrict__ q,
                                                    double *__restrict__ e_old, double beta, uint64_t seed,
-                                                   uint32_t traj)
+                                                   uint32_t traj, float d)
 {
 	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (long)batch * g.V)
 		return;
-	int c = (int)(i / g.V), x = (int)(i - (long)c * g.V);
-	const long o = (long)c * g.nd * g.V;
+	const int c = (int)((unsigned)i / (unsigned)g.V), x = (int)(i - (long)c * g.V);
+	const long o = (long)c * ND * g.V;
 	const float *t = th + o;
+	const Nb<ND> nb(g, x);
+	float tx[ND];
+#pragma unroll
+	for (int mu = 0; mu < ND; ++mu)
+		tx[mu] = t[mu * g.V + x];
 	double e = 0.0;
-	for (int mu = 0; mu < g.nd; ++mu)
-		for (int nu = mu + 1; nu < g.nd; ++nu)
-			e += beta * (1.0 - cos((double)plaq_n(g, t, mu, nu, x)));
-	for (int mu = 0; mu < g.nd; ++mu)
+#pragma unroll
+	for (int mu = 0; mu < ND; ++mu)
+#pragma unroll
+		for (int nu = mu + 1; nu < ND; ++nu)
+		{
+			const float p = tx[mu] + t[nu * g.V + nb.f[mu]] - t[mu * g.V + nb.f[nu]] - tx[nu];
+			e += beta * (1.0 - cos1((double)p));
+		}
+#pragma unroll
+	for (int mu = 0; mu < ND; ++mu)
 	{
-		float qq = (float)(u1_normal(seed, TAG_U1MOM, traj, c, mu, x) * 0.70710678118654752440);
+		const float qq = (float)(u1_normal(seed, TAG_U1MOM, traj, c, mu, x) * 0.70710678118654752440);
 		q[o + mu * g.V + x] = qq;
 		e += (double)qq * qq;
-		th_old[o + mu * g.V + x] = t[mu * g.V + x];
+		work[o + mu * g.V + x] = wrap_pi(fmaf(d, qq, tx[mu]));
 	}
 	e_old[i] = e;
 }
 
-__global__ __launch_bounds__(256) void k_u1n_link(long n, float *__restrict__ th, const float *__restrict__ q, float d)
-{
-	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n)
-		th[i] = wrap_pi(fmaf(d, q[i], th[i]));
-}
-
-// sin theta_P of every plane at every site
-__global__ __launch_bounds__(256) void k_u1n_sinp(U1NGeo g, int batch, const float *__restrict__ th,
-                                                  float *__restrict__ sp)
-{
-	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= (long)batch * g.V)
-		return;
-	int c = (int)(i / g.V), x = (int)(i - (long)c * g.V);
-	const float *t = th + (long)c * g.nd * g.V;
-	float *s = sp + (long)c * g.np * g.V;
-	for (int mu = 0; mu < g.nd; ++mu)
-		for (int nu = mu + 1; nu < g.nd; ++nu)
-			s[plane_of(g, mu, nu) * g.V + x] = sinf(plaq_n(g, t, mu, nu, x));
-}
-
-__global__ __launch_bounds__(256) void k_u1n_mom(U1NGeo g, int batch, const float *__restrict__ sp,
-                                                 float *__restrict__ q, float dh)
+// A momentum step and the link step after it, in -> out: thread x forms its 3
+// nd (nd - 1) / 2 plaquette sines (its own and those of the backward
+// neighbours' planes that its links bound) from the angles.  The sines bound
+// it; forming each three times is still cheaper than sharing them through
+// memory, which took three launches a step (sines, momenta, links): 12.7 us
+// instead of 25 for four chains of 16^4.
+template <int ND>
+__global__ __launch_bounds__(256) void k_u1n_step(U1NGeo g, int batch, const float *__restrict__ in,
+                                                  float *__restrict__ out, float *__restrict__ q, float dh, float d)
 {
 	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (long)batch * g.V)
 		return;
-	int c = (int)(i / g.V), x = (int)(i - (long)c * g.V);
-	const float *s = sp + (long)c * g.np * g.V;
-	float *qc = q + (long)c * g.nd * g.V;
-	for (int mu = 0; mu < g.nd; ++mu)
-	{
-		float f = 0.0f;
-		bool first = true;
-		for (int nu = 0; nu < g.nd; ++nu)
+	const int c = (int)((unsigned)i / (unsigned)g.V), x = (int)(i - (long)c * g.V);
+	const long o = (long)c * ND * g.V;
+	const float *t = in + o;
+	const Nb<ND> nb(g, x);
+	float tx[ND];
+#pragma unroll
+	for (int mu = 0; mu < ND; ++mu)
+		tx[mu] = t[mu * g.V + x];
+	// s[mu][nu], mu < nu: sin theta_{mu nu}(x); sb[mu][nu]: that of the plane at x - nu
+	float s[ND][ND], sb[ND][ND];
+#pragma unroll
+	for (int mu = 0; mu < ND; ++mu)
+#pragma unroll
+		for (int nu = 0; nu < ND; ++nu)
 		{
 			if (nu == mu)
 				continue;
-			const int xb = n_bwd(g, x, nu);
-			float a, b;
 			if (mu < nu)
-			{
-				const float *sv = s + plane_of(g, mu, nu) * g.V;
-				a = sv[x];
-				b = sv[xb];
-			}
-			else
-			{
-				const float *sv = s + plane_of(g, nu, mu) * g.V;
-				a = -sv[x];
-				b = -sv[xb];
-			}
-			const float term = a - b;
-			f = first ? term : f + term;
-			first = false;
+				s[mu][nu] = sinf(tx[mu] + t[nu * g.V + nb.f[mu]] - t[mu * g.V + nb.f[nu]] - tx[nu]);
+			// the plane's corner y = x - nu; y + mu keeps the step x -> x + mu
+			const int y = nb.b[nu], ym = y + (nb.f[mu] - x);
+			const float mu_y = t[mu * g.V + y], nu_y = t[nu * g.V + y], nu_ym = t[nu * g.V + ym];
+			sb[mu][nu] = mu < nu ? sinf(mu_y + nu_ym - tx[mu] - nu_y) : sinf(nu_y + tx[mu] - nu_ym - mu_y);
 		}
-		qc[mu * g.V + x] = fmaf(-dh, f, qc[mu * g.V + x]);
+#pragma unroll
+	for (int mu = 0; mu < ND; ++mu)
+	{
+		float f = 0.0f;
+#pragma unroll
+		for (int nu = 0; nu < ND; ++nu)
+		{
+			if (nu == mu)
+				continue;
+			const float term = mu < nu ? s[mu][nu] - sb[mu][nu] : -s[nu][mu] - (-sb[mu][nu]);
+			f = nu == (mu == 0 ? 1 : 0) ? term : f + term;
+		}
+		const long j = o + mu * g.V + x;
+		const float qq = fmaf(-dh, f, q[j]);
+		q[j] = qq;
+		out[j] = wrap_pi(fmaf(d, qq, tx[mu]));
 	}
 }
 
 // block partial sums per configuration of (e_new - e_old, S_new / beta);
 // grid = batch * nbk blocks
+template <int ND>
 __global__ __launch_bounds__(256) void k_u1n_energy(U1NGeo g, int nbk, const float *__restrict__ th,
                                                     const float *__restrict__ q, const double *__restrict__ e_old,
                                                     double beta, double *__restrict__ partials)
@@ -385,13 +470,21 @@ __global__ __launch_bounds__(256) void k_u1n_energy(U1NGeo g, int nbk, const flo
 	double v[2] = {0.0, 0.0};
 	if (x < g.V)
 	{
-		const long o = (long)c * g.nd * g.V;
+		const long o = (long)c * ND * g.V;
 		const float *t = th + o;
+		const Nb<ND> nb(g, x);
 		double sn = 0.0, k = 0.0;
-		for (int mu = 0; mu < g.nd; ++mu)
-			for (int nu = mu + 1; nu < g.nd; ++nu)
-				sn += 1.0 - cos((double)plaq_n(g, t, mu, nu, x));
-		for (int mu = 0; mu < g.nd; ++mu)
+#pragma unroll
+		for (int mu = 0; mu < ND; ++mu)
+#pragma unroll
+			for (int nu = mu + 1; nu < ND; ++nu)
+			{
+				const float p =
+				    t[mu * g.V + x] + t[nu * g.V + nb.f[mu]] - t[mu * g.V + nb.f[nu]] - t[nu * g.V + x];
+				sn += 1.0 - cos1((double)p);
+			}
+#pragma unroll
+		for (int mu = 0; mu < ND; ++mu)
 		{
 			double qq = q[o + mu * g.V + x];
 			k += qq * qq;
@@ -407,38 +500,40 @@ __global__ __launch_bounds__(256) void k_u1n_energy(U1NGeo g, int nbk, const flo
 	}
 }
 
-// per configuration: Delta H, Metropolis (the uniform of the LDS kernel)
-__global__ __launch_bounds__(256) void k_u1n_accept(int batch, int nbk, const double *__restrict__ partials,
-                                                    uint64_t seed, uint32_t traj, int metropolis, double *out)
+// a workgroup per configuration: Delta H, Metropolis (the uniform of the LDS kernel)
+__global__ __launch_bounds__(256) void k_u1n_accept(int nbk, const double *__restrict__ partials, uint64_t seed,
+                                                    uint32_t traj, int metropolis, double *out)
 {
-	int c = blockIdx.x * blockDim.x + threadIdx.x;
-	if (c >= batch)
-		return;
-	double dH = 0.0, sn = 0.0;
-	for (int b = 0; b < nbk; ++b)
+	__shared__ double red[4][4];
+	const int c = blockIdx.x;
+	double v[2] = {0.0, 0.0};
+	for (int b = threadIdx.x; b < nbk; b += 256)
 	{
-		dH += partials[2 * ((long)c * nbk + b) + 0];
-		sn += partials[2 * ((long)c * nbk + b) + 1];
+		v[0] += partials[2 * ((long)c * nbk + b) + 0];
+		v[1] += partials[2 * ((long)c * nbk + b) + 1];
 	}
+	bsum<2>(v, red);
+	if (threadIdx.x)
+		return;
 	u4 ctr = {traj, (uint32_t)c, 0u, TAG_U1METRO};
 	u4 r = philox4x32_10(ctr, (uint32_t)seed, (uint32_t)(seed >> 32));
 	double u = u01_from_bits(r.x, r.y);
-	int a = metropolis ? (u < exp(-dH)) : 1;
-	out[4 * c + 0] = dH;
+	int a = metropolis ? (u < exp(-v[0])) : 1;
+	out[4 * c + 0] = v[0];
 	out[4 * c + 1] = a;
 	out[4 * c + 2] = u;
-	out[4 * c + 3] = sn;
+	out[4 * c + 3] = v[1];
 }
 
-// rejected configurations get their start angles back
-__global__ __launch_bounds__(256) void k_u1n_restore(long n, long per, float *__restrict__ th,
-                                                     const float *__restrict__ th_old, const double *__restrict__ out)
+// accepted configurations take the trajectory's angles
+__global__ __launch_bounds__(256) void k_u1n_commit(long n, long per, float *__restrict__ th,
+                                                    const float *__restrict__ work, const double *__restrict__ out)
 {
 	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n)
 		return;
-	if (out[4 * (i / per) + 1] == 0.0)
-		th[i] = th_old[i];
+	if (out[4 * (i / per) + 1] != 0.0)
+		th[i] = work[i];
 }
 
 // block partial sums per configuration of (sum (1 - cos), sum cos, sum wrap theta_P)
@@ -500,7 +595,6 @@ int u1n_setup(mesh_ctx *ctx, const mesh_grid *g, int batch, U1NGeo *ug)
 		return mesh_fail(ctx, MESH_E_SIZE, "U(1) batch x links exceeds 2^31");
 	ug->nd = g->nd;
 	ug->V = (int)V;
-	ug->np = g->nd * (g->nd - 1) / 2;
 	int s = 1;
 	for (int i = g->nd - 1; i >= 0; --i)
 	{
@@ -540,35 +634,33 @@ int u1n_workspace(mesh_ctx *ctx, size_t bytes)
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// The caller's field keeps the start angles until the decision; the link steps
+// alternate between two fields of the workspace.
+template <int ND>
 int u1n_hmc(mesh_ctx *ctx, U1NGeo const &ug, int batch, float *theta, const double *deltas, int ndeltas, double beta,
             uint64_t seed, uint32_t traj, int metropolis, double *out)
 {
-	const long nl = (long)batch * ug.nd * ug.V, ns = (long)batch * ug.V;
+	const long nl = (long)batch * ND * ug.V, ns = (long)batch * ug.V;
 	const int nbk = (ug.V + 255) / 256;
-	const size_t b_q = align256(nl * sizeof(float)), b_sp = align256((size_t)batch * ug.np * ug.V * sizeof(float)),
-	             b_e = align256(ns * sizeof(double)), b_p = align256((size_t)batch * nbk * 2 * sizeof(double));
-	if (int rc = u1n_workspace(ctx, 2 * b_q + b_sp + b_e + b_p))
+	const size_t b_q = align256(nl * sizeof(float)), b_e = align256(ns * sizeof(double)),
+	             b_p = align256((size_t)batch * nbk * 2 * sizeof(double));
+	if (int rc = u1n_workspace(ctx, 3 * b_q + b_e + b_p))
 		return rc;
 	char *w = (char *)ctx->u1_ws;
-	float *q = (float *)w, *th_old = (float *)(w + b_q), *sp = (float *)(w + 2 * b_q);
-	double *e_old = (double *)(w + 2 * b_q + b_sp), *partials = (double *)(w + 2 * b_q + b_sp + b_e);
+	float *q = (float *)w, *cur = (float *)(w + b_q), *next = (float *)(w + 2 * b_q);
+	double *e_old = (double *)(w + 3 * b_q), *partials = (double *)(w + 3 * b_q + b_e);
 	const int gl = (int)((nl + 255) / 256), gs = (int)((ns + 255) / 256);
-	k_u1n_start<<<gs, 256, 0, ctx->stream>>>(ug, batch, theta, th_old, q, e_old, beta, seed, traj);
 	const float hb = (float)(0.5 * beta);
-	for (int s = 0; s < ndeltas; ++s)
+	k_u1n_start<ND><<<gs, 256, 0, ctx->stream>>>(ug, batch, theta, cur, q, e_old, beta, seed, traj, (float)deltas[0]);
+	for (int s = 1; s < ndeltas; s += 2)
 	{
-		const float d = (float)deltas[s];
-		if (s % 2 == 0)
-			k_u1n_link<<<gl, 256, 0, ctx->stream>>>(nl, theta, q, d);
-		else
-		{
-			k_u1n_sinp<<<gs, 256, 0, ctx->stream>>>(ug, batch, theta, sp);
-			k_u1n_mom<<<gs, 256, 0, ctx->stream>>>(ug, batch, sp, q, d * hb);
-		}
+		k_u1n_step<ND><<<gs, 256, 0, ctx->stream>>>(ug, batch, cur, next, q, (float)deltas[s] * hb,
+		                                            (float)deltas[s + 1]);
+		std::swap(cur, next);
 	}
-	k_u1n_energy<<<batch * nbk, 256, 0, ctx->stream>>>(ug, nbk, theta, q, e_old, beta, partials);
-	k_u1n_accept<<<(batch + 255) / 256, 256, 0, ctx->stream>>>(batch, nbk, partials, seed, traj, metropolis, out);
-	k_u1n_restore<<<gl, 256, 0, ctx->stream>>>(nl, (long)ug.nd * ug.V, theta, th_old, out);
+	k_u1n_energy<ND><<<batch * nbk, 256, 0, ctx->stream>>>(ug, nbk, cur, q, e_old, beta, partials);
+	k_u1n_accept<<<batch, 256, 0, ctx->stream>>>(nbk, partials, seed, traj, metropolis, out);
+	k_u1n_commit<<<gl, 256, 0, ctx->stream>>>(nl, (long)ND * ug.V, theta, cur, out);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }
@@ -907,7 +999,8 @@ int mesh_u1_hmc(mesh_ctx *ctx, const mesh_grid *g, int batch, float *theta, cons
 			return rc;
 		if (!theta || !deltas || !out_dev || ndeltas < 1 || ndeltas % 2 != 1)
 			return mesh_fail(ctx, MESH_E_ARG, "bad u1_hmc arguments (deltas must have odd length)");
-		return u1n_hmc(ctx, ng, batch, theta, deltas, ndeltas, beta, seed, traj, metropolis, out_dev);
+		auto hmc = ng.nd == 2 ? u1n_hmc<2> : (ng.nd == 3 ? u1n_hmc<3> : u1n_hmc<4>);
+		return hmc(ctx, ng, batch, theta, deltas, ndeltas, beta, seed, traj, metropolis, out_dev);
 	}
 	U1Geo ug;
 	if (int rc = u1_setup(ctx, g, batch, &ug))
@@ -918,10 +1011,11 @@ int mesh_u1_hmc(mesh_ctx *ctx, const mesh_grid *g, int batch, float *theta, cons
 		return mesh_fail(ctx, MESH_E_SIZE, "U(1) HMC keeps a configuration in LDS: volume <= 4096");
 	if (int rc = mesh_stage_doubles(ctx, deltas, ndeltas))
 		return rc;
-	size_t lds = 5 * (size_t)ug.V * sizeof(float);
-	MESH_HIP(ctx, hipFuncSetAttribute((const void *)k_u1_hmc, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-	k_u1_hmc<<<batch, U1_THREADS, lds, ctx->stream>>>(ug, theta, ctx->aux, ndeltas, beta, seed, traj, metropolis,
-	                                                  out_dev);
+	// one site a thread up to 1024, then 2 or 4
+	const int spt = ug.V <= 1024 ? 1 : (ug.V <= 2048 ? 2 : 4), nt = ((ug.V + spt - 1) / spt + 63) / 64 * 64;
+	auto kernel = spt == 1 ? k_u1_hmc<1> : (spt == 2 ? k_u1_hmc<2> : k_u1_hmc<4>);
+	const size_t lds = 3 * (size_t)ug.V * sizeof(float); // at most 48 KB
+	kernel<<<batch, nt, lds, ctx->stream>>>(ug, theta, ctx->aux, ndeltas, beta, seed, traj, metropolis, out_dev);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }

@@ -619,3 +619,46 @@ def test_u1_4d_strong_coupling(ctx):
     u = sp.iv(1, beta) / sp.iv(0, beta)
     assert r["acc"].mean() > 0.5
     assert abs(est - u) < 5 * err + 3e-5, (est, u, err)
+
+
+@pytest.mark.parametrize("L0,L1,B", [(2, 2, 3), (3, 5, 4), (8, 8, 2), (5, 13, 2), (32, 32, 2), (25, 41, 2), (32, 64, 2),
+                                    (3, 683, 2), (64, 64, 2), (2, 2048, 1)])
+def test_u1_hmc_sites_per_thread(ctx, L0, L1, B):
+    """the on-chip kernel at its edges -- a wavefront partly filled, the step
+    from one to two and from two to four sites a thread (1024, 2048 sites),
+    the largest lattice -- against the site-parallel kernels: the same angles
+    bit for bit, the sums to FP64 rounding"""
+    d = gauge.makeDeltas("2mn", 0.5, 4)
+    res = []
+    for general in (0, 1):
+        ens = U1.U1Ensemble(L0, L1, B, ctx)
+        ens.random_start(71)
+        with options(ctx, u1_general=general):
+            out = [ens.hmc(2.0, d, 72, t, metropolis=bool(t)) for t in range(3)]
+        res.append((ens.angles(), out))
+    np.testing.assert_array_equal(res[0][0], res[1][0])
+    for a, b in zip(res[0][1], res[1][1]):
+        np.testing.assert_array_equal(a["acc"], b["acc"])
+        # |H| is at most beta V + 4 V of order 1e4: sums in FP64 differ below 1e-9
+        np.testing.assert_allclose(a["dH"], b["dH"], atol=1e-9)
+        np.testing.assert_allclose(a["S"], b["S"], rtol=1e-12)
+
+
+@pytest.mark.parametrize("dims,B", [((2, 2, 2), 3), ((3, 4, 5), 2), ((7, 2, 19), 1), ((2, 2, 2, 2), 2),
+                                    ((3, 2, 5, 4), 2), ((5, 3, 3, 7), 1)])
+def test_u1n_hmc_odd_extents(ctx, dims, B):
+    """the site-parallel trajectory in 3-d and 4-d on odd, smallest (both
+    neighbours the same site) and uneven extents against the FP64 oracle
+    (bounds of test_u1_hmc_against_oracle: FP32 angles, eight steps)"""
+    beta, seed, traj = 1.5, 81, 2
+    ens = U1.U1Ensemble(0, 0, B, ctx, dims=dims)
+    ens.random_start(seed)
+    th0 = ens.angles().astype(np.float64)
+    d = gauge.makeDeltas("2lf", 0.5, 8)
+    ens.hmc(beta, d, seed, traj, metropolis=False)
+    raw, th1 = ens._hmc.download().reshape(B, 4), ens.angles()
+    for c in range(B):
+        t_ref, _, dh_ref = U.nd_hmc_trajectory(th0[c], U.nd_momenta(seed, traj, c, dims), beta, d)
+        assert _wrapdiff(th1[c], t_ref).max() < 2e-4
+        assert abs(raw[c, 0] - dh_ref) < 2e-3 * (1 + abs(dh_ref))
+        assert raw[c, 3] == pytest.approx(U.nd_action_over_beta(t_ref), rel=1e-4)
