@@ -235,25 +235,26 @@ __device__ __forceinline__ void pc_forward(PCGeo const &g, int nl, const float *
 	double v[3] = {ld, 0.0, 0.0}; // log det, S of the free plaquettes, their sum
 	for (int x = threadIdx.x; x < g.V - 1; x += NT)
 	{
-		v[1] += 1.0 - cos((double)phi[x]);
+		v[1] += 1.0 - cos1((double)phi[x]);
 		v[2] += (double)phi[x];
 	}
-	block_sum<3, NT / 64>(v, sh.red);
+	block_sum<3>(v, sh.red);
 	double S = v[1] + (1.0 - cos(wrapd(-v[2])));
 	if (theta_out)
 	{
 		float *o = theta_out + (long)c * 2 * g.V;
 		const float h0 = u1_plaq::uniform_angle(seed, step, (uint32_t)g.V, cc, TAG_PCFZ);
 		const float h1 = u1_plaq::uniform_angle(seed, step, (uint32_t)g.V + 1u, cc, TAG_PCFZ);
-		u1_plaq::links_from_plaquettes(g, phi, h0, h1, al, reinterpret_cast<float *>(cs), o, NT);
+		float *t = reinterpret_cast<float *>(cs);
+		u1_plaq::links_from_plaquettes(g, phi, h0, h1, al, t, o, NT);
 		__syncthreads();
 		double s[1] = {0.0};
 		for (int x = threadIdx.x; x < g.V; x += NT)
 		{
 			const int x0 = x / g.L1, x1 = x - x0 * g.L1;
-			s[0] += 1.0 - cos((double)plaqp(g, o, x0, x1));
+			s[0] += 1.0 - cos1((double)plaqp(g, t, x0, x1));
 		}
-		block_sum<1, NT / 64>(s, sh.red);
+		block_sum<1>(s, sh.red);
 		S = s[0];
 	}
 	if (threadIdx.x == 0)
@@ -286,7 +287,7 @@ __device__ __forceinline__ void pc_inverse(PCGeo const &g, int nl, const float *
 	{
 		const int x0 = x / g.L1, x1 = x - x0 * g.L1;
 		const float tp = plaqp(g, th, x0, x1);
-		v[1] += 1.0 - cos((double)tp);
+		v[1] += 1.0 - cos1((double)tp);
 		phi[x] = x < g.V - 1 ? FM::wrapf(tp) : 0.f;
 	}
 	__syncthreads(); // the links are read; cs takes their place
@@ -302,7 +303,7 @@ __device__ __forceinline__ void pc_inverse(PCGeo const &g, int nl, const float *
 		layer_apply<true, NT>(g, ll, phi, cs, layer & 3, sh, v[0]);
 	}
 	__syncthreads();
-	block_sum<2, NT / 64>(v, sh.red);
+	block_sum<2>(v, sh.red);
 	if (threadIdx.x == 0)
 	{
 		out[2 * c + 0] = -v[0] - 2.0 * g.V * LOG_2PI;

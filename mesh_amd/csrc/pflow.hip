@@ -29,11 +29,6 @@
 #include "rng_dev.h"
 #include "u1_plaq.h"
 
-// log q: table-guided inverse of the circle map (0: Newton from the target)
-#ifndef MESH_PFLOW_TABLE
-#define MESH_PFLOW_TABLE 1
-#endif
-
 using namespace mesh_dev;
 using u1_plaq::block_sum;
 using u1_plaq::PGeo;
@@ -45,7 +40,17 @@ namespace {
 
 constexpr int K = 8;             // components
 constexpr int NPF = 2 * K + 2;   // parameters
-constexpr int THREADS = 256;
+constexpr int THREADS = 256; // of the gradient kernel
+// Sampling and log q of up to two workgroups a CU run on 512 threads (a
+// thread's plaquettes are then the chain that bounds them: 64^2, 256 chains,
+// log q 23.9 us against 35.1 on 256 threads), more of them on 256 (32^2, a
+// round of 1024 chains: 41.1 us against 50.8).
+constexpr int MAX_THREADS = 512;
+int threads_for(u1_plaq::PGeo const &g, int blocks)
+{
+	const int most = blocks <= 2 * 256 ? MAX_THREADS : 256;
+	return g.V >= most ? most : (g.V + 63) / 64 * 64;
+}
 constexpr uint32_t TAG_PFLOW = 0x50464c57u;
 constexpr float PI_F = 3.14159265358979323846f;
 constexpr float TWO_PI_F = 6.28318530717958647692f;
@@ -62,37 +67,55 @@ struct Map
 	float s[K], w[K], t, ta, tb;
 };
 
-__device__ __forceinline__ Map map_params(const float *__restrict__ y)
+// The map's parameters from y by the first nine threads, through LDS (m[2 K + 1])
+// to all: at a thread a plaquette, every thread forming them for itself took as
+// long as a plaquette
+__device__ __forceinline__ Map map_params(const float *__restrict__ y, float *m)
 {
-	Map p;
-	float m = y[K];
-	for (int k = 1; k < K; ++k)
-		m = fmaxf(m, y[K + k]);
-	float z = 0.f;
-	for (int k = 0; k < K; ++k)
+	const int k = threadIdx.x;
+	if (k < K)
 	{
-		p.s[k] = expf(fminf(fmaxf(y[k], -8.f), 8.f));
-		p.w[k] = expf(y[K + k] - m);
-		z += p.w[k];
+		float top = y[K];
+		for (int j = 1; j < K; ++j)
+			top = fmaxf(top, y[K + j]);
+		m[k] = expf(fminf(fmaxf(y[k], -8.f), 8.f));
+		m[K + k] = expf(y[K + k] - top);
 	}
-	for (int k = 0; k < K; ++k)
-		p.w[k] /= z;
+	else if (k == K)
+		m[2 * K] = atan2f(y[2 * K + 1], y[2 * K]);
+	__syncthreads();
+	Map p;
+	p.t = m[2 * K];
+	float z = 0.f;
+	for (int j = 0; j < K; ++j)
+	{
+		p.s[j] = m[j];
+		p.w[j] = m[K + j];
+		z += p.w[j];
+	}
+	__syncthreads();
+	if (k < K)
+		m[K + k] = m[K + k] / z;
+	__syncthreads();
+	for (int j = 0; j < K; ++j)
+		p.w[j] = m[K + j];
 	p.ta = y[2 * K];
 	p.tb = y[2 * K + 1];
-	p.t = atan2f(p.tb, p.ta);
 	return p;
 }
 
 __device__ __forceinline__ void g_eval(Map const &p, float v, float &G, float &Gp)
 {
-	float c = cosf(0.5f * v), sn = sinf(0.5f * v);
+	float c, sn;
+	sincos1(0.5f * v, sn, c);
 	G = 0.f;
 	Gp = 0.f;
+#pragma unroll
 	for (int k = 0; k < K; ++k)
 	{
-		float d = fmaf(c, c, p.s[k] * p.s[k] * sn * sn);
-		G = fmaf(p.w[k], 2.f * atan2f(p.s[k] * sn, c), G);
-		Gp = fmaf(p.w[k], p.s[k] / d, Gp);
+		const float d = fmaf(c, c, p.s[k] * p.s[k] * sn * sn); // e^-16 .. e^16
+		G = fmaf(p.w[k], 2.f * atan2_1(p.s[k] * sn, c), G);
+		Gp = fmaf(p.w[k], div1(p.s[k], d), Gp);
 	}
 }
 
@@ -101,18 +124,20 @@ __device__ __forceinline__ void g_eval(Map const &p, float v, float &G, float &G
 // step or the bracket is below 2e-7 max(1, |v|) -- an FP32 ulp of v is up to
 // 2.4e-7 on [-pi, pi], so an absolute bound would let an iterate that
 // alternates between neighbouring floats run to the cap (at most 40
-// evaluations); returns g'(v) in Gp
-__device__ __forceinline__ float g_inverse(Map const &p, float target, float &Gp, float lo = -PI_F, float hi = PI_F,
-                                           float u = 2.f * PI_F)
+// evaluations) -- or until |g(v) - target| is at the rounding level of g,
+// 2.5e-7 max(1, |target|): where g' is small the residual is noise there, and
+// further steps only wander inside the noise band until the bracket closes (proposal
+// rounds of 256 chains of 32^2 on a trained-looking map: 69 us without this, 38 with it).  Returns g'(v) in Gp
+__device__ __forceinline__ float g_inverse(Map const &p, float target, float &Gp, float lo, float hi, float u)
 {
-	if (u > PI_F)
-		u = target;
 	float G;
+	bool fresh = false; // Gp belongs to the current u
 	for (int b = 0; b < 40; ++b)
 	{
 		g_eval(p, u, G, Gp);
+		fresh = true;
 		float f = G - target;
-		if (f == 0.f)
+		if (fabsf(f) <= 2.5e-7f * fmaxf(1.f, fabsf(target)))
 			break;
 		if (f < 0.f)
 			lo = u;
@@ -120,7 +145,8 @@ __device__ __forceinline__ float g_inverse(Map const &p, float target, float &Gp
 			hi = u;
 		if (hi - lo <= 2e-7f * fmaxf(1.f, fabsf(u)))
 			break;
-		float un = u - f / Gp;
+		float un = u - f * __builtin_amdgcn_rcpf(Gp);
+		fresh = false;
 		if (un > lo && un < hi)
 		{
 			bool done = fabsf(un - u) <= 2e-7f * fmaxf(1.f, fabsf(un));
@@ -131,39 +157,48 @@ __device__ __forceinline__ float g_inverse(Map const &p, float target, float &Gp
 		else
 			u = 0.5f * (lo + hi);
 	}
-	g_eval(p, u, G, Gp);
+	if (!fresh)
+		g_eval(p, u, G, Gp);
 	return u;
 }
 
-// g on the grid v_j = -pi + j 2 pi / NTAB, j = 0..NTAB, one value per thread
-// of the workgroup: G is monotone, so a table lookup brackets the root of
-// g(v) = target within three cells and interpolation starts Newton within
-// about (2 pi / NTAB)^2 of it
+// g and g' on the grid v_j = -pi + j 2 pi / NTAB, j = 0..NTAB: G is monotone, so
+// a table lookup brackets the root of g(v) = target within three cells, and the
+// cubic through the cell's end values and slopes of the inverse starts Newton
+// within about (2 pi / NTAB)^4 of it: one step and the evaluation at its end
+// where the straight line (2 pi / NTAB)^2 took three
 constexpr int NTAB = 256;
-__device__ __forceinline__ void g_table(Map const &p, float *tab)
+struct Table
 {
-	for (int j = threadIdx.x; j <= NTAB; j += THREADS)
-	{
-		float G, Gp;
-		g_eval(p, fmaf((float)j, TWO_PI_F / NTAB, -PI_F), G, Gp);
-		tab[j] = G;
-	}
+	float g[NTAB + 1], gp[NTAB + 1];
+};
+__device__ __forceinline__ void g_table(Map const &p, Table &tab)
+{
+	for (int j = threadIdx.x; j <= NTAB; j += blockDim.x)
+		g_eval(p, fmaf((float)j, TWO_PI_F / NTAB, -PI_F), tab.g[j], tab.gp[j]);
 }
-__device__ __forceinline__ float g_inverse_tab(Map const &p, const float *tab, float target, float &Gp)
+__device__ __forceinline__ float g_inverse_tab(Map const &p, Table const &tab, float target, float &Gp)
 {
 	int a = 0, b = NTAB;
 	while (b - a > 1)
 	{
 		int m = (a + b) >> 1;
-		if (tab[m] <= target)
+		if (tab.g[m] <= target)
 			a = m;
 		else
 			b = m;
 	}
 	const float h = TWO_PI_F / NTAB;
-	const float va = fmaf((float)a, h, -PI_F);
-	const float dG = tab[a + 1] - tab[a];
-	float u = dG > 0.f ? fmaf((target - tab[a]) / dG, h, va) : va + 0.5f * h;
+	const float va = fmaf((float)a, h, -PI_F), ga = tab.g[a];
+	const float dG = tab.g[a + 1] - ga;
+	float u = va + 0.5f * h;
+	if (dG > 0.f)
+	{
+		const float x = fminf(fmaxf((target - ga) / dG, 0.f), 1.f), y = 1.f - x;
+		const float m0 = dG / tab.gp[a], m1 = dG / tab.gp[a + 1]; // slopes of v over x
+		const float e = x * y * (m0 * y - m1 * x) + h * x * x * (3.f - 2.f * x);
+		u = va + fminf(fmaxf(e, 0.f), h);
+	}
 	// one cell of margin either side: the table holds g rounded to FP32
 	const float lo = a > 0 ? va - h : -PI_F, hi = a + 2 <= NTAB ? va + 2.f * h : PI_F;
 	u = fminf(fmaxf(u, lo), hi);
@@ -183,15 +218,16 @@ __device__ __forceinline__ float uniform_angle(uint64_t seed, uint32_t step, uin
 // (V, 2c, ..) and (V+1, 2c, ..); gauge angle a(x) (x, 2c+1, ..).
 // LDS: 4V floats.
 __device__ void pflow_sample(PGeo const &g, const float *__restrict__ params, uint64_t seed, uint32_t step,
-                             float *__restrict__ theta_out, double *out, int c, float *lds, double (*red)[4])
+                             float *__restrict__ theta_out, double *out, int c, float *lds, double (*red)[16])
 {
 	float *P = lds;          // V plaquette angles (the last unused)
 	float *t = lds + g.V;    // 2V links
 	float *al = lds + 3 * g.V; // V gauge angles
-	const Map p = map_params(params);
+	__shared__ float mp[2 * K + 1];
+	const Map p = map_params(params, mp);
 	const uint32_t cc = (uint32_t)c << 1;
 	double v[1] = {0.0};
-	for (int x = threadIdx.x; x < g.V; x += THREADS)
+	for (int x = threadIdx.x; x < g.V; x += blockDim.x)
 	{
 		if (x < g.V - 1)
 		{
@@ -206,15 +242,15 @@ __device__ void pflow_sample(PGeo const &g, const float *__restrict__ params, ui
 	const float h0 = uniform_angle(seed, step, (uint32_t)g.V, cc);
 	const float h1 = uniform_angle(seed, step, (uint32_t)g.V + 1u, cc);
 	float *o = theta_out + (long)c * 2 * g.V;
-	u1_plaq::links_from_plaquettes(g, P, h0, h1, al, t, o, THREADS);
+	u1_plaq::links_from_plaquettes(g, P, h0, h1, al, t, o, blockDim.x);
 	if (!out)
 		return;
 	__syncthreads();
 	double w[2] = {v[0], 0.0};
-	for (int x = threadIdx.x; x < g.V; x += THREADS)
+	for (int x = threadIdx.x; x < g.V; x += blockDim.x)
 	{
 		const int x0 = x / g.L1, x1 = x - x0 * g.L1;
-		w[1] += 1.0 - cos((double)plaqp(g, o, x0, x1));
+		w[1] += 1.0 - cos1((double)plaqp(g, t, x0, x1));
 	}
 	block_sum<2>(w, red);
 	if (threadIdx.x == 0)
@@ -227,27 +263,24 @@ __device__ void pflow_sample(PGeo const &g, const float *__restrict__ params, ui
 // out[2c + {0,1}] = {log q(U), S(U)/beta} of configurations theta[c][2V];
 // LDS: 2V floats
 __device__ void pflow_logq(PGeo const &g, const float *__restrict__ params, const float *__restrict__ theta,
-                           double *out, int c, float *t, double (*red)[4], float *tab)
+                           double *out, int c, float *t, double (*red)[16], Table &tab)
 {
-	const Map p = map_params(params);
-	for (int i = threadIdx.x; i < 2 * g.V; i += THREADS)
+	__shared__ float mp[2 * K + 1];
+	const Map p = map_params(params, mp);
+	for (int i = threadIdx.x; i < 2 * g.V; i += blockDim.x)
 		t[i] = theta[(long)c * 2 * g.V + i];
-	if (MESH_PFLOW_TABLE)
-		g_table(p, tab);
+	g_table(p, tab);
 	__syncthreads();
 	double v[2] = {0.0, 0.0};
-	for (int x = threadIdx.x; x < g.V; x += THREADS)
+	for (int x = threadIdx.x; x < g.V; x += blockDim.x)
 	{
 		int x0 = x / g.L1, x1 = x - x0 * g.L1;
 		float tp = plaqp(g, t, x0, x1);
-		v[1] += 1.0 - cos((double)tp);
+		v[1] += 1.0 - cos1((double)tp);
 		if (x < g.V - 1)
 		{
 			float Gp;
-			if (MESH_PFLOW_TABLE)
-				g_inverse_tab(p, tab, wrapf(tp - p.t), Gp);
-			else
-				g_inverse(p, wrapf(tp - p.t), Gp);
+			g_inverse_tab(p, tab, wrapf(tp - p.t), Gp);
 			v[0] -= (double)logf(Gp);
 		}
 	}
@@ -259,33 +292,33 @@ __device__ void pflow_logq(PGeo const &g, const float *__restrict__ params, cons
 	}
 }
 
-__global__ __launch_bounds__(THREADS) void k_pflow_sample(PGeo g, const float *__restrict__ params, uint64_t seed,
+__global__ __launch_bounds__(MAX_THREADS) void k_pflow_sample(PGeo g, const float *__restrict__ params, uint64_t seed,
                                                           uint32_t step, float *__restrict__ theta_out)
 {
 	extern __shared__ float lds[];
 	pflow_sample(g, params, seed, step, theta_out, nullptr, blockIdx.x, lds, nullptr);
 }
 
-__global__ __launch_bounds__(THREADS) void k_pflow_logq(PGeo g, const float *__restrict__ params,
+__global__ __launch_bounds__(MAX_THREADS) void k_pflow_logq(PGeo g, const float *__restrict__ params,
                                                         const float *__restrict__ theta, double *out)
 {
 	extern __shared__ float t[]; // 2V
-	__shared__ double red[2][4];
-	__shared__ float tab[NTAB + 1];
+	__shared__ double red[2][16];
+	__shared__ Table tab;
 	pflow_logq(g, params, theta, out, blockIdx.x, t, red, tab);
 }
 
 // one MH proposal round in one launch: workgroups 0..batch-1 take log q of
 // the current configurations, batch..2 batch-1 draw the proposals with their
 // log q and S/beta, side by side on the CUs
-__global__ __launch_bounds__(THREADS) void k_pflow_propose(PGeo g, const float *__restrict__ params, int batch,
+__global__ __launch_bounds__(MAX_THREADS) void k_pflow_propose(PGeo g, const float *__restrict__ params, int batch,
                                                            const float *__restrict__ theta, double *state,
                                                            uint64_t seed, uint32_t step, float *theta_prop,
                                                            double *prop_out)
 {
 	extern __shared__ float lds[];
-	__shared__ double red[2][4];
-	__shared__ float tab[NTAB + 1];
+	__shared__ double red[2][16];
+	__shared__ Table tab;
 	if ((int)blockIdx.x < batch)
 		pflow_logq(g, params, theta, state, blockIdx.x, lds, red, tab);
 	else
@@ -303,7 +336,8 @@ __global__ __launch_bounds__(THREADS) void k_pflow_grad(PGeo g, const float *__r
 	__shared__ double s_last;
 	const int c = blockIdx.x;
 	const float *y = params;
-	const Map p = map_params(y);
+	__shared__ float mp[2 * K + 1];
+	const Map p = map_params(y, mp);
 	const uint32_t cc = (uint32_t)c << 1;
 	// pass 1: sum of the free plaquettes (fixes the last one)
 	double v1[1] = {0.0};
@@ -326,23 +360,24 @@ __global__ __launch_bounds__(THREADS) void k_pflow_grad(PGeo g, const float *__r
 	for (int x = threadIdx.x; x < g.V - 1; x += THREADS)
 	{
 		float v = wrapf(uniform_angle(seed, step, (uint32_t)x, cc) - p.t);
-		float cs = cosf(0.5f * v), sn = sinf(0.5f * v);
+		float cs, sn;
+		sincos1(0.5f * v, sn, cs);
 		float G = 0.f, Gp = 0.f, Gpp = 0.f, gk[K], gpk[K], dgs[K], dgps[K];
 		for (int k = 0; k < K; ++k)
 		{
-			float s2 = p.s[k] * p.s[k];
-			float d = fmaf(cs, cs, s2 * sn * sn);
-			gk[k] = 2.f * atan2f(p.s[k] * sn, cs);
-			gpk[k] = p.s[k] / d;
-			dgs[k] = 2.f * sn * cs / d;
-			dgps[k] = (cs * cs - s2 * sn * sn) / (d * d);
+			const float s2 = p.s[k] * p.s[k];
+			const float d = fmaf(cs, cs, s2 * sn * sn), id = div1(1.f, d);
+			gk[k] = 2.f * atan2_1(p.s[k] * sn, cs);
+			gpk[k] = p.s[k] * id;
+			dgs[k] = 2.f * sn * cs * id;
+			dgps[k] = (cs * cs - s2 * sn * sn) * (id * id);
 			G = fmaf(p.w[k], gk[k], G);
 			Gp = fmaf(p.w[k], gpk[k], Gp);
-			Gpp = fmaf(p.w[k], -p.s[k] * (s2 - 1.f) * sn * cs / (d * d), Gpp);
+			Gpp = fmaf(p.w[k], -p.s[k] * (s2 - 1.f) * sn * cs * (id * id), Gpp);
 		}
 		float th = wrapf(G + p.t);
 		acc[NPF] += -(double)logf(Gp);
-		acc[NPF + 1] += 1.0 - cos((double)th);
+		acc[NPF + 1] += 1.0 - cos1((double)th);
 		// dL/dtheta_P (through beta S and the last plaquette)
 		float A = (float)beta * (sinf(th) - sin_last);
 		float iG = 1.f / Gp;
@@ -436,7 +471,7 @@ int mesh_pflow_sample(mesh_ctx *ctx, const mesh_grid *g, int batch, const float 
 	size_t lds = 4 * (size_t)pg.V * sizeof(float);
 	MESH_HIP(ctx, hipFuncSetAttribute((const void *)k_pflow_sample, hipFuncAttributeMaxDynamicSharedMemorySize,
 	                                  (int)lds));
-	k_pflow_sample<<<batch, THREADS, lds, ctx->stream>>>(pg, params, seed, step, theta_out);
+	k_pflow_sample<<<batch, threads_for(pg, batch), lds, ctx->stream>>>(pg, params, seed, step, theta_out);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }
@@ -455,8 +490,8 @@ int mesh_pflow_propose(mesh_ctx *ctx, const mesh_grid *g, int batch, const float
 	size_t lds = 4 * (size_t)pg.V * sizeof(float);
 	MESH_HIP(ctx, hipFuncSetAttribute((const void *)k_pflow_propose, hipFuncAttributeMaxDynamicSharedMemorySize,
 	                                  (int)lds));
-	k_pflow_propose<<<2 * batch, THREADS, lds, ctx->stream>>>(pg, params, batch, theta, state_dev, seed, step,
-	                                                          theta_prop, prop_dev);
+	k_pflow_propose<<<2 * batch, threads_for(pg, 2 * batch), lds, ctx->stream>>>(pg, params, batch, theta, state_dev,
+	                                                                             seed, step, theta_prop, prop_dev);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }
@@ -471,7 +506,7 @@ int mesh_pflow_logq(mesh_ctx *ctx, const mesh_grid *g, int batch, const float *p
 	if (!params || !theta || !out_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pflow_logq");
 	size_t lds = 2 * (size_t)pg.V * sizeof(float);
-	k_pflow_logq<<<batch, THREADS, lds, ctx->stream>>>(pg, params, theta, out_dev);
+	k_pflow_logq<<<batch, threads_for(pg, batch), lds, ctx->stream>>>(pg, params, theta, out_dev);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }

@@ -18,6 +18,7 @@
 
 #include "mesh_internal.h"
 #include "rng_dev.h"
+#include "trig_dev.h"
 
 namespace u1_plaq {
 
@@ -56,10 +57,10 @@ __device__ __forceinline__ float uniform_angle(uint64_t seed, uint32_t step, uin
 	return (float)(6.283185307179586477 * u - 3.141592653589793238);
 }
 
-// sums over the NW wavefronts of a workgroup, in a fixed order
-template <int NQ, int NW = 4> __device__ __forceinline__ void block_sum(double (&v)[NQ], double (*red)[NW])
+// sums over the wavefronts of a workgroup (at most NW), in a fixed order
+template <int NQ, int NW> __device__ __forceinline__ void block_sum(double (&v)[NQ], double (*red)[NW])
 {
-	int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
 	for (int q = 0; q < NQ; ++q)
 	{
 		double s = v[q];
@@ -72,7 +73,7 @@ template <int NQ, int NW = 4> __device__ __forceinline__ void block_sum(double (
 	for (int q = 0; q < NQ; ++q)
 	{
 		v[q] = red[q][0];
-		for (int i = 1; i < NW; ++i)
+		for (int i = 1; i < nw; ++i)
 			v[q] += red[q][i];
 	}
 	__syncthreads();
@@ -86,44 +87,76 @@ __device__ __forceinline__ float wrapf_p(float a)
 }
 
 // links out[2V] of the free plaquettes P[V] (the last unused), holonomies
-// h0, h1 and gauge angles al[V]; t[2V] is LDS scratch.  Called by every
-// thread of the workgroup; P and al must be visible to all of them.
-__device__ void links_from_plaquettes(PGeo const &g, const float *P, float h0, float h1, const float *al, float *t,
-                                      float *__restrict__ out, int nthreads)
+// h0, h1 and gauge angles al[V]; t[2V] is LDS, which holds the links as well
+// at the end (a barrier before another thread's).  Called by every thread of
+// the workgroup; P and al must be visible to all of them.  The sums run in the
+// order of the formulas above; what a sum adds is read ahead of it, so that
+// only the additions are a chain.
+__device__ __forceinline__ void links_from_plaquettes(PGeo const &g, const float *P, float h0, float h1,
+                                                      const float *al, float *t, float *__restrict__ out, int nthreads)
 {
+	constexpr int AHEAD = 8;
 	// direction 0: suffix sums along each row (one thread per row)
 	for (int x0 = threadIdx.x; x0 < g.L0; x0 += nthreads)
 	{
+		const float *p = P + x0 * g.L1;
+		float *r = t + x0 * g.L1;
 		double acc = x0 == g.L0 - 1 ? (double)h0 : 0.0;
-		t[x0 * g.L1 + g.L1 - 1] = (float)wrapd(acc);
-		for (int x1 = g.L1 - 2; x1 >= 0; --x1)
+		r[g.L1 - 1] = (float)wrapd(acc);
+		int x1 = g.L1 - 2;
+		for (; x1 >= AHEAD - 1; x1 -= AHEAD)
 		{
-			acc += (double)P[x0 * g.L1 + x1];
-			t[x0 * g.L1 + x1] = (float)wrapd(acc);
+			float v[AHEAD];
+#pragma unroll
+			for (int k = 0; k < AHEAD; ++k)
+				v[k] = p[x1 - k];
+#pragma unroll
+			for (int k = 0; k < AHEAD; ++k)
+			{
+				acc += (double)v[k];
+				r[x1 - k] = (float)wrapd(acc);
+			}
 		}
-		for (int x1 = 0; x1 < g.L1 - 1; ++x1)
-			t[g.V + x0 * g.L1 + x1] = 0.f;
+		for (; x1 >= 0; --x1)
+		{
+			acc += (double)p[x1];
+			r[x1] = (float)wrapd(acc);
+		}
 	}
 	__syncthreads();
-	// direction 1, last column: prefix sum over rows (one thread)
-	if (threadIdx.x == 0)
+	// direction 1, last column: prefix sum over rows by one wavefront, a row a
+	// lane (the other columns are zero)
+	float *t1 = t + g.V;
+	if (threadIdx.x < 64)
 	{
 		double acc = (double)h1;
-		t[g.V + g.L1 - 1] = (float)wrapd(acc);
-		for (int x0 = 0; x0 + 1 < g.L0; ++x0)
+		for (int r0 = 0; r0 < g.L0; r0 += 64)
 		{
-			int r = x0 * g.L1;
-			acc += (double)P[r + g.L1 - 1] - (double)t[r + g.L1 - 1] + (double)t[r];
-			t[g.V + r + g.L1 + g.L1 - 1] = (float)wrapd(acc);
+			const int x0 = r0 + (int)threadIdx.x, r = x0 * g.L1;
+			// t1(x0) is h1 and the terms of the rows before x0
+			const double term =
+			    x0 < g.L0 ? (double)P[r + g.L1 - 1] - (double)t[r + g.L1 - 1] + (double)t[r] : 0.0;
+			const int n = g.L0 - r0 < 64 ? g.L0 - r0 : 64;
+			double mine = acc;
+			for (int i = 0; i < n; ++i)
+			{
+				if ((int)threadIdx.x == i)
+					mine = acc;
+				acc += __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(term), i),
+				                        __builtin_amdgcn_readlane(__double2loint(term), i));
+			}
+			if (x0 < g.L0)
+				t1[r + g.L1 - 1] = (float)wrapd(mine);
 		}
 	}
 	__syncthreads();
 	// gauge transformation into the output
 	for (int x = threadIdx.x; x < g.V; x += nthreads)
 	{
-		int x0 = x / g.L1, x1 = x - x0 * g.L1;
-		out[x] = wrapf_p(t[x] + al[x] - al[site(g, x0 + 1, x1)]);
-		out[g.V + x] = wrapf_p(t[g.V + x] + al[x] - al[site(g, x0, x1 + 1)]);
+		const int x0 = x / g.L1, x1 = x - x0 * g.L1;
+		const float a = t[x], b = x1 == g.L1 - 1 ? t1[x] : 0.f;
+		out[x] = t[x] = wrapf_p(a + al[x] - al[site(g, x0 + 1, x1)]);
+		out[g.V + x] = t1[x] = wrapf_p(b + al[x] - al[site(g, x0, x1 + 1)]);
 	}
 }
 

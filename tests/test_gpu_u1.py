@@ -412,6 +412,41 @@ def test_pflow_logq_of_given_configurations(ctx):
     np.testing.assert_allclose(out[:, 1], S, rtol=1e-5)
 
 
+@pytest.mark.parametrize("L0,L1,scale", [(2, 2, 0.5), (3, 11, 2.0), (130, 2, 0.5), (2, 514, 0.5), (64, 64, 1.0),
+                                         (2, 2048, 0.5)])
+def test_pflow_edges(ctx, L0, L1, scale):
+    """smallest and largest lattices, more rows than a wavefront (the column's
+    prefix sum goes on over 64 rows), rows past and between the read-ahead
+    blocks, and a steep map (log s_k of width 2): links and log q of samples
+    against the oracle, log q of the samples by the table-guided inverse
+    against its bisection.  Bounds: one FP32 log g' a plaquette, as above;
+    links sum up to V / 2 plaquettes of FP32 error 1e-6."""
+    torch = pytest.importorskip("torch")
+    B, seed, step, V = 2, 65, 3, L0 * L1
+    tol = 5e-3 * max(1.0, V / 64)
+    p = _pparams(66, scale)
+    f = U1.PlaqFlow(L0, L1, ctx)
+    f.set_params(p)
+    ens = U1.U1Ensemble(L0, L1, B, ctx)
+    out = f.sample(ens, seed, step).download().reshape(B, 2)
+    th = ens.angles().astype(np.float64)
+    state, pout = (U1.Buffer(2 * B, np.float64, ctx) for _ in range(2))
+    prop = U1.Buffer(2 * B * V, np.float32, ctx)
+    f.propose(ens, state, seed, step, prop, pout)
+    np.testing.assert_array_equal(prop.download().reshape(th.shape), th.astype(np.float32))
+    np.testing.assert_array_equal(state.download().reshape(B, 2), out)
+    pt = torch.tensor(p.astype(np.float64))
+    for c in range(B):
+        u, a, h0, h1 = U.pflow_draws(seed, step, c, L0, L1)
+        thP, nlg = U.pflow_h(pt, torch.tensor(u.astype(np.float64)))
+        ref = U.pflow_links(thP.numpy(), h0, h1, a, L0, L1)
+        assert _wrapdiff(th[c], ref).max() < 2e-4 + 1e-6 * V, c
+        lq, S = U.pflow_logq(p, th[c])
+        assert abs(out[c, 0] - lq) < tol, (c, out[c, 0], lq)
+        assert abs(pout.download().reshape(B, 2)[c, 0] - (nlg.sum().item() - 2 * V * math.log(2 * math.pi))) < tol
+        assert out[c, 1] == pytest.approx(S, rel=1e-5)
+
+
 def test_pflow_propose(ctx):
     """mesh_pflow_propose: the states' (log q, S/beta) are mesh_pflow_logq's
     bit for bit, the proposals mesh_pflow_sample's, and the proposals' log q
