@@ -826,6 +826,38 @@ MHD void x3_slots(Geo const &g, long x, int const *c, int &sp, int &sm)
 	sm = block_slot(o0 + (c3 == 0 ? L3 - 1 : c3 - 1));
 }
 
+// Slots of a block staged in LDS by the fused MD step, for any L3: a block of n
+// consecutive sites has at most four x3-neighbours outside it -- those of its
+// first row if it starts inside that row (the site before the block, and the
+// row's start, where the row's end wraps to) and those of its last row if it
+// ends inside it.  They are staged in slots 64 .. 67.
+
+// what a lane of the staged kernels reads: its own slot and those of x +/- e3
+struct LaneSlots
+{
+	int me, sp, sm;
+};
+
+// the block of n sites from b0: slots of lane site b0 + l with coordinate c3 along x3
+MHD LaneSlots halo_slots(int L3, int n, int l, int c3)
+{
+	const int fwd = c3 + 1 < L3 ? l + 1 : l + 1 - L3, bwd = c3 > 0 ? l - 1 : l - 1 + L3;
+	LaneSlots s;
+	s.me = block_slot(l);
+	s.sp = fwd < 0 ? 65 : (fwd >= n ? 66 : block_slot(fwd));
+	s.sm = bwd < 0 ? 64 : (bwd >= n ? 67 : block_slot(bwd));
+	return s;
+}
+// site of halo slot 64 + h: the site before the block, the first row's start,
+// the site behind the block, the last row's end (b0, or a site of the block,
+// where no lane reads the slot)
+MHD long halo_site(int L3, long b0, int n, int h)
+{
+	const long bl = b0 + n - 1;
+	const int c3f = (int)((unsigned)b0 % (unsigned)L3), c3l = (int)((unsigned)bl % (unsigned)L3);
+	return h == 0 ? (c3f > 0 ? b0 - 1 : b0) : (h == 1 ? b0 - c3f : (h == 2 ? (c3l < L3 - 1 ? bl + 1 : b0) : bl - c3l + L3 - 1));
+}
+
 // Rows path of the fused MD step (4-d, V % 64 == 0, L3 | 64 and
 // (L2 L3) % 64 == 0): a 64-site block holds whole x3-rows and lies within one
 // (x0, x1) plane.  A shift along x0 or x1 then moves every site of a block by

@@ -19,7 +19,7 @@
 
 using namespace mesh_dev;
 
-// FP64 row-staged staples software-pipelined (staple_rows_pipe; same bits)
+// FP64 staged staples software-pipelined (staple_pipe; same bits)
 #ifndef MESH_PIPE_F64
 #define MESH_PIPE_F64 1
 #endif
@@ -47,7 +47,7 @@ using namespace mesh_dev;
 #ifndef MESH_FORCE_WAVES_F32
 #define MESH_FORCE_WAVES_F32 0
 #endif
-// ... and for the FP64 kernel with the row-staged staple path (0: as above;
+// ... and for the FP64 staged kernels (0: as above;
 // 3 fits in 168 VGPRs but measured slower than two).  The pipelined staples
 // would take 260 registers and one wave; 2 holds them at two waves with three
 // VGPRs spilled, 1.1% faster than the unpipelined kernel at two waves and 16%
@@ -55,20 +55,20 @@ using namespace mesh_dev;
 #ifndef MESH_FORCE_WAVES_ROWS
 #define MESH_FORCE_WAVES_ROWS (MESH_PIPE_F64 ? 2 : 0)
 #endif
-// upper bound of waves per SIMD for the FP64 kernel with the row-staged staple
-// path (8: none): it runs at two either way (170 VGPRs), and with the bound the
-// compiler may spend the registers up to 256 on loads in flight
+// upper bound of waves per SIMD for the FP64 staged kernels (8: none): they run
+// at two either way (170 VGPRs), and with the bound the compiler may spend the
+// registers up to 256 on loads in flight
 #ifndef MESH_FORCE_MAXW_ROWS
 #define MESH_FORCE_MAXW_ROWS 2
 #endif
 template <class R, int PATH = 0> constexpr int force_max_waves()
 {
-	return (std::is_same<R, double>::value && PATH == 2) ? MESH_FORCE_MAXW_ROWS : 8;
+	return (std::is_same<R, double>::value && PATH != 0) ? MESH_FORCE_MAXW_ROWS : 8;
 }
 template <class R, int PATH = 0> constexpr int force_min_waves()
 {
 	return (std::is_same<R, float>::value && MESH_FORCE_WAVES_F32 > 0) ? MESH_FORCE_WAVES_F32
-	       : (std::is_same<R, double>::value && PATH == 2 && MESH_FORCE_WAVES_ROWS > 0)
+	       : (std::is_same<R, double>::value && PATH != 0 && MESH_FORCE_WAVES_ROWS > 0)
 	           ? MESH_FORCE_WAVES_ROWS
 	           : (MESH_FORCE_WAVES > 0 ? MESH_FORCE_WAVES : 1);
 }
@@ -116,14 +116,6 @@ __host__ __device__ constexpr int shared_planes(int m) { return m == 2 ? 6 : (m 
 #define DH_OCC __attribute__((amdgpu_waves_per_eu(1, MESH_DH_WAVES)))
 #else
 #define DH_OCC
-#endif
-// variant 0 stages the workgroup's own-site links in LDS (4-d, V % 64 == 0)
-#ifndef MESH_OWN_LDS
-#define MESH_OWN_LDS 1
-#endif
-// ... and, when the block holds whole x3-rows, the links of the x3-neighbours
-#ifndef MESH_OWN_ROWS
-#define MESH_OWN_ROWS 1
 #endif
 // staples with the direction as a compile-time constant (4-d lattices)
 #ifndef MESH_STATIC_MU
@@ -222,46 +214,19 @@ template <class R> __device__ __forceinline__ m3<R> staple_at(Geo const &g, cons
 	return S;
 }
 
-// The same for a compile-time direction of a 4-d lattice: no branch between
-// the six staples, so the compiler can issue the loads of later staples
-// while earlier ones multiply (same operations in the same order).
-template <int MU, class R>
-__device__ __forceinline__ m3<R> staple_4d(Geo const &g, const R *__restrict__ U, long x, int const *c)
-{
-	m3<R> S = zero_m3<R>();
-	long xpm = shift_c(g, x, MU, c[MU], 1);
-#pragma unroll
-	for (int nu = 0; nu < 4; ++nu)
-	{
-		if (nu == MU)
-			continue;
-		long xpn = shift_c(g, x, nu, c[nu], 1);
-		long xmn = shift_c(g, x, nu, c[nu], -1);
-		long xpmmn = shift_c(g, xpm, nu, c[nu], -1);
-		{
-			m3<R> T1 = upper_factor(load(U, nu, g, xpm), load(U, MU, g, xpn), nu < MU);
-			madd_nd(S, T1, load(U, nu, g, x));
-		}
-		{
-			m3<R> T2 = mul_dd(load(U, nu, g, xpmmn), load(U, MU, g, xmn));
-			madd_nn(S, T2, load(U, nu, g, xmn));
-		}
-	}
-	return S;
-}
-
-// The same with links read from the workgroup's 64-site block staged in LDS
+// The 4-d kernels read links of the workgroup's 64-site block from LDS
 // (own[d][k][slot], staged once by the workgroup instead of once per
-// direction's wavefront): the four links of site x, and with ROWS (the block
-// holds whole x3-rows, L3 | 64) also those of its x3-neighbours.
+// direction's wavefront): the four links of site x and those of its
+// x3-neighbours (LaneSlots).
 
-template <class R> __device__ __forceinline__ m3<R> lds_m3(vec2_t<R> (*a)[9][64], int d, int slot)
+// matrix d of a slot
+template <class V, int N> __device__ __forceinline__ auto lds_m3(V (*a)[9][N], int d, int slot)
 {
-	m3<R> m;
+	m3<decltype(V::x)> m;
 #pragma unroll
 	for (int k = 0; k < 9; ++k)
 	{
-		vec2_t<R> v = a[d][k][slot];
+		const V v = a[d][k][slot];
 		m.e[k] = {v.x, v.y};
 	}
 	return m;
@@ -359,8 +324,8 @@ template <int W, int MODE, class F> __device__ __forceinline__ void for_shared_p
 		f(I0{}, I3{}, I0{});
 }
 
-// the factors' operands that come from global memory (with ROWS the x3-
-// neighbour ones come from the staged block): loaded by share_fetch before
+// the factors' operands that come from global memory (the x3-neighbour ones
+// come from the staged block): loaded by share_fetch before
 // the staging barrier, since they do not depend on it, so that their latency
 // overlaps the staging's
 template <class R> struct ShareOps
@@ -377,29 +342,26 @@ __device__ __forceinline__ void share_fetch(Geo const &g, const R *__restrict__ 
 		A = rows_at(g, x, c);
 	for_shared_planes<W, MODE>([&](auto P, auto Q, auto I) {
 		constexpr int p = decltype(P)::value, q = decltype(Q)::value, i = decltype(I)::value;
-		if constexpr (!(ROWS && p == 3))
+		if constexpr (p != 3)
 			F.a[i] = load_disp<ROWS>(U, q, g, A, p, 1, -1, 0, shift_c(g, x, p, c[p], 1));
-		if constexpr (!(ROWS && q == 3))
+		if constexpr (q != 3)
 			F.b[i] = load_disp<ROWS>(U, p, g, A, q, 1, -1, 0, shift_c(g, x, q, c[q], 1));
 	});
 }
 
-template <int W, bool ROWS, int MODE, class R>
-__device__ __forceinline__ void share_upper_factors(Geo const &g, long x, int const *c, vec2_t<R> (*own)[9][64],
-                                                    vec2_t<R> (*sh)[9][64], int lane, ShareOps<R> const &F)
+template <int W, int MODE, class R, int N>
+__device__ __forceinline__ void share_upper_factors(vec2_t<R> (*own)[9][N], vec2_t<R> (*sh)[9][64],
+                                                    LaneSlots const &at, int lane, ShareOps<R> const &F)
 {
-	int sp = 0, sm = 0;
-	if constexpr (ROWS)
-		x3_slots(g, x, c, sp, sm);
 	for_shared_planes<W, MODE>([&](auto P, auto Q, auto I) {
 		constexpr int p = decltype(P)::value, q = decltype(Q)::value, i = decltype(I)::value;
 		m3<R> a, b;
-		if constexpr (ROWS && p == 3)
-			a = lds_m3<R>(own, q, sp);
+		if constexpr (p == 3)
+			a = lds_m3(own, q, at.sp);
 		else
 			a = F.a[i];
-		if constexpr (ROWS && q == 3)
-			b = lds_m3<R>(own, p, sp);
+		if constexpr (q == 3)
+			b = lds_m3(own, p, at.sp);
 		else
 			b = F.b[i];
 		m3<R> A = mul_nd(a, b);
@@ -409,17 +371,17 @@ __device__ __forceinline__ void share_upper_factors(Geo const &g, long x, int co
 	});
 }
 
-// SH: share mode of the first upper-staple factors (share_upper_factors)
-template <int MU, bool ROWS, class R, int SH = 0>
+// SH: share mode of the first upper-staple factors (share_upper_factors);
+// ROWS: the links displaced along x0, x1 and x3 alone are addressed from the
+// block's index in scalar registers (STAPLE_ROWS)
+template <int MU, bool ROWS, int SH, class R, int N>
 __device__ __forceinline__ m3<R> staple_4d_own(Geo const &g, const R *__restrict__ U, long x, int const *c,
-                                               vec2_t<R> (*own)[9][64], int lane, vec2_t<R> (*sh)[9][64] = nullptr)
+                                               vec2_t<R> (*own)[9][N], LaneSlots const &at, int lane,
+                                               vec2_t<R> (*sh)[9][64])
 {
-	auto own_at = [&](int d, int slot) { return lds_m3<R>(own, d, slot); };
-	// slots of the x3-neighbours x +/- e3 (used with ROWS only)
 	RowsAt A{};
 	if constexpr (ROWS)
 		A = rows_at(g, x, c);
-	const int sp = A.sp, sm = A.sm;
 	m3<R> S = zero_m3<R>();
 	long xpm = shift_c(g, x, MU, c[MU], 1);
 #pragma unroll
@@ -427,47 +389,48 @@ __device__ __forceinline__ m3<R> staple_4d_own(Geo const &g, const R *__restrict
 	{
 		if (nu == MU)
 			continue;
-		const bool fwd3 = ROWS && MU == 3; // x + mu is an x3-neighbour
-		const bool nu3 = ROWS && nu == 3;  // x +/- nu are x3-neighbours
+		const bool nu3 = nu == 3; // x +/- nu are x3-neighbours
 		long xpn = nu3 ? 0 : shift_c(g, x, nu, c[nu], 1);
 		long xmn = nu3 ? 0 : shift_c(g, x, nu, c[nu], -1);
 		long xpmmn = shift_c(g, xpm, nu, c[nu], -1);
 		if (plane_shared(SH, nu < MU ? nu : MU, nu < MU ? MU : nu))
 		{
-			m3<R> T1 = nu < MU ? adj_m3(lds_m3<R>(sh, share_slot(SH, nu, MU), lane))
-			                   : lds_m3<R>(sh, share_slot(SH, MU, nu), lane);
-			madd_nd(S, T1, own_at(nu, lane));
+			m3<R> T1 = nu < MU ? adj_m3(lds_m3(sh, share_slot(SH, nu, MU), lane))
+			                   : lds_m3(sh, share_slot(SH, MU, nu), lane);
+			madd_nd(S, T1, lds_m3(own, nu, at.me));
 		}
 		else
 		{
-			m3<R> a = fwd3 ? own_at(nu, sp) : load_disp<ROWS>(U, nu, g, A, MU, 1, -1, 0, xpm);
-			m3<R> b = nu3 ? own_at(MU, sp) : load_disp<ROWS>(U, MU, g, A, nu, 1, -1, 0, xpn);
+			m3<R> a = MU == 3 ? lds_m3(own, nu, at.sp) : load_disp<ROWS>(U, nu, g, A, MU, 1, -1, 0, xpm);
+			m3<R> b = nu3 ? lds_m3(own, MU, at.sp) : load_disp<ROWS>(U, MU, g, A, nu, 1, -1, 0, xpn);
 			m3<R> T1 = upper_factor(a, b, nu < MU);
-			madd_nd(S, T1, own_at(nu, lane));
+			madd_nd(S, T1, lds_m3(own, nu, at.me));
 		}
 		{
 			m3<R> a = load_disp<ROWS>(U, nu, g, A, MU, 1, nu, -1, xpmmn);
-			m3<R> b = nu3 ? own_at(MU, sm) : load_disp<ROWS>(U, MU, g, A, nu, -1, -1, 0, xmn);
+			m3<R> b = nu3 ? lds_m3(own, MU, at.sm) : load_disp<ROWS>(U, MU, g, A, nu, -1, -1, 0, xmn);
 			m3<R> T2 = mul_dd(a, b);
-			madd_nn(S, T2, nu3 ? own_at(nu, sm) : load_disp<ROWS>(U, nu, g, A, nu, -1, -1, 0, xmn));
+			madd_nn(S, T2, nu3 ? lds_m3(own, nu, at.sm) : load_disp<ROWS>(U, nu, g, A, nu, -1, -1, 0, xmn));
 		}
 	}
 	return S;
 }
 
-// staple_4d_own for whole x3-rows in the block (ROWS) with shared upper
-// factors, software-pipelined: every product's phase first issues the global
+// staple_4d_own software-pipelined: every product's phase first issues the global
 // loads the next phase needs, and __builtin_amdgcn_sched_barrier keeps them
 // ahead of the arithmetic, so that a wavefront multiplies while its next links
 // are in flight (the compiler's own schedule waits on one link's loads at a
 // time).  The operations and their order are those of staple_4d_own, so the
 // bits are the same; at most five links are live.
-template <int MU, int SH, class R>
-__device__ __forceinline__ m3<R> staple_rows_pipe(Geo const &g, const R *__restrict__ U, long x, int const *c,
-                                                  vec2_t<R> (*own)[9][64], int lane, vec2_t<R> (*sh)[9][64])
+template <int MU, bool ROWS, int SH, class R, int N>
+__device__ __forceinline__ m3<R> staple_pipe(Geo const &g, const R *__restrict__ U, long x, int const *c,
+                                             vec2_t<R> (*own)[9][N], LaneSlots const &at, int lane,
+                                             vec2_t<R> (*sh)[9][64])
 {
-	const RowsAt At = rows_at(g, x, c);
-	const int sp = At.sp, sm = At.sm;
+	RowsAt At{};
+	if constexpr (ROWS)
+		At = rows_at(g, x, c);
+	const int sp = at.sp, sm = at.sm;
 	const long xpm = shift_c(g, x, MU, c[MU], 1);
 	m3<R> S = zero_m3<R>(), A, B, La, Lb, Lc;
 	// operands of the upper staple's first product (planes not shared)
@@ -475,27 +438,27 @@ __device__ __forceinline__ m3<R> staple_rows_pipe(Geo const &g, const R *__restr
 		constexpr int nu = decltype(NU)::value;
 		if constexpr (!plane_shared(SH, nu < MU ? nu : MU, nu < MU ? MU : nu))
 		{
-			A = MU == 3 ? lds_m3<R>(own, nu, sp) : load_disp<true>(U, nu, g, At, MU, 1, -1, 0, xpm);
-			B = nu == 3 ? lds_m3<R>(own, MU, sp)
-			            : load_disp<true>(U, MU, g, At, nu, 1, -1, 0, shift_c(g, x, nu, c[nu], 1));
+			A = MU == 3 ? lds_m3(own, nu, sp) : load_disp<ROWS>(U, nu, g, At, MU, 1, -1, 0, xpm);
+			B = nu == 3 ? lds_m3(own, MU, sp)
+			            : load_disp<ROWS>(U, MU, g, At, nu, 1, -1, 0, shift_c(g, x, nu, c[nu], 1));
 		}
 	};
 	// the upper and lower staples of plane (MU, nu); NEXT: the next nu (-1: none)
 	auto step = [&](auto NU, auto NEXT) {
 		constexpr int nu = decltype(NU)::value, nx = decltype(NEXT)::value;
 		const long xmn = nu == 3 ? 0 : shift_c(g, x, nu, c[nu], -1);
-		La = load_disp<true>(U, nu, g, At, MU, 1, nu, -1, shift_c(g, xpm, nu, c[nu], -1));
+		La = load_disp<ROWS>(U, nu, g, At, MU, 1, nu, -1, shift_c(g, xpm, nu, c[nu], -1));
 		__builtin_amdgcn_sched_barrier(0);
 		m3<R> T1;
 		if constexpr (plane_shared(SH, nu < MU ? nu : MU, nu < MU ? MU : nu))
-			T1 = nu < MU ? adj_m3(lds_m3<R>(sh, share_slot(SH, nu, MU), lane))
-			             : lds_m3<R>(sh, share_slot(SH, MU, nu), lane);
+			T1 = nu < MU ? adj_m3(lds_m3(sh, share_slot(SH, nu, MU), lane))
+			             : lds_m3(sh, share_slot(SH, MU, nu), lane);
 		else
 			T1 = upper_factor(A, B, nu < MU);
-		Lb = nu == 3 ? lds_m3<R>(own, MU, sm) : load_disp<true>(U, MU, g, At, nu, -1, -1, 0, xmn);
+		Lb = nu == 3 ? lds_m3(own, MU, sm) : load_disp<ROWS>(U, MU, g, At, nu, -1, -1, 0, xmn);
 		__builtin_amdgcn_sched_barrier(0);
-		madd_nd(S, T1, lds_m3<R>(own, nu, lane));
-		Lc = nu == 3 ? lds_m3<R>(own, nu, sm) : load_disp<true>(U, nu, g, At, nu, -1, -1, 0, xmn);
+		madd_nd(S, T1, lds_m3(own, nu, at.me));
+		Lc = nu == 3 ? lds_m3(own, nu, sm) : load_disp<ROWS>(U, nu, g, At, nu, -1, -1, 0, xmn);
 		__builtin_amdgcn_sched_barrier(0);
 		m3<R> T2 = mul_dd(La, Lb);
 		if constexpr (nx >= 0)
@@ -509,24 +472,6 @@ __device__ __forceinline__ m3<R> staple_rows_pipe(Geo const &g, const R *__restr
 	step(std::integral_constant<int, n1>{}, std::integral_constant<int, n2>{});
 	step(std::integral_constant<int, n2>{}, std::integral_constant<int, -1>{});
 	return S;
-}
-
-template <class R>
-__device__ __forceinline__ m3<R> staple_any(Geo const &g, const R *__restrict__ U, int mu, long x, int const *c)
-{
-	if (g.nd != 4)
-		return staple_at(g, U, mu, x, c);
-	switch (mu)
-	{
-	case 0:
-		return staple_4d<0>(g, U, x, c);
-	case 1:
-		return staple_4d<1>(g, U, x, c);
-	case 2:
-		return staple_4d<2>(g, U, x, c);
-	default:
-		return staple_4d<3>(g, U, x, c);
-	}
 }
 
 // Re tr of all plaquettes at x, in double
@@ -778,23 +723,30 @@ __device__ __forceinline__ void fused_link_step(Geo const &g, R *__restrict__ Un
 // since neighbouring threads still read U), and P is in the compact
 // antihermitian layout (the fused kernels run only inside a trajectory).
 // Staple paths of k_force_update, one per kernel (a kernel is compiled for
-// the registers of its largest path, and the general ones need more):
+// the registers of its largest path):
 //   STAPLE_ROWS  4-d, V % 64 == 0, L3 | 64, (L2 L3) % 64 == 0: the block's
-//                links staged in LDS,
-//                own and x3-neighbour links read there;
-//   STAPLE_OWN   4-d, V % 64 == 0: the block's links staged, own links read there;
-//   STAPLE_ANY   any geometry: every link from global memory.
+//                links staged in LDS, own and x3-neighbour links read there,
+//                the links displaced along x0, x1 and x3 addressed from the
+//                block's index;
+//   STAPLE_HALO  any other 4-d lattice: as above with the x3-neighbours outside
+//                the block staged beside it, and every other link addressed a
+//                lane at a time (where V % 64 == 0 against reading the
+//                x3-neighbours from global memory: 40^4 FP64 1853 -> 1716 us,
+//                FP32 1102 -> 1040 us; elsewhere against reading every link
+//                there and sharing no factor: 18 x 15 x 20 x 22 FP64 118 -> 79
+//                us, 10^4 FP32 24.9 -> 14.4 us);
+//   STAPLE_ANY   2-d and 3-d: every link from global memory.
 enum
 {
 	STAPLE_ANY = 0,
-	STAPLE_OWN = 1,
+	STAPLE_HALO = 1,
 	STAPLE_ROWS = 2
 };
 inline int staple_path(Geo const &g)
 {
-	if (!MESH_OWN_LDS || g.nd != 4 || (g.V & 63) != 0)
+	if (g.nd != 4)
 		return STAPLE_ANY;
-	return (MESH_OWN_ROWS && 64 % g.L[3] == 0 && (g.L[2] * g.L[3]) % 64 == 0) ? STAPLE_ROWS : STAPLE_OWN;
+	return ((g.V & 63) == 0 && 64 % g.L[3] == 0 && (g.L[2] * g.L[3]) % 64 == 0) ? STAPLE_ROWS : STAPLE_HALO;
 }
 
 template <class R, bool FUSE, bool PC, int PATH>
@@ -806,123 +758,83 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 	int lb = ordered_block(g, nb, SB, remap);
 	if (lb < 0)
 		return;
-	int mu = threadIdx.x >> 6;
-	long x = lane_site(g, (long)lb * SB + (threadIdx.x & 63));
+	const int mu = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	long x = lane_site(g, (long)lb * SB + lane);
 	m3<R> S, u;
 	if constexpr (PATH != STAPLE_ANY)
 	{
-		// every thread of the workgroup is a valid (site, direction): stage the
-		// block's own links, then the staples read them from LDS
-		__shared__ vec2_t<R> own[4][9][64];
-		const int lane = threadIdx.x & 63;
+		// stage the block's links, then the staples read them from LDS
+		constexpr bool RW = PATH == STAPLE_ROWS;
+		constexpr int SH = share_mode<R>(), NS = RW ? 64 : 68;
+		static_assert(SH > 0, "the staged kernels share the planes' upper factors");
+		__shared__ vec2_t<R> own[4][9][NS];
+		__shared__ vec2_t<R> sh[shared_planes(SH)][9][64];
+		const long b0 = (long)lb * SB;
+		const int n = RW || g.V - b0 >= SB ? SB : (int)(g.V - b0);
+		if (n < SB)
+			x = b0 + min(lane, n - 1); // the lanes past the last site repeat it and store nothing
 		int c[4];
 		coords<R>(g, x, c);
-		constexpr bool RW = PATH == STAPLE_ROWS; // the block holds whole x3-rows
-		constexpr int SH = share_mode<R>();
+		LaneSlots at;
+		if constexpr (RW)
+		{
+			at.me = lane;
+			x3_slots(g, x, c, at.sp, at.sm);
+		}
+		else
+			at = halo_slots(g.L[3], n, (int)(x - b0), c[3]);
 		ShareOps<R> F;
 		constexpr bool PF = std::is_same<R, float>::value ? MESH_SHARE_PREFETCH : MESH_SHARE_PREFETCH_F64;
-		if constexpr (SH > 0 && PF)
-			switch (mu)
-			{
-			case 0:
-				share_fetch<0, RW, SH>(g, U, x, c, F);
-				break;
-			case 1:
-				share_fetch<1, RW, SH>(g, U, x, c, F);
-				break;
-			case 2:
-				share_fetch<2, RW, SH>(g, U, x, c, F);
-				break;
-			default:
-				share_fetch<3, RW, SH>(g, U, x, c, F);
-				break;
-			}
+		constexpr bool PIPE = MESH_PIPE_F64 && std::is_same<R, double>::value;
+#define MESH_BY_DIRECTION(CALL)                                                                    \
+	switch (mu)                                                                                    \
+	{                                                                                              \
+	case 0:                                                                                        \
+		CALL(0);                                                                                   \
+		break;                                                                                     \
+	case 1:                                                                                        \
+		CALL(1);                                                                                   \
+		break;                                                                                     \
+	case 2:                                                                                        \
+		CALL(2);                                                                                   \
+		break;                                                                                     \
+	default:                                                                                       \
+		CALL(3);                                                                                   \
+		break;                                                                                     \
+	}
+#define MESH_FETCH(W) share_fetch<W, RW, SH>(g, U, x, c, F)
+#define MESH_SHARE(W) share_upper_factors<W, SH>(own, sh, at, lane, F)
+#define MESH_STAPLE(M)                                                                             \
+	S = PIPE ? staple_pipe<M, RW, SH>(g, U, x, c, own, at, lane, sh)                               \
+	         : staple_4d_own<M, RW, SH>(g, U, x, c, own, at, lane, sh)
+		if constexpr (PF)
+			MESH_BY_DIRECTION(MESH_FETCH)
 		{
 			const vec2_t<R> *p = reinterpret_cast<const vec2_t<R> *>(U) + site_off(g, mu, x);
 #pragma unroll
 			for (int k = 0; k < 9; ++k)
-				own[mu][k][lane] = p[k * plane_step(g)];
+				own[mu][k][at.me] = p[k * plane_step(g)];
 		}
+		if constexpr (!RW)
+			if (threadIdx.x < 4 * 4 * 9)
+			{
+				const int h = threadIdx.x & 3, d = (threadIdx.x >> 2) & 3, k = threadIdx.x >> 4;
+				own[d][k][64 + h] = reinterpret_cast<const vec2_t<R> *>(
+				    U)[site_off(g, d, halo_site(g.L[3], b0, n, h)) + k * plane_step(g)];
+			}
 		__syncthreads();
-		if constexpr (SH > 0)
-		{
-			// planes (0, q) are indices 0..2, so mode 1 needs three
-			__shared__ vec2_t<R> sh[shared_planes(SH)][9][64];
-			if constexpr (!PF)
-				switch (mu)
-				{
-				case 0:
-					share_fetch<0, RW, SH>(g, U, x, c, F);
-					break;
-				case 1:
-					share_fetch<1, RW, SH>(g, U, x, c, F);
-					break;
-				case 2:
-					share_fetch<2, RW, SH>(g, U, x, c, F);
-					break;
-				default:
-					share_fetch<3, RW, SH>(g, U, x, c, F);
-					break;
-				}
-			switch (mu)
-			{
-			case 0:
-				share_upper_factors<0, RW, SH>(g, x, c, own, sh, lane, F);
-				break;
-			case 1:
-				share_upper_factors<1, RW, SH>(g, x, c, own, sh, lane, F);
-				break;
-			case 2:
-				share_upper_factors<2, RW, SH>(g, x, c, own, sh, lane, F);
-				break;
-			default:
-				share_upper_factors<3, RW, SH>(g, x, c, own, sh, lane, F);
-				break;
-			}
-			__syncthreads();
-			constexpr bool PIPE = RW && MESH_PIPE_F64 && std::is_same<R, double>::value;
-			switch (mu)
-			{
-			case 0:
-				S = PIPE ? staple_rows_pipe<0, SH>(g, U, x, c, own, lane, sh)
-				         : staple_4d_own<0, RW, R, SH>(g, U, x, c, own, lane, sh);
-				break;
-			case 1:
-				S = PIPE ? staple_rows_pipe<1, SH>(g, U, x, c, own, lane, sh)
-				         : staple_4d_own<1, RW, R, SH>(g, U, x, c, own, lane, sh);
-				break;
-			case 2:
-				S = PIPE ? staple_rows_pipe<2, SH>(g, U, x, c, own, lane, sh)
-				         : staple_4d_own<2, RW, R, SH>(g, U, x, c, own, lane, sh);
-				break;
-			default:
-				S = PIPE ? staple_rows_pipe<3, SH>(g, U, x, c, own, lane, sh)
-				         : staple_4d_own<3, RW, R, SH>(g, U, x, c, own, lane, sh);
-				break;
-			}
-		}
-		else
-			switch (mu)
-			{
-			case 0:
-				S = staple_4d_own<0, RW>(g, U, x, c, own, lane);
-				break;
-			case 1:
-				S = staple_4d_own<1, RW>(g, U, x, c, own, lane);
-				break;
-			case 2:
-				S = staple_4d_own<2, RW>(g, U, x, c, own, lane);
-				break;
-			default:
-				S = staple_4d_own<3, RW>(g, U, x, c, own, lane);
-				break;
-			}
-#pragma unroll
-		for (int k = 0; k < 9; ++k)
-		{
-			vec2_t<R> v = own[mu][k][lane];
-			u.e[k] = {v.x, v.y};
-		}
+		if constexpr (!PF)
+			MESH_BY_DIRECTION(MESH_FETCH)
+		MESH_BY_DIRECTION(MESH_SHARE)
+		__syncthreads();
+		MESH_BY_DIRECTION(MESH_STAPLE)
+#undef MESH_FETCH
+#undef MESH_SHARE
+#undef MESH_STAPLE
+#undef MESH_BY_DIRECTION
+		u = lds_m3(own, mu, at.me);
+		if (n < SB && lane >= n)
+			return;
 	}
 	else
 	{
@@ -930,7 +842,7 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 			return;
 		int c[4];
 		coords<R>(g, x, c);
-		S = MESH_STATIC_MU ? staple_any(g, U, mu, x, c) : staple_at(g, U, mu, x, c);
+		S = staple_at(g, U, mu, x, c);
 		u = load(U, mu, g, x);
 	}
 	m3<R> p = mom_step<PC>(load_mom<PC>(P, mu, g, x), mul_nn(u, S), kc);
@@ -1360,8 +1272,8 @@ int launch_force_update(mesh_ctx *ctx, Geo const &geo, int prec, const void *U, 
 			case STAPLE_ROWS:
 				launch(tag, std::integral_constant<int, STAPLE_ROWS>{});
 				break;
-			case STAPLE_OWN:
-				launch(tag, std::integral_constant<int, STAPLE_OWN>{});
+			case STAPLE_HALO:
+				launch(tag, std::integral_constant<int, STAPLE_HALO>{});
 				break;
 			default:
 				launch(tag, std::integral_constant<int, STAPLE_ANY>{});

@@ -163,6 +163,25 @@ def test_fused_trajectory_own_path_bitexact(ctx, shape, prec):
         np.testing.assert_array_equal(hmc.U.download(), U)
 
 
+@pytest.mark.parametrize("prec", [F64, F32])
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (2, 2, 3, 3), (3, 2, 4, 5), (3, 5, 2, 7), (2, 2, 3, 22), (2, 3, 2, 66),
+                                   (2, 2, 2, 100), (3, 3, 3, 43), (2, 2, 2, 130)])
+def test_fused_trajectory_halo_bitexact(ctx, shape, prec):
+    """the staged kernel on 4-d lattices whose blocks start and end inside
+    x3-rows: one partly filled block, a last block of 16 .. 56 sites, rows
+    within a block and rows longer than one -- the oracle's bits"""
+    shape = list(shape)
+    hmc = gauge.Hmc(mesh_amd.Grid(shape), prec, seed=9, ctx=ctx)
+    hmc.randomizeGaugeField()
+    U = O.random_gauge(shape, 9, _pname(prec))
+    deltas = gauge.makeDeltas("2mn", 0.4, 2)
+    for traj in range(2):
+        r = hmc.runHmcUpdate(5.5, deltas, metropolis=bool(traj))
+        o = O.hmc_trajectory(U, shape, 5.5, deltas, 9, traj, metropolis=bool(traj))
+        assert r["accepted"] == o["accepted"]
+        np.testing.assert_array_equal(hmc.U.download(), U)
+
+
 @pytest.mark.parametrize("order", [3, 4])
 @pytest.mark.parametrize("tile", [1, 2, 4])
 @pytest.mark.parametrize("variant", [0, 2])
