@@ -145,25 +145,49 @@ __device__ __forceinline__ int logical_block(int nb, int remap)
 //      range of row-blocks and, within it, x0 fastest then x1, so the
 //      x0-neighbours of a workgroup were staged by the previous one and the
 //      x1-neighbours L0 workgroups earlier, all in the same L2;
-//   3: slab order for 4-d lattices with 8 | L0 and T | (L2*L3/sbk) -- XCD k
-//      owns the slab x0 in [k L0/8, (k+1) L0/8) and walks it x0 fastest, then
-//      T row-blocks, then x1, then the next tile of T row-blocks, so the x1-
-//      and rb-neighbours of a workgroup are at most (L0/8) T workgroups back
-//      and only the two x0 faces of the slab come from another XCD;
+//   3: slab order for 4-d lattices with 8 | L0 -- XCD k owns the slab x0 in
+//      [k L0/8, (k+1) L0/8) and walks it x0 fastest, then a tile of T
+//      row-blocks, then x1, then the next tile, so the x1- and rb-neighbours of
+//      a workgroup are at most (L0/8) T workgroups back and only the two x0
+//      faces of the slab come from another XCD; T: tile_of(the argument's);
 //   4: as 3 with XCD k owning x0 in a quarter (k % 4) and x1 in a half (k / 4)
 //      of the lattice (4 | L0, 2 | L1); also order 3's fallback where 8 does
 //      not divide L0.
+// Where a plane is no whole number of blocks, or the extents allow neither,
+// orders 3 and 4 give XCD k the k-th eighth of the blocks in memory order, about
+// L0/8 slices of x0, walked side by side (slice fastest, then the position in
+// the slice), so the x0-neighbours of a workgroup are the launches before and
+// after it, to within a block -- if a slice has more than 128 blocks: below
+// that an XCD has the x0-neighbours in flight in memory order as well
+// (18x15x20x22, 103 blocks: 83 us a fused step in memory order, 85 so; 36^4,
+// 729 blocks: 1109 and 1053 us; 44^4 2536 and 2344; 40^4, whose planes of 25
+// blocks take tiles of 5 in order 3, 1740 and 1485).
 // Returns the memory-order block index (-1: padding workgroup).  The order
 // only permutes workgroups; every site's arithmetic is unchanged.  GEO: any
 // geometry with nd and L[4] (the SU(3) and SU(2) ones).
-template <class GEO> __device__ __forceinline__ int ordered_block_of(GEO const &g, int nb, int sbk, int arg, int b)
+// the row-blocks of a tile of orders 3 and 4: the divisor of nb2 (row-blocks of
+// a plane) nearest below or just above the one asked for
+__host__ __device__ __forceinline__ int tile_of(int nb2, int t)
 {
-	const int order = arg & 15, T = arg >> 4;
+	if (nb2 % t == 0)
+		return t;
+	if (nb2 % (t + 1) == 0)
+		return t + 1;
+	while (nb2 % t)
+		--t;
+	return t;
+}
+
+template <class GEO>
+__host__ __device__ __forceinline__ int ordered_block_of(GEO const &g, int nb, int sbk, int arg, int b)
+{
+	const int order = arg & 15;
 	if (order == 0)
 		return b < nb ? b : -1;
 	const bool planes = g.nd == 4 && (g.L[2] * g.L[3]) % sbk == 0;
 	const int nb2 = planes ? (g.L[2] * g.L[3]) / sbk : 1;
-	if (order == 3 && planes && (g.L[0] & 7) == 0 && T > 0 && nb2 % T == 0)
+	const int T = order >= 3 ? tile_of(nb2, (arg >> 4) > 0 ? arg >> 4 : 1) : 1;
+	if (order == 3 && planes && (g.L[0] & 7) == 0)
 	{
 		const int X = g.L[0] >> 3;
 		const int j = b >> 3;
@@ -177,8 +201,7 @@ template <class GEO> __device__ __forceinline__ int ordered_block_of(GEO const &
 		rb += (t / g.L[1]) * T;
 		return (x0 * g.L[1] + x1) * nb2 + rb;
 	}
-	if ((order == 4 || order == 3) && planes && (g.L[0] & 3) == 0 && (g.L[1] & 1) == 0 && T > 0 &&
-	    nb2 % T == 0)
+	if ((order == 4 || order == 3) && planes && (g.L[0] & 3) == 0 && (g.L[1] & 1) == 0)
 	{
 		// XCD k owns x0 in a quarter (k % 4) and x1 in a half (k / 4) of the
 		// lattice, walked as in order 3 (and order 3's fallback where 8 does
@@ -199,6 +222,20 @@ template <class GEO> __device__ __forceinline__ int ordered_block_of(GEO const &
 	int o = (b & 7) * chunk + (b >> 3);
 	if (o >= nb)
 		return -1;
+	if (order >= 3 && g.nd == 4)
+	{
+		// this XCD's C blocks as slices of S: R positions have w + 1 of them,
+		// the others w
+		const int first = (b & 7) * chunk, C = nb - first < chunk ? nb - first : chunk;
+		const int S = nb / g.L[0], w = S > 128 ? C / S : 0;
+		if (w == 0)
+			return o;
+		const int R = C - w * S, j = b >> 3;
+		if (j < R * (w + 1))
+			return first + (j % (w + 1)) * S + j / (w + 1);
+		const int i = j - R * (w + 1);
+		return first + (i % w) * S + R + i / w;
+	}
 	if (order == 1 || !planes)
 		return o;
 	int x0 = o % g.L[0];

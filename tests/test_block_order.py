@@ -1,0 +1,21 @@
+"""The block orders of the stencil kernels (mesh_internal.h ordered_block_of):
+each is a permutation of the blocks on every geometry it accepts.  Host only:
+the check is compiled with hipcc for the host."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not found")
+def test_block_order(tmp_path):
+    exe = str(tmp_path / "block_order")
+    subprocess.run([HIPCC, "-O2", "-std=c++17", "--offload-arch=gfx950",
+                    os.path.join(ROOT, "tests", "block_order.cpp"), "-o", exe],
+                   check=True, capture_output=True, timeout=300)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert " 0 wrong" in r.stdout
