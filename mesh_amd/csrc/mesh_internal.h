@@ -32,12 +32,12 @@ struct mesh_ctx
 	int device;
 	hipStream_t stream;
 	std::string err;
-	// reduction scratch: per-block partial sums (device) and the final
-	// values (device + pinned host)
+	// reduction scratch: per-block partial sums (device) and the final values
+	// (pinned host memory, and its address for the device)
 	double *partials = nullptr;
 	size_t partials_cap = 0; // doubles
-	double *red_dev = nullptr;
 	double *red_host = nullptr;
+	double *red_out = nullptr;
 	double *aux = nullptr; // small device buffer (integrator step tables)
 	size_t aux_cap = 0;    // doubles
 	std::vector<double> aux_host; // host copy of what aux holds

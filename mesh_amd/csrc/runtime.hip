@@ -110,19 +110,26 @@ int mesh_stage_doubles(mesh_ctx *ctx, const double *host, size_t n)
 	return MESH_OK;
 }
 
-// second reduction pass: one workgroup, fixed summation order
-template <int NQ> __global__ __launch_bounds__(1024) void k_reduce_partials(const double *p, int nb, double *out)
+// second reduction pass: a workgroup a quantity, in a fixed summation order
+__global__ __launch_bounds__(1024) void k_reduce_partials(const double *__restrict__ p, int nb, double *out)
 {
-	double v[NQ];
-#pragma unroll
-	for (int q = 0; q < NQ; ++q)
+	constexpr int AHEAD = 4; // loads in flight a thread, added in order
+	const double *q = p + (long)blockIdx.x * nb;
+	double v[1] = {0.0};
+	int i = threadIdx.x;
+	for (; i + (AHEAD - 1) * 1024 < nb; i += AHEAD * 1024)
 	{
-		double s = 0.0;
-		for (int i = threadIdx.x; i < nb; i += blockDim.x)
-			s += p[(long)q * nb + i];
-		v[q] = s;
+		double t[AHEAD];
+#pragma unroll
+		for (int k = 0; k < AHEAD; ++k)
+			t[k] = q[i + k * 1024];
+#pragma unroll
+		for (int k = 0; k < AHEAD; ++k)
+			v[0] += t[k];
 	}
-	block_sum_store<NQ>(v, out, 1, 0);
+	for (; i < nb; i += 1024)
+		v[0] += q[i];
+	block_sum_store<1>(v, out + blockIdx.x, 1, 0);
 }
 
 static const char *const PROF_NAMES[PROF_NKINDS] = {"force_update", "link_update", "delta_h",   "momenta",
@@ -175,25 +182,11 @@ void mesh_prof_collect(mesh_ctx *ctx)
 
 int mesh_finish_reduction(mesh_ctx *ctx, int nb, int nq, double *out)
 {
-	double *p = ctx->partials, *o = ctx->red_dev;
-	hipStream_t st = ctx->stream;
-	switch (nq)
-	{
-	case 1: k_reduce_partials<1><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 2: k_reduce_partials<2><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 3: k_reduce_partials<3><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 4: k_reduce_partials<4><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 5: k_reduce_partials<5><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 6: k_reduce_partials<6><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 7: k_reduce_partials<7><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 8: k_reduce_partials<8><<<1, 1024, 0, st>>>(p, nb, o); break;
-	case 18: k_reduce_partials<18><<<1, 1024, 0, st>>>(p, nb, o); break;
-	default:
+	if (nq < 1 || nq > RED_MAX_Q)
 		return mesh_fail(ctx, MESH_E_ARG, "unsupported reduction width");
-	}
+	// the sums go to pinned host memory: no copy behind the kernel
+	k_reduce_partials<<<nq, 1024, 0, ctx->stream>>>(ctx->partials, nb, ctx->red_out);
 	MESH_LAUNCHED(ctx);
-	MESH_HIP(ctx, hipMemcpyAsync(ctx->red_host, ctx->red_dev, nq * sizeof(double), hipMemcpyDeviceToHost,
-	                             ctx->stream));
 	MESH_HIP(ctx, hipStreamSynchronize(ctx->stream));
 	mesh_prof_collect(ctx);
 	for (int q = 0; q < nq; ++q)
@@ -203,7 +196,7 @@ int mesh_finish_reduction(mesh_ctx *ctx, int nb, int nq, double *out)
 
 int mesh_reduce_to_device(mesh_ctx *ctx, const double *partials, int nb, double *out_dev)
 {
-	k_reduce_partials<1><<<1, 1024, 0, ctx->stream>>>(partials, nb, out_dev);
+	k_reduce_partials<<<1, 1024, 0, ctx->stream>>>(partials, nb, out_dev);
 	MESH_LAUNCHED(ctx);
 	return MESH_OK;
 }
@@ -232,8 +225,8 @@ int mesh_ctx_create(mesh_ctx **out, int device)
 		delete ctx;
 		return MESH_E_HIP;
 	}
-	if (hipMalloc(&ctx->red_dev, RED_MAX_Q * sizeof(double)) != hipSuccess ||
-	    hipHostMalloc(&ctx->red_host, RED_MAX_Q * sizeof(double), hipHostMallocDefault) != hipSuccess)
+	if (hipHostMalloc(&ctx->red_host, RED_MAX_Q * sizeof(double), hipHostMallocMapped) != hipSuccess ||
+	    hipHostGetDevicePointer((void **)&ctx->red_out, ctx->red_host, 0) != hipSuccess)
 	{
 		(void)hipStreamDestroy(ctx->stream);
 		delete ctx;
@@ -241,7 +234,6 @@ int mesh_ctx_create(mesh_ctx **out, int device)
 	}
 	if (mesh_scratch_setup(ctx) != MESH_OK)
 	{
-		(void)hipFree(ctx->red_dev);
 		(void)hipHostFree(ctx->red_host);
 		(void)hipStreamDestroy(ctx->stream);
 		delete ctx;
@@ -266,7 +258,6 @@ int mesh_ctx_destroy(mesh_ctx *ctx)
 		(void)hipFree(ctx->md_spare);
 	if (ctx->u1_ws)
 		(void)hipFree(ctx->u1_ws);
-	(void)hipFree(ctx->red_dev);
 	(void)hipHostFree(ctx->red_host);
 	(void)hipStreamDestroy(ctx->stream);
 	ctx->magic = 0;

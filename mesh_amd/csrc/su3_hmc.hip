@@ -99,6 +99,11 @@ __host__ __device__ constexpr bool plane_shared(int m, int p, int q)
 // number of shared planes in mode m
 __host__ __device__ constexpr int shared_planes(int m) { return m == 2 ? 6 : (m == 3 ? 4 : 3); }
 
+// largest volume whose Delta H takes a plane a wavefront (k_delta_h_planes): a
+// workgroup of 64 sites a CU.  10^4 23.3 -> 15.4 us, 8 x 8 x 16 x 16 21.6 ->
+// 15.3; 12^4, where CUs get two, 21.3 -> 26.1
+constexpr long DH_PLANES_V = 64 * 256;
+
 // non-temporal hints on the once-touched fields of the force kernels
 #ifndef MESH_STREAM_HINTS
 #define MESH_STREAM_HINTS 1
@@ -474,6 +479,16 @@ __device__ __forceinline__ m3<R> staple_pipe(Geo const &g, const R *__restrict__
 	return S;
 }
 
+// Re tr of the plaquette of plane (mu, nu) at x, in double
+template <class R>
+__device__ __forceinline__ double plaq_plane(Geo const &g, const R *__restrict__ U, long x, int const *c, int mu, int nu)
+{
+	const long xpm = shift_c(g, x, mu, c[mu], 1), xpn = shift_c(g, x, nu, c[nu], 1);
+	const m3<double> A = mul_nn(to_f64(load(U, mu, g, x)), to_f64(load(U, nu, g, xpm)));
+	const m3<double> B = mul_nn(to_f64(load(U, nu, g, x)), to_f64(load(U, mu, g, xpn)));
+	return retr_nd(A, B);
+}
+
 // Re tr of all plaquettes at x, in double
 template <class R> __device__ __forceinline__ double plaq_site(Geo const &g, const R *__restrict__ U, long x,
                                                              int const *c)
@@ -486,10 +501,7 @@ template <class R> __device__ __forceinline__ double plaq_site(Geo const &g, con
 		{
 			if (nu >= g.nd)
 				continue;
-			long xpm = shift_c(g, x, mu, c[mu], 1), xpn = shift_c(g, x, nu, c[nu], 1);
-			m3<double> A = mul_nn(to_f64(load(U, mu, g, x)), to_f64(load(U, nu, g, xpm)));
-			m3<double> B = mul_nn(to_f64(load(U, nu, g, x)), to_f64(load(U, mu, g, xpn)));
-			s += retr_nd(A, B);
+			s += plaq_plane(g, U, x, c, mu, nu);
 		}
 	return s;
 }
@@ -539,23 +551,25 @@ template <class R> __global__ __launch_bounds__(256) void k_momenta(Geo g, R *P,
 // momenta refresh fused with the first link step of the trajectory:
 // P_mu(x) drawn as in k_momenta, then Uout_mu(x) = exp(t TA(P_mu(x))) Uin_mu(x)
 // as in k_link_update (the same operations, so the same bits); PC: P in the
-// compact antihermitian layout
+// compact antihermitian layout.  A workgroup takes 64 sites, wavefront mu their
+// direction mu; k(x) adds the directions in order.  (A thread a site over the
+// four directions left 8^4 16 workgroups: 19 -> 12 us; 32^4 FP32 155 -> 142 us,
+// FP64 267 -> 254.)
 template <class R, bool PC>
 __global__ __launch_bounds__(256) void k_momenta_link(Geo g, R *__restrict__ P, double *__restrict__ K, uint64_t seed,
                                                       uint32_t traj, R *__restrict__ Uout, const R *__restrict__ Uin,
                                                       R t, int reunit_flag)
 {
-	long x = lane_site(g, (long)blockIdx.x * blockDim.x + threadIdx.x);
-	if (x >= g.V)
-		return;
-	double k = 0.0;
-	for (int mu = 0; mu < g.nd; ++mu)
+	__shared__ double kn[4][64];
+	const int mu = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	const long x = lane_site(g, (long)blockIdx.x * 64 + lane);
+	if (mu < g.nd && x < g.V)
 	{
 		double z[8];
 		link_normals<8>(seed, TAG_MOM, traj, (uint32_t)x, (uint32_t)mu, z);
 		m3<R> p = from_f64<R>(algebra_from_normals(z));
 		store_mom<PC>(P, mu, g, x, p);
-		k += norm2_m3(to_f64(p));
+		kn[mu][lane] = norm2_m3(to_f64(p));
 		m3<R> X = ta(p);
 #pragma unroll
 		for (int e = 0; e < 9; ++e)
@@ -568,7 +582,14 @@ __global__ __launch_bounds__(256) void k_momenta_link(Geo g, R *__restrict__ P, 
 			u = reunit(u);
 		store_once(Uout, mu, g, x, u);
 	}
-	K[x] = k;
+	__syncthreads();
+	if (mu == 0 && x < g.V)
+	{
+		double k = 0.0;
+		for (int m = 0; m < g.nd; ++m)
+			k += kn[m][lane];
+		K[x] = k;
+	}
 }
 
 template <class R>
@@ -667,6 +688,54 @@ __global__ __launch_bounds__(256) void k_delta_h_split(Geo g, const R *__restric
 			v[1] = ps;
 	}
 	block_sum_store<5>(v, partials, nb, lb);
+}
+
+// The same for lattices that leave the chip idle: a workgroup takes 64 sites
+// and a wavefront one plane of one field (waves 0-5 U_old, 6-11 U_new; the
+// first nd also one direction's kinetic energy), and the first wavefront adds
+// them in the order of plaq_site and kin_site: the same per-site values.
+template <class R, bool PC>
+__global__ __launch_bounds__(768) void k_delta_h_planes(Geo g, const R *__restrict__ Uo, const R *__restrict__ Un,
+                                                        const R *__restrict__ P, const double *__restrict__ Ko,
+                                                        double c3, double *partials, int nb)
+{
+	__shared__ double ps[12][64], kn[4][64];
+	const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	const long x = lane_site(g, (long)blockIdx.x * 64 + lane);
+	const int planes = g.nd * (g.nd - 1) / 2;
+	if (x < g.V)
+	{
+		int c[4];
+		coords<R>(g, x, c);
+		if (w < g.nd)
+			kn[w][lane] = norm2_m3(to_f64(PC ? load_alg<R, false>(P, w, g, x) : load(P, w, g, x)));
+		const int q = w % 6;
+		if (q < planes)
+		{
+			int mu = 0, k = q;
+			while (k >= g.nd - 1 - mu)
+				k -= g.nd - 1 - mu++;
+			const int nu = mu + 1 + k;
+			ps[w][lane] = plaq_plane(g, w < 6 ? Uo : Un, x, c, mu, nu);
+		}
+	}
+	__syncthreads();
+	double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+	if (w == 0 && x < g.V)
+	{
+		double pso = 0.0, psn = 0.0, k = 0.0;
+		for (int q = 0; q < planes; ++q)
+			pso += ps[q][lane], psn += ps[6 + q][lane];
+		for (int mu = 0; mu < g.nd; ++mu)
+			k += kn[mu][lane];
+		const double dps = psn - pso, dk = k - Ko[x];
+		v[0] = fma(-c3, dps, dk);
+		v[1] = pso;
+		v[2] = psn;
+		v[3] = k;
+		v[4] = Ko[x];
+	}
+	block_sum_store<5>(v, partials, nb, blockIdx.x);
 }
 
 template <class R>
@@ -1325,7 +1394,7 @@ int launch_momenta(mesh_ctx *ctx, Geo const &geo, int prec, void *P, double *K, 
 int launch_momenta_link(mesh_ctx *ctx, Geo const &geo, int prec, void *P, double *K, uint64_t seed, uint32_t traj,
                         void *Uout, const void *Uin, double t, int reunit_flag, bool compact)
 {
-	int nb = nblk(geo.V, 256);
+	int nb = nblk(geo.V, 64);
 	int ph = mesh_prof_begin(ctx, PROF_MOMENTA_LINK);
 	auto launch = [&](auto tag, auto pc) {
 		using Rt = decltype(tag);
@@ -1395,7 +1464,8 @@ int float_energy(mesh_ctx *ctx, Geo const &geo, const float *U, const float *P, 
 int delta_h(mesh_ctx *ctx, Geo const &geo, int prec, const void *Uo, const void *Un, const void *P, const double *Ko,
             double beta, double *out, bool compact = false)
 {
-	const int sbk = MESH_DH_SPLIT ? 128 : 256; // sites per workgroup
+	const bool by_plane = geo.V <= DH_PLANES_V;
+	const int sbk = by_plane ? 64 : (MESH_DH_SPLIT ? 128 : 256); // sites per workgroup
 	int nb = nblk(geo.V, sbk);
 	if (int rc = mesh_reserve_partials(ctx, 5 * (size_t)nb))
 		return rc;
@@ -1404,7 +1474,10 @@ int delta_h(mesh_ctx *ctx, Geo const &geo, int prec, const void *Uo, const void 
 	int ph = mesh_prof_begin(ctx, PROF_DELTA_H);
 	auto launch = [&](auto tag, auto pc) {
 		using Rt = decltype(tag);
-		if (MESH_DH_SPLIT)
+		if (by_plane)
+			k_delta_h_planes<Rt, decltype(pc)::value><<<nb, 768, 0, ctx->stream>>>(
+			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb);
+		else if (MESH_DH_SPLIT)
 			k_delta_h_split<Rt, decltype(pc)::value><<<gb, 256, 0, ctx->stream>>>(
 			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb, mesh_order(ctx));
 		else
