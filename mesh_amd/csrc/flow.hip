@@ -144,7 +144,7 @@ __device__ __forceinline__ void layer_apply(FGeo const &g, float *th, int mu, in
 		float x[NI / 4];
 		features(g, th, mu, a, min(tix * 16 + (l & 15), g.NA - 1), x);
 		f4 h1[4], h2[4];
-		put_outputs(y, mlp_rows<NI, false, true>(sh.lw, x, [&](int s) { return feature_row(q, s); }, h1, h2));
+		put_outputs(y, mlp_rows<NI, false>(sh.lw, x, [&](int s) { return feature_row(q, s); }, h1, h2));
 		wave_sync();
 		const int r = tix * 16 + (l >> 2);
 		if (r < g.NA)
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(THREADS) void k_flow_backward(FGeo g, int nl, const
 			float x[NI / 4], *y = sh.buf.y[w];
 			features(g, th, mu, a, min(r, g.NA - 1), x);
 			f4 h1[4], h2[4], dxr[GradP<NI>::NB];
-			put_outputs(y, mlp_rows<NI, false, true>(sh.lw, x, [&](int s) { return feature_row(l >> 4, s); }, h1, h2));
+			put_outputs(y, mlp_rows<NI, false>(sh.lw, x, [&](int s) { return feature_row(l >> 4, s); }, h1, h2));
 			wave_sync();
 			{
 				// the updated link moves by g(u) + t - theta_P, so its adjoint A

@@ -59,8 +59,8 @@ __device__ __forceinline__ float wrapf(float a)
 // 1e-7, saturating to +-1 (e = inf or 0)
 __device__ __forceinline__ float tanh_fast(float x)
 {
-	const float e = __expf(2.f * x);
-	return 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + e);
+	const float e = __builtin_amdgcn_exp2f(x * 2.88539008177792681f); // exp(2 x)
+	return fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f);
 }
 
 template <bool FAST> __device__ __forceinline__ float act(float x) { return FAST ? tanh_fast(x) : tanhf(x); }
@@ -165,12 +165,11 @@ template <bool FAST> __device__ __forceinline__ f4 act4(f4 a)
 // h1[b][j], h2[b][j]: hidden columns 16 b + 4 (l / 16) + j; the return value:
 // outputs 4 (l / 16) + j.
 //
-// AHEAD (kernels with one wavefront a SIMD): the weights come a chunk of 16
-// ahead of their products; the scheduling barriers keep the loads there, which
-// left alone are placed two products before their use, so that each pair of
-// products waits out the LDS.  16^2 sample, 256 chains: 47.2 -> 43.7 us; with
-// more wavefronts its registers cost more (32^2 propose 210 -> 228 us).
-template <int NI, bool FAST, bool AHEAD, class ROW>
+// The weights come a chunk of 16 ahead of their products; the scheduling
+// barriers keep the loads there, which left alone are placed two products before
+// their use, so that each pair of products waits out the LDS (plaquette flow,
+// 16^2 sample, 256 chains: 47.2 -> 43.7 us).
+template <int NI, bool FAST, class ROW>
 __device__ __forceinline__ f4 mlp_rows(LWP<NI> const &lw, const float (&x)[NI / 4], ROW row, f4 (&h1)[4], f4 (&h2)[4])
 {
 	constexpr int NS = NI / 4, C1 = (NS + 3) / 4; // steps and chunks of the first layer
@@ -206,17 +205,13 @@ __device__ __forceinline__ f4 mlp_rows(LWP<NI> const &lw, const float (&x)[NI / 
 	}
 	// two chains: the products of one block of columns are each other's input
 	f4 y0 = *reinterpret_cast<const f4 *>(lw.b3 + q4), y1 = {0.f, 0.f, 0.f, 0.f};
-	if (AHEAD)
-		load(0, w[0]);
+	load(0, w[0]);
 #pragma unroll
 	for (int c = 0; c < C1 + 5; ++c)
 	{
-		if (!AHEAD)
-			load(c, w[c & 1]);
-		else if (c < C1 + 4)
+		if (c < C1 + 4)
 			load(c + 1, w[(c + 1) & 1]);
-		if (AHEAD)
-			__builtin_amdgcn_sched_barrier(0);
+		__builtin_amdgcn_sched_barrier(0);
 		float (&d)[16] = w[c & 1];
 		const int k = c - C1;
 		if (k < 0)
@@ -263,6 +258,226 @@ __device__ __forceinline__ f4 mlp_rows(LWP<NI> const &lw, const float (&x)[NI / 
 		}
 	}
 	return y0 + y1;
+}
+
+// ---- the same products on the BF16 matrix units, to FP32's precision ------
+//
+// FP32 MFMA runs on the vector ALUs (the chip's FP32 rate is the same either
+// way), so a tile's products and its activations, feature sums and circle maps
+// add up; BF16 MFMA has units of its own.  A float is the sum of three BF16
+// numbers, each the rounding of what the ones before it leave (8 + 8 + 8 bits
+// with signs hold all 24), and of the nine products of two such sums the six
+// that reach FP32's rounding are formed and accumulated in FP32: the three
+// left out are below 2^-24 of the product.  Against 64 bits, 32 seeds of 64
+// chains: links of a 32^2 proposal 7.2e-7 on FP32 MFMA, 7.2e-7 here, its log q
+// 2.9e-9 and 3.3e-9 (1.4e-8 with layers and tails in separate passes).
+// 32^2 propose, 256 chains: 209 -> 159 us; 64^2: 872 -> 615.
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// v[e] = p[0][e] + p[1][e] + p[2][e], two BF16 numbers a word
+template <int N> struct Split
+{
+	typedef __bf16 vec __attribute__((ext_vector_type(N)));
+	typedef uint32_t words __attribute__((ext_vector_type(N / 2)));
+	words p[3];
+	__device__ __forceinline__ vec part(int k) const { return __builtin_bit_cast(vec, p[k]); }
+};
+// a, b rounded to BF16 in the halves of a word (one instruction), and what it leaves of them
+__device__ __forceinline__ uint32_t take_bf16(float &a, float &b)
+{
+	typedef __bf16 pair __attribute__((ext_vector_type(2)));
+	const uint32_t w = __builtin_bit_cast(uint32_t, pair{(__bf16)a, (__bf16)b});
+	a -= __uint_as_float(w << 16);
+	b -= __uint_as_float(w & 0xffff0000u);
+	return w;
+}
+template <int N> __device__ __forceinline__ Split<N> split(const float (&v)[N])
+{
+	Split<N> s;
+#pragma unroll
+	for (int e = 0; e < N; e += 2)
+	{
+		float a = v[e], b = v[e + 1];
+#pragma unroll
+		for (int k = 0; k < 3; ++k)
+			s.p[k][e / 2] = take_bf16(a, b);
+	}
+	return s;
+}
+
+// LDS image of one layer's weights as the MFMA's A operands: lane l = 16 q + i
+// of step t, column block b holds in element e the parts of the weight of
+// output column 16 b + i and contraction index (t, q, e) -- for W2 and W3
+// column 16 (2t + e / 4) + 4 q + e % 4 of the layer before, for W1 the quarter's
+// feature row(q, 8 t + e); the features past the last eight are a step of four
+template <int NI> struct alignas(16) LWS
+{
+	static constexpr int T8 = NI / 4 / 8, R4 = (NI / 4) % 8;
+	static_assert(R4 <= 4, "the last features fill a step of four");
+	bf8 w1[T8 ? T8 : 1][4][3][64];
+	Split<4>::vec w1r[R4 ? 4 : 1][3][64];
+	bf8 w2[2][4][3][64], w3[2][3][64];
+	float b1[NH], b2[NH], b3[16];
+};
+
+// One layer's parameters in registers, the floats of a thread's operand
+// fragments, so that the next layer's global loads overlap the current layer's
+// work; store() splits them into the LDS image.
+template <int NI, int THREADS, class ROW> struct WeightFrags
+{
+	using Y = Layout<NI>;
+	using W = LWS<NI>;
+	static constexpr int N2 = 512 / THREADS; // fragments of W2 a thread
+	static_assert(W::T8 == 1 && W::R4 > 0 && (THREADS == 256 || THREADS == 512), "one step of eight features and a rest");
+	float w1[8], w1r[4], w2[N2][8], w3[8] = {}, b[1] = {}; // (zero past column NO)
+
+	// a fragment's block b (of W1: 0..3) and lane
+	static __device__ __forceinline__ bool has_w1() { return threadIdx.x < 256; }
+	static __device__ __forceinline__ bool has_w1r() { return THREADS == 256 || threadIdx.x >= 256; }
+	static __device__ __forceinline__ bool has_w3() { return threadIdx.x < 128; }
+
+	// (unsigned offsets from the uniform p: one register an address)
+	__device__ __forceinline__ void load(const float *__restrict__ p)
+	{
+		const unsigned l = threadIdx.x & 63, i = l & 15, q = l >> 4, f = (threadIdx.x >> 6) & 3;
+		if (has_w1())
+#pragma unroll
+			for (int e = 0; e < 8; ++e)
+				w1[e] = p[Y::OW1 + (unsigned)ROW::row(q, e) * NH + 16 * f + i];
+		if (has_w1r())
+#pragma unroll
+			for (int e = 0; e < 4; ++e)
+				w1r[e] = e < W::R4 ? p[Y::OW1 + (unsigned)ROW::row(q, 8 * W::T8 + (e < W::R4 ? e : 0)) * NH + 16 * f + i] : 0.f;
+#pragma unroll
+		for (int k = 0; k < N2; ++k)
+		{
+			const unsigned u = (threadIdx.x >> 6) + k * (THREADS / 64), o = (32 * (u >> 2) + 4 * q) * NH + 16 * (u & 3) + i;
+#pragma unroll
+			for (int e = 0; e < 8; ++e)
+				w2[k][e] = p[Y::OW2 + o + (16 * (e / 4) + e % 4) * NH];
+		}
+		if (has_w3() && i < NO)
+		{
+			const unsigned o = (32 * (threadIdx.x >> 6) + 4 * q) * NO + i;
+#pragma unroll
+			for (int e = 0; e < 8; ++e)
+				w3[e] = p[Y::OW3 + o + (16 * (e / 4) + e % 4) * NO];
+		}
+		// the biases: b1, b2, b3 by the first 138 threads
+		const unsigned x = threadIdx.x;
+		if (x < 2 * NH + NO)
+			b[0] = p[x < NH ? Y::OB1 + x : (x < 2 * NH ? Y::OB2 + x - NH : Y::OB3 + x - 2 * NH)];
+	}
+
+	// infinite weights as the largest BF16 number: a part of an activation may
+	// be 0, and 0 times infinity would not be what the activation times it is
+	static __device__ __forceinline__ float finite(float v)
+	{
+		return fabsf(v) > 3.38953139e38f ? copysignf(3.38953139e38f, v) : v;
+	}
+	template <int N, class DST> static __device__ __forceinline__ void put(const float (&v)[N], DST *dst, int l)
+	{
+		float w[N];
+#pragma unroll
+		for (int e = 0; e < N; ++e)
+			w[e] = finite(v[e]);
+		const Split<N> s = split<N>(w);
+#pragma unroll
+		for (int k = 0; k < 3; ++k)
+			dst[k][l] = s.part(k);
+	}
+	__device__ __forceinline__ void store(W &lw) const
+	{
+		const int l = threadIdx.x & 63, f = (threadIdx.x >> 6) & 3;
+		if (has_w1())
+			put<8>(w1, lw.w1[0][f], l);
+		if (has_w1r())
+			put<4>(w1r, lw.w1r[f], l);
+#pragma unroll
+		for (int k = 0; k < N2; ++k)
+		{
+			const int u = (threadIdx.x >> 6) + k * (THREADS / 64);
+			put<8>(w2[k], lw.w2[u >> 2][u & 3], l);
+		}
+		if (has_w3())
+			put<8>(w3, lw.w3[threadIdx.x >> 6], l);
+		const int x = threadIdx.x;
+		if (x < NH)
+			lw.b1[x] = b[0];
+		else if (x < 2 * NH)
+			lw.b2[x - NH] = b[0];
+		else if (x < 2 * NH + 16)
+			lw.b3[x - 2 * NH] = b[0];
+	}
+};
+
+// mlp_rows on the split weights.  A part of the weights is read once for the
+// products it is in (with the activations' parts 0; 1, 0; 2, 1, 0), one part
+// ahead of them: the scheduling barriers let arithmetic through but no LDS
+// read, which left alone are all placed early and take half the wavefronts'
+// registers.
+template <int NI, bool FAST>
+__device__ __forceinline__ f4 mlp_rows_split(LWS<NI> const &lw, const float (&x)[NI / 4])
+{
+	using W = LWS<NI>;
+	const int l = threadIdx.x & 63, q4 = (l >> 4) * 4;
+	// acc[b] += the six products of weight fragments at(b, part) and activation parts s
+	auto products = [&](auto at, auto const &s, auto mm, auto &acc) {
+		constexpr int B = sizeof(acc) / sizeof(f4);
+		decltype(at(0, 0)) w[2][B];
+#pragma unroll
+		for (int b = 0; b < B; ++b)
+			w[0][b] = at(b, 2);
+#pragma unroll
+		for (int k = 2; k >= 0; --k)
+		{
+			if (k > 0)
+#pragma unroll
+				for (int b = 0; b < B; ++b)
+					w[(k + 1) & 1][b] = at(b, k - 1);
+			__builtin_amdgcn_sched_barrier(1);
+#pragma unroll
+			for (int j = 2 - k; j >= 0; --j)
+#pragma unroll
+				for (int b = 0; b < B; ++b)
+					acc[b] = mm(w[k & 1][b], s.part(j), acc[b]);
+		}
+	};
+	auto mm8 = [](bf8 a, bf8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); };
+	auto mm4 = [](Split<4>::vec a, Split<4>::vec b, f4 c) {
+		return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0,
+		                                                 0);
+	};
+	f4 h[4], g[4], y[1];
+#pragma unroll
+	for (int b = 0; b < 4; ++b)
+	{
+		h[b] = *reinterpret_cast<const f4 *>(lw.b1 + 16 * b + q4);
+		g[b] = *reinterpret_cast<const f4 *>(lw.b2 + 16 * b + q4);
+	}
+	y[0] = *reinterpret_cast<const f4 *>(lw.b3 + q4);
+	float v[8], r[4];
+#pragma unroll
+	for (int e = 0; e < 8; ++e)
+		v[e] = x[e];
+#pragma unroll
+	for (int e = 0; e < 4; ++e)
+		r[e] = e < W::R4 ? x[8 + (e < W::R4 ? e : 0)] : 0.f;
+	products([&](int b, int k) { return lw.w1[0][b][k][l]; }, split<8>(v), mm8, h);
+	products([&](int b, int k) { return lw.w1r[b][k][l]; }, split<4>(r), mm4, h);
+	auto parts = [](f4 a, f4 b) {
+		const float v[8] = {act<FAST>(a[0]), act<FAST>(a[1]), act<FAST>(a[2]), act<FAST>(a[3]),
+		                    act<FAST>(b[0]), act<FAST>(b[1]), act<FAST>(b[2]), act<FAST>(b[3])};
+		return split<8>(v);
+	};
+#pragma unroll
+	for (int t = 0; t < 2; ++t)
+		products([&](int b, int k) { return lw.w2[t][b][k][l]; }, parts(h[2 * t], h[2 * t + 1]), mm8, g);
+#pragma unroll
+	for (int t = 0; t < 2; ++t)
+		products([&](int, int k) { return lw.w3[t][k][l]; }, parts(g[2 * t], g[2 * t + 1]), mm8, y);
+	return y[0];
 }
 
 // outputs of mlp_rows to y[row * YS + column] (one wavefront's scratch, 16 YS floats)

@@ -26,8 +26,9 @@
 // any plaquette it has not transformed (a link-space coupling layer moves a
 // second, passive plaquette with every link it updates).
 //
-// Kernels: one workgroup (256 threads) per configuration, plaquettes in LDS,
-// the dense layers on FP32 MFMA (flow_mlp.h).
+// Kernels: one workgroup per configuration, plaquettes in LDS, the dense layers
+// on MFMA (flow_mlp.h): BF16 MFMA on split numbers in the forward and inverse
+// kernels, FP32 MFMA in the backward one.
 #include "flow_mlp.h"
 #include "mesh_internal.h"
 #include "rng_dev.h"
@@ -50,11 +51,13 @@ constexpr int NI = 40; // features: 20 loops, (cos, sin) each
 constexpr int NP_LAYER = FM::Layout<NI>::NP;
 constexpr int MAX_LAYERS = 64;
 constexpr int THREADS = 256; // of the backward kernel
-// smallest volume on 512 threads (forward and inverse): every one of the eight
-// wavefronts has a tile in a layer from V / 4 = 8 * 16 on.  32^2, 256 chains:
-// sample 126.5 us on 256 threads, 117.6 on 512; propose 217 and 209; 64^2
-// propose 1003 and 876
-constexpr int WIDE_V = 512;
+// Forward and inverse run on 512 threads from WIDE_V plaquettes on, where each
+// of the eight wavefronts has a tile in a layer (V / 4 >= 8 * 16), unless the
+// launch has more workgroups than CUs and two of 256 threads fit a CU's LDS
+// (V <= PAIR_V): those run side by side without each other's barriers.  256
+// chains: sample 32^2 103 us on 256 threads, 90 on 512, 64^2 342 and 282; propose
+// (512 workgroups) 32^2 161 and 179, 64^2 772 and 617.
+constexpr int WIDE_V = 512, PAIR_V = 1664;
 constexpr bool FAST = true; // tanh_fast in every kernel of this flow
 constexpr uint32_t TAG_PCFZ = 0x5043465au; // prior, holonomies, gauge
 constexpr uint32_t TAG_PCFI = 0x50434649u; // initial weights
@@ -101,7 +104,7 @@ __device__ __forceinline__ float2 sincos2(float a)
 // LDS of the forward and inverse kernels of NT threads
 template <int NT> struct PCSharedF
 {
-	FM::LWP<NI> lw;
+	FM::LWS<NI> lw;
 	float y[NT / 64][16 * FM::YS];
 	double red[4][NT / 64];
 };
@@ -144,7 +147,7 @@ struct LaneLoops
 };
 
 // One layer on the workgroup: wavefront w takes tiles w, w + NT / 64, ... of
-// the NA active plaquettes: features and MLP in registers (mlp_rows), then the
+// the NA active plaquettes: features and MLP in registers (mlp_rows_split), then the
 // circle map on quads (lane 4i + k: row i of the tile, mixture component k),
 // to which the outputs go through 1.25 KB of LDS.  Features read only frozen
 // plaquettes, so a wavefront may move its active ones while the others still
@@ -162,9 +165,7 @@ __device__ __forceinline__ void layer_apply(PCGeo const &g, LaneLoops const &ll,
 		active_xy(g, m, min(tix * 16 + (l & 15), NA - 1), x0, x1);
 		float x[NI / 4];
 		ll.features(g, cs, x0, x1, x);
-		FM::f4 h1[4], h2[4];
-		const FM::f4 out = FM::mlp_rows<NI, FAST, NT == 256>(sh.lw, x, [&](int s) { return LaneLoops::row(ll.q, s); }, h1, h2);
-		FM::put_outputs(y, out);
+		FM::put_outputs(y, FM::mlp_rows_split<NI, FAST>(sh.lw, x));
 		FM::wave_sync();
 		const int row = l >> 2, r = tix * 16 + row;
 		if (r < NA)
@@ -204,10 +205,9 @@ __device__ __forceinline__ void pc_forward(PCGeo const &g, int nl, const float *
 	float2 *cs = reinterpret_cast<float2 *>(dyn + g.V);
 	float *al = dyn + 3 * g.V;
 	const uint32_t cc = (uint32_t)c << 1;
-	FM::WeightRegsP<NI, NT> wr;
+	FM::WeightFrags<NI, NT, LaneLoops> wr;
 	const LaneLoops ll;
 	wr.load(params);
-	FM::zero_pad<NI>(sh.lw);
 	for (int x = threadIdx.x; x < g.V; x += NT)
 	{
 		const float z = x < g.V - 1 ? u1_plaq::uniform_angle(seed, step, (uint32_t)x, cc, TAG_PCFZ) : 0.f;
@@ -275,10 +275,9 @@ __device__ __forceinline__ void pc_inverse(PCGeo const &g, int nl, const float *
 	float *th = dyn;
 	float2 *cs = reinterpret_cast<float2 *>(dyn);
 	float *phi = dyn + 2 * g.V;
-	FM::WeightRegsP<NI, NT> wr;
+	FM::WeightFrags<NI, NT, LaneLoops> wr;
 	const LaneLoops ll;
 	wr.load(params + (long)(nl - 1) * NP_LAYER);
-	FM::zero_pad<NI>(sh.lw);
 	for (int i = threadIdx.x; i < 2 * g.V; i += NT)
 		th[i] = theta[(long)c * 2 * g.V + i];
 	__syncthreads();
@@ -316,9 +315,10 @@ __device__ __forceinline__ void pc_inverse(PCGeo const &g, int nl, const float *
 
 // The kernels run on 256 or 512 threads (by_width()).
 template <int NT>
-__global__ __launch_bounds__(NT) void k_pc_forward(PCGeo g, int nl, const float *__restrict__ params, uint64_t seed,
-                                                   uint32_t step, float *theta_out, float *phi_layers,
-                                                   float *phi_final, double *out)
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
+void k_pc_forward(PCGeo g, int nl, const float *__restrict__ params, uint64_t seed,
+                  uint32_t step, float *theta_out, float *phi_layers,
+                  float *phi_final, double *out)
 {
 	extern __shared__ float dyn[];
 	__shared__ PCSharedF<NT> sh;
@@ -326,8 +326,9 @@ __global__ __launch_bounds__(NT) void k_pc_forward(PCGeo g, int nl, const float 
 }
 
 template <int NT>
-__global__ __launch_bounds__(NT) void k_pc_inverse(PCGeo g, int nl, const float *__restrict__ params,
-                                                   const float *__restrict__ theta, float *z_out, double *out)
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
+void k_pc_inverse(PCGeo g, int nl, const float *__restrict__ params,
+                  const float *__restrict__ theta, float *z_out, double *out)
 {
 	extern __shared__ float dyn[];
 	__shared__ PCSharedF<NT> sh;
@@ -338,9 +339,10 @@ __global__ __launch_bounds__(NT) void k_pc_inverse(PCGeo g, int nl, const float 
 // the current configurations, batch..2 batch-1 draw the proposals, so that on
 // small lattices (two workgroups' LDS per CU) the two passes share the CUs
 template <int NT>
-__global__ __launch_bounds__(NT) void k_pc_propose(PCGeo g, int nl, const float *__restrict__ params, int batch,
-                                                   const float *__restrict__ theta, double *state, uint64_t seed,
-                                                   uint32_t step, float *theta_prop, double *prop_out)
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
+void k_pc_propose(PCGeo g, int nl, const float *__restrict__ params, int batch,
+                  const float *__restrict__ theta, double *state, uint64_t seed,
+                  uint32_t step, float *theta_prop, double *prop_out)
 {
 	extern __shared__ float dyn[];
 	__shared__ PCSharedF<NT> sh;
@@ -410,7 +412,7 @@ __global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const 
 			float x[NI / 4], *y = sh.buf.y[w];
 			ll.features(g, cs, x0, x1, x);
 			FM::f4 h1[4], h2[4], dx[FM::GradP<NI>::NB];
-			const FM::f4 out = FM::mlp_rows<NI, FAST, true>(sh.lw, x, [&](int k) { return row(ll.q, k); }, h1, h2);
+			const FM::f4 out = FM::mlp_rows<NI, FAST>(sh.lw, x, [&](int k) { return row(ll.q, k); }, h1, h2);
 			FM::put_outputs(y, out);
 			FM::wave_sync();
 			{
@@ -505,10 +507,10 @@ template <class K> int set_lds(mesh_ctx *ctx, K kernel, size_t bytes)
 	return MESH_OK;
 }
 
-// kernel(std::integral_constant<int, threads>) on 512 threads from WIDE_V on
-template <class F> int by_width(PCGeo const &g, F &&kernel)
+// kernel(std::integral_constant<int, threads>) for a launch of so many workgroups
+template <class F> int by_width(PCGeo const &g, int blocks, F &&kernel)
 {
-	if (g.V >= WIDE_V)
+	if (g.V >= WIDE_V && (blocks <= 256 || g.V > PAIR_V))
 		return kernel(std::integral_constant<int, 512>{});
 	return kernel(std::integral_constant<int, 256>{});
 }
@@ -552,7 +554,7 @@ int mesh_pcflow_sample(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers,
 		return rc;
 	if (!params || !theta_out || !out_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_sample");
-	return by_width(pg, [&](auto nt) {
+	return by_width(pg, batch, [&](auto nt) {
 		return launch_forward<decltype(nt)::value>(ctx, pg, batch, layers, params, seed, step, theta_out, nullptr,
 		                                           nullptr, out_dev);
 	});
@@ -567,7 +569,7 @@ int mesh_pcflow_logq(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers, c
 		return rc;
 	if (!params || !theta || !out_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_logq");
-	return by_width(pg, [&](auto nt) -> int {
+	return by_width(pg, batch, [&](auto nt) -> int {
 		constexpr int NT = decltype(nt)::value;
 		const size_t lds = 3 * (size_t)pg.V * sizeof(float);
 		if (int rc = set_lds(ctx, k_pc_inverse<NT>, lds))
@@ -590,7 +592,7 @@ int mesh_pcflow_propose(mesh_ctx *ctx, const mesh_grid *g, int batch, int layers
 		return mesh_fail(ctx, MESH_E_ARG, "NULL argument to pcflow_propose");
 	if (theta == theta_prop || state_dev == prop_dev)
 		return mesh_fail(ctx, MESH_E_ARG, "pcflow_propose: the proposals and their log q need their own buffers");
-	return by_width(pg, [&](auto nt) -> int {
+	return by_width(pg, 2 * batch, [&](auto nt) -> int {
 		constexpr int NT = decltype(nt)::value;
 		const size_t lds = 4 * (size_t)pg.V * sizeof(float);
 		if (int rc = set_lds(ctx, k_pc_propose<NT>, lds))
@@ -627,7 +629,7 @@ int mesh_pcflow_gradient(mesh_ctx *ctx, const mesh_grid *g, int batch, int layer
 	float *pf = pl + (size_t)batch * layers * pg.V;
 	float *drs = pf + (size_t)batch * pg.V;
 	float *part = drs + (size_t)batch * (pg.V / 4) * 8;
-	if (int rc = by_width(pg, [&](auto nt) {
+	if (int rc = by_width(pg, batch, [&](auto nt) {
 		    return launch_forward<decltype(nt)::value>(ctx, pg, batch, layers, params, seed, step, nullptr, pl, pf,
 		                                               out_dev);
 	    }))

@@ -118,6 +118,43 @@ def test_pcflow_tile_edges(ctx, L0, L1):
     np.testing.assert_allclose(inv[:, 0], out[:, 0], atol=tol)
 
 
+@pytest.mark.parametrize("L0,L1", [(4, 128), (24, 24), (26, 64), (28, 60)])
+def test_pcflow_width_by_batch(ctx, L0, L1):
+    """more workgroups than CUs run on 256 threads up to 1664 plaquettes: the
+    first chains of a large batch are those of a small one (the same steps a
+    plaquette; the sums of V terms below 1 in another order)"""
+    B, n, V = 257, 3, L0 * L1
+    f = U1.PlaqCouplingFlow(L0, L1, ctx)
+    f.set_params(_params(21, 0.2))
+    runs = []
+    for b in (B, n):
+        ens = U1.U1Ensemble(L0, L1, b, ctx)
+        out = f.sample(ens, 23, 4).download().reshape(b, 2)[:n]
+        runs.append((out, ens.angles()[:n], f.logq(ens).download().reshape(b, 2)[:n]))
+    (out, th, inv), (out1, th1, inv1) = runs
+    np.testing.assert_array_equal(th, th1)
+    for a, b in ((out, out1), (inv, inv1)):
+        np.testing.assert_allclose(a, b, rtol=1e-6, atol=8 * V * 2.0**-24)
+
+
+def test_pcflow_infinite_weights(ctx):
+    """an infinite weight saturates its unit as any other large one does"""
+    L, B = 8, 2
+    res = []
+    for big in (np.inf, 3.40e38, 1e30):
+        p = _params(22, 0.2)
+        p[5], p[-814] = big, -big # of the first layer's W1, the last one's W2
+        f = U1.PlaqCouplingFlow(L, L, ctx)
+        f.set_params(p)
+        ens = U1.U1Ensemble(L, L, B, ctx)
+        out = f.sample(ens, 29, 1).download().reshape(B, 2)
+        res.append((ens.angles(), out))
+    for th, out in res:
+        assert np.isfinite(out).all()
+        np.testing.assert_array_equal(th, res[2][0])
+        np.testing.assert_array_equal(out, res[2][1])
+
+
 def test_pcflow_inverse_roundtrip(ctx):
     """log q by the inverse of a sample equals the sampler's log q and
     recovers its prior draws"""
