@@ -185,19 +185,21 @@ template <class R> __device__ __forceinline__ void or_site(Geo const &g, R *U, R
 {
 	int f = g.nd - 1;
 	int hl = g.L[f] >> 1;
-	// sites are below 2^26: 32-bit divisions
-	long row = (long)((unsigned)t / (unsigned)hl);
+	long row = g.by[f]((unsigned)(2 * t)); // 2 t below 2^26
 	int j = (int)(t - row * hl);
 	long x0 = row * g.L[f];
 	// x's coordinates: the row start's in the slower directions, 2 j + the
 	// parity bit along the row (one division per direction in all)
 	int cc[4] = {0, 0, 0, 0}, ps = 0;
+	unsigned r = (unsigned)row;
 #pragma unroll
-	for (int mu = 0; mu < 3; ++mu)
+	for (int mu = 2; mu >= 0; --mu)
 		if (mu < f)
 		{
-			cc[mu] = coord(g, x0, mu);
+			const unsigned q = g.by[mu](r);
+			cc[mu] = (int)(r - q * (unsigned)g.L[mu]);
 			ps += cc[mu];
+			r = q;
 		}
 	long x = x0 + 2 * j + ((parity + ps) & 1);
 	m3<R> K = zero_m3<R>();
@@ -269,9 +271,9 @@ template <class R> __global__ __launch_bounds__(256) void k_or_half(Geo g, R *U,
 // holding its backward neighbours run close together and share the L2 lines
 // that each half-sweep touches half of.
 template <class R>
-__global__ __launch_bounds__(128) void k_or_half_span(Geo g, R *U, R *h, int parity, R omega, int nb, int order)
+__global__ __launch_bounds__(128) void k_or_half_span(Geo g, R *U, R *h, int parity, R omega, BlockOrder ord)
 {
-	int lb = ordered_block(g, nb, 256, order);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	or_site(g, U, h, parity, omega, (long)lb * 128 + threadIdx.x);
@@ -381,12 +383,12 @@ int mesh_landau_or_halfsweep(mesh_ctx *ctx, const mesh_grid *g, int prec, void *
 	{
 		int nb = (int)(geo.V / 256);
 		int gb = mesh_grid_blocks(ctx, nb);
+		const BlockOrder ord = block_order(geo, nb, 256, mesh_order(ctx));
 		if (prec == MESH_F64)
-			k_or_half_span<double><<<gb, 128, 0, ctx->stream>>>(geo, (double *)U, (double *)h, parity, omega, nb,
-			                                                    mesh_order(ctx));
+			k_or_half_span<double><<<gb, 128, 0, ctx->stream>>>(geo, (double *)U, (double *)h, parity, omega, ord);
 		else
 			k_or_half_span<float><<<gb, 128, 0, ctx->stream>>>(geo, (float *)U, (float *)h, parity, (float)omega,
-			                                                   nb, mesh_order(ctx));
+			                                                   ord);
 	}
 	else
 	{

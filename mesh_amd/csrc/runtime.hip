@@ -55,10 +55,12 @@ int mesh_make_geo(mesh_ctx *ctx, const mesh_grid *g, Geo *geo)
 		{
 			geo->L[i] = 1;
 			geo->st[i] = 0;
+			geo->by[i] = FastDiv(1);
 			continue;
 		}
 		geo->L[i] = g->dims[i];
 		geo->st[i] = (int)s;
+		geo->by[i] = FastDiv((uint32_t)g->dims[i]);
 		s *= g->dims[i];
 	}
 	geo->V = V;

@@ -127,6 +127,7 @@ struct G2
 	int nd;
 	int L[4], st[4];
 	long V, stride;
+	FastDiv by[4]; // division by L
 };
 
 // neighbour x + s mu^ (|s| <= L_mu); 32-bit arithmetic (V <= 2^26 sites): a
@@ -151,7 +152,7 @@ __device__ __forceinline__ void coords2(G2 const &g, long x, int (&c)[4])
 	{
 		if (mu < g.nd)
 		{
-			const unsigned q = t / (unsigned)g.L[mu];
+			const unsigned q = g.by[mu](t);
 			c[mu] = (int)(t - q * (unsigned)g.L[mu]);
 			t = q;
 		}
@@ -316,15 +317,15 @@ __global__ __launch_bounds__(256) void k_su2_force_link(G2 g, const R *__restric
 // 4 x 64 links in LDS, and reads there the link itself and the staple links
 // at x and at its x3-neighbours (7 of 18); the others come from global memory.
 // Workgroups follow the XCD-aware block order of the SU(3) stencil kernels
-// (ordered_block_of).  The arithmetic is that of k_su2_force_link (staple():
+// (BlockOrder).  The arithmetic is that of k_su2_force_link (staple():
 // the same products in the same order), so the bits are the same.
 template <class R>
 __global__ __launch_bounds__(256) void k_su2_force_link_rows(G2 g, const R *__restrict__ U, R *__restrict__ P,
-                                                             double k, R *__restrict__ Unext, R t, int reunit, int nb,
-                                                             int order)
+                                                             double k, R *__restrict__ Unext, R t, int reunit,
+                                                             BlockOrder ord)
 {
 	__shared__ v4<R> own[4][64];
-	const int lb = ordered_block_of(g, nb, 64, order, blockIdx.x);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	const int mu = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(256) void k_su2_force_link_rows(G2 g, const R *__re
 		return qt<R>{v.x, v.y, v.z, v.w};
 	};
 	// slots of the x3-neighbours (the block starts a row: 64 % L3 == 0)
-	const int L3 = g.L[3], c3 = lane % L3, o0 = lane - c3;
+	const int L3 = g.L[3], c3 = lane & (L3 - 1), o0 = lane - c3; // L3 | 64
 	const int sp = o0 + (c3 + 1 == L3 ? 0 : c3 + 1), sm = o0 + (c3 == 0 ? L3 - 1 : c3 - 1);
 	qt<R> S = {R(0), R(0), R(0), R(0)};
 	int c[4];
@@ -576,12 +577,12 @@ template <class R> __device__ __forceinline__ qt<R> or_step(qt<R> K, R omega)
 // each thread reads its site's 8 links once (in this half-sweep no other
 // thread touches them: a link joins one site of each parity).
 template <class R>
-__global__ __launch_bounds__(256) void k_su2_or_half(G2 g, R *U, R *h, int parity, R omega, int nb, int order)
+__global__ __launch_bounds__(256) void k_su2_or_half(G2 g, R *U, R *h, int parity, R omega, int nb, BlockOrder ord)
 {
 	long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (nb > 0)
 	{
-		const int lb = ordered_block_of(g, nb, 512, order, blockIdx.x);
+		const int lb = ord.at(blockIdx.x);
 		if (lb < 0)
 			return;
 		t = (long)lb * 256 + threadIdx.x;
@@ -589,18 +590,20 @@ __global__ __launch_bounds__(256) void k_su2_or_half(G2 g, R *U, R *h, int parit
 	if (t >= (g.V >> 1))
 		return;
 	const int f = g.nd - 1, hl = g.L[f] >> 1;
-	// sites are below 2^31 (nbr's 32-bit arithmetic): 32-bit divisions
-	const long row = (long)((unsigned)t / (unsigned)hl);
+	const long row = g.by[f]((unsigned)(2 * t)); // 2 t below 2^26
 	const long x0 = row * g.L[f];
 	// coordinates of the row's first site in the slower directions, then x's
 	// along the row
 	int cc[4] = {0, 0, 0, 0}, ps = 0;
+	unsigned r = (unsigned)row;
 #pragma unroll
-	for (int mu = 0; mu < 3; ++mu)
+	for (int mu = 2; mu >= 0; --mu)
 		if (mu < f)
 		{
-			cc[mu] = (int)(((unsigned)x0 / (unsigned)g.st[mu]) % (unsigned)g.L[mu]);
+			const unsigned q = g.by[mu](r);
+			cc[mu] = (int)(r - q * (unsigned)g.L[mu]);
 			ps += cc[mu];
+			r = q;
 		}
 	const long x = x0 + 2 * (t - row * hl) + ((parity + ps) & 1);
 	qt<R> fw[4], bw[4];
@@ -665,6 +668,7 @@ int make_g2(mesh_ctx *ctx, const mesh_grid *g, G2 *o)
 	{
 		o->L[i] = geo.L[i];
 		o->st[i] = geo.st[i];
+		o->by[i] = geo.by[i];
 	}
 	o->V = geo.V;
 	o->stride = geo.stride;
@@ -731,7 +735,7 @@ int launch_force_link(mesh_ctx *ctx, G2 const &g, int prec, const void *U, void 
 		{
 			const int nb = (int)(g.V / 64);
 			k_su2_force_link_rows<R><<<mesh_grid_blocks(ctx, nb), 256, 0, ctx->stream>>>(
-			    g, as<R>(U), as<R>(P), k, as<R>(Unext), (R)t, reunit, nb, mesh_order(ctx));
+			    g, as<R>(U), as<R>(P), k, as<R>(Unext), (R)t, reunit, block_order(g, nb, 64, mesh_order(ctx)));
 		}
 		else
 			k_su2_force_link<R><<<nblk(g.V * g.nd), 256, 0, ctx->stream>>>(g, as<R>(U), as<R>(P), k,
@@ -1181,7 +1185,7 @@ int mesh_su2_landau_or_halfsweep(mesh_ctx *ctx, const mesh_grid *g, int prec, vo
 		using R = decltype(tag);
 		const int nb = geo.V % 512 == 0 ? (int)(geo.V / 512) : 0;
 		k_su2_or_half<R><<<nb > 0 ? mesh_grid_blocks(ctx, nb) : nblk(geo.V / 2), 256, 0, ctx->stream>>>(
-		    geo, as<R>(U), as<R>(h), parity, (R)omega, nb, mesh_order(ctx));
+		    geo, as<R>(U), as<R>(h), parity, (R)omega, nb, block_order(geo, nb, 512, mesh_order(ctx)));
 	});
 	mesh_prof_end(ctx, ph);
 	MESH_LAUNCHED(ctx);

@@ -582,6 +582,27 @@ template <bool AH, class R> MHD m3<R> mom_step(m3<R> const &p, m3<R> const &M, d
 
 // ---- geometry ---------------------------------------------------------------
 
+// n / d for 0 <= n < 2^31 by a multiplication, an addition and a shift: the
+// divisors are known at launch, and the compiler's division by a variable is
+// some thirty instructions, a reciprocal and four 32-bit products among them.
+// With 2^l the power of two at or above d and m = floor(2^32 (2^l - d) / d) + 1,
+// n / d = (floor(m n / 2^32) + n) / 2^l (Granlund and Montgomery 1994).
+struct FastDiv
+{
+	uint32_t m = 1, l = 0;
+	FastDiv() = default;
+	explicit FastDiv(uint32_t d)
+	{
+		while ((1ull << l) < d)
+			++l;
+		m = (uint32_t)((((1ull << l) - d) << 32) / d) + 1;
+	}
+	__host__ __device__ __forceinline__ uint32_t operator()(uint32_t n) const
+	{
+		return ((uint32_t)(((uint64_t)m * n) >> 32) + n) >> l;
+	}
+};
+
 struct Geo
 {
 	int nd;
@@ -589,6 +610,7 @@ struct Geo
 	int st[4]; // site strides, st[nd-1] = 1
 	long V;
 	long stride; // sites per direction block, V rounded up to a multiple of 256
+	FastDiv by[4]; // division by L
 };
 
 // ---- field access -------------------------------------------------------------
@@ -856,10 +878,10 @@ MHD LaneSlots halo_slots(int L3, int n, int l, int c3)
 // site of halo slot 64 + h: the site before the block, the first row's start,
 // the site behind the block, the last row's end (b0, or a site of the block,
 // where no lane reads the slot)
-MHD long halo_site(int L3, long b0, int n, int h)
+MHD long halo_site(int L3, FastDiv by_L3, long b0, int n, int h)
 {
 	const long bl = b0 + n - 1;
-	const int c3f = (int)((unsigned)b0 % (unsigned)L3), c3l = (int)((unsigned)bl % (unsigned)L3);
+	const int c3f = (int)b0 - (int)by_L3((unsigned)b0) * L3, c3l = (int)bl - (int)by_L3((unsigned)bl) * L3;
 	return h == 0 ? (c3f > 0 ? b0 - 1 : b0) : (h == 1 ? b0 - c3f : (h == 2 ? (c3l < L3 - 1 ? bl + 1 : b0) : bl - c3l + L3 - 1));
 }
 

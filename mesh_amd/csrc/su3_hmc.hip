@@ -24,16 +24,11 @@ using namespace mesh_dev;
 #define MESH_PIPE_F64 1
 #endif
 // The global operands of the shared upper-staple factors loaded before the
-// staging barrier (share_fetch; same bits), FP32 / FP64; 0: after it.  With
-// three FP32 workgroups per CU it gained 1.2% (0.3443 -> 0.3401 ms at 32^4);
-// with four (the four-plane mode) it costs 0.4% (0.3417 vs 0.3432 ms, three
-// same-box rounds), and in FP64 it is even (0.5626 vs 0.5626 ms).
-#ifndef MESH_SHARE_PREFETCH
-#define MESH_SHARE_PREFETCH 0
-#endif
-#ifndef MESH_SHARE_PREFETCH_F64
-#define MESH_SHARE_PREFETCH_F64 0
-#endif
+// staging barrier (share_fetch; same bits) instead of after it: in FP64 on the
+// rows path, 32^4 568.5 -> 566.5 us.  With the halo slots it loses (FP64 36^4
+// 1045 -> 1087, 48^4 3047 -> 3162), and in FP32 the four workgroups of a CU cover
+// the latency (32^4 341.7 -> 343.2).
+template <class R, bool ROWS> constexpr bool share_prefetch() { return ROWS && std::is_same<R, double>::value; }
 // waves per SIMD the force kernels are compiled for (0: the compiler's choice)
 #ifndef MESH_FORCE_WAVES
 #define MESH_FORCE_WAVES 0
@@ -181,7 +176,7 @@ template <class R> __device__ __forceinline__ void coords(Geo const &g, long x, 
 	{
 		if (mu < g.nd)
 		{
-			unsigned q = t / (unsigned)g.L[mu];
+			const unsigned q = g.by[mu](t);
 			c[mu] = (int)(t - q * (unsigned)g.L[mu]);
 			t = q;
 		}
@@ -593,9 +588,9 @@ __global__ __launch_bounds__(256) void k_momenta_link(Geo g, R *__restrict__ P, 
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void k_plaq(Geo g, const R *__restrict__ U, double *partials, int nb, int remap)
+__global__ __launch_bounds__(256) void k_plaq(Geo g, const R *__restrict__ U, double *partials, int nb, BlockOrder ord)
 {
-	int lb = ordered_block(g, nb, 256, remap);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	long x = lane_site(g, (long)lb * 256 + threadIdx.x);
@@ -614,9 +609,9 @@ __global__ __launch_bounds__(256) void k_plaq(Geo g, const R *__restrict__ U, do
 template <class R, bool PC>
 __global__ __launch_bounds__(256) DH_OCC void k_delta_h(Geo g, const R *__restrict__ Uo, const R *__restrict__ Un,
                                                  const R *__restrict__ P, const double *__restrict__ Ko,
-                                                 double c3, double *partials, int nb, int remap)
+                                                 double c3, double *partials, int nb, BlockOrder ord)
 {
-	int lb = ordered_block(g, nb, 256, remap);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	long x = lane_site(g, (long)lb * 256 + threadIdx.x);
@@ -646,10 +641,10 @@ __global__ __launch_bounds__(256) DH_OCC void k_delta_h(Geo g, const R *__restri
 template <class R, bool PC>
 __global__ __launch_bounds__(256) void k_delta_h_split(Geo g, const R *__restrict__ Uo, const R *__restrict__ Un,
                                                        const R *__restrict__ P, const double *__restrict__ Ko,
-                                                       double c3, double *partials, int nb, int remap)
+                                                       double c3, double *partials, int nb, BlockOrder ord)
 {
 	__shared__ double pso_s[128];
-	int lb = ordered_block(g, nb, 128, remap);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	const bool newer = threadIdx.x >= 128;
@@ -821,10 +816,10 @@ inline int staple_path(Geo const &g)
 template <class R, bool FUSE, bool PC, int PATH>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R, PATH>()))) void k_force_update(
-    Geo g, const R *__restrict__ U, R *__restrict__ P, double kc, int nb, int remap, R *__restrict__ Unext, R tl,
+    Geo g, const R *__restrict__ U, R *__restrict__ P, double kc, BlockOrder ord, R *__restrict__ Unext, R tl,
     int reunit_flag)
 {
-	int lb = ordered_block(g, nb, SB, remap);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	const int mu = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -853,7 +848,7 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 		else
 			at = halo_slots(g.L[3], n, (int)(x - b0), c[3]);
 		ShareOps<R> F;
-		constexpr bool PF = std::is_same<R, float>::value ? MESH_SHARE_PREFETCH : MESH_SHARE_PREFETCH_F64;
+		constexpr bool PF = share_prefetch<R, RW>();
 		constexpr bool PIPE = MESH_PIPE_F64 && std::is_same<R, double>::value;
 #define MESH_BY_DIRECTION(CALL)                                                                    \
 	switch (mu)                                                                                    \
@@ -889,7 +884,7 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 			{
 				const int h = threadIdx.x & 3, d = (threadIdx.x >> 2) & 3, k = threadIdx.x >> 4;
 				own[d][k][64 + h] = reinterpret_cast<const vec2_t<R> *>(
-				    U)[site_off(g, d, halo_site(g.L[3], b0, n, h)) + k * plane_step(g)];
+				    U)[site_off(g, d, halo_site(g.L[3], g.by[3], b0, n, h)) + k * plane_step(g)];
 			}
 		__syncthreads();
 		if constexpr (!PF)
@@ -929,7 +924,7 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 // direction w; the arithmetic (and the layout of P) is that of k_force_update.
 template <class R, int L3, bool FUSE, bool PC = FUSE>
 __global__ __launch_bounds__(256) FORCE_OCC void k_force_update_tile(Geo g, const R *__restrict__ U, R *__restrict__ P,
-                                                                     double kc, int nb, int remap, R *__restrict__ Unext,
+                                                                     double kc, BlockOrder ord, R *__restrict__ Unext,
                                                                      R tl, int reunit_flag)
 {
 	constexpr int RW = 64 / L3; // rows per tile
@@ -941,7 +936,7 @@ __global__ __launch_bounds__(256) FORCE_OCC void k_force_update_tile(Geo g, cons
 	constexpr int RS = 36 * L3 + 128 / (int)sizeof(vec2_t<R>);
 	__shared__ vec2_t<R> lds[NR * RS];
 	auto slot3 = [](int c3) { return MESH_SITE_PAIRS ? ((c3 & 1) * (L3 / 2) + (c3 >> 1)) : c3; };
-	int lb = ordered_block(g, nb, 64, remap);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	const long base = (long)lb * 64; // first site of the tile (x3 = 0 of its first row)
@@ -1046,9 +1041,9 @@ __global__ __launch_bounds__(256) FORCE_OCC void k_force_update_tile(Geo g, cons
 // variant: one thread per site looping over the directions
 template <class R>
 __global__ __launch_bounds__(256) void k_force_update_site(Geo g, const R *__restrict__ U, R *__restrict__ P, double kc,
-                                                           int nb, int remap)
+                                                           BlockOrder ord)
 {
-	int lb = ordered_block(g, nb, 256, remap);
+	const int lb = ord.at(blockIdx.x);
 	if (lb < 0)
 		return;
 	long x = lane_site(g, (long)lb * 256 + threadIdx.x);
@@ -1246,9 +1241,11 @@ int plaq_sum(mesh_ctx *ctx, Geo const &geo, int prec, const void *U, double *out
 	int gb = mesh_grid_blocks(ctx, nb);
 	int ph = mesh_prof_begin(ctx, PROF_PLAQ);
 	if (prec == MESH_F64)
-		k_plaq<double><<<gb, 256, 0, ctx->stream>>>(geo, (const double *)U, ctx->partials, nb, mesh_order(ctx));
+		k_plaq<double><<<gb, 256, 0, ctx->stream>>>(geo, (const double *)U, ctx->partials, nb,
+		                                            block_order(geo, nb, 256, mesh_order(ctx)));
 	else
-		k_plaq<float><<<gb, 256, 0, ctx->stream>>>(geo, (const float *)U, ctx->partials, nb, mesh_order(ctx));
+		k_plaq<float><<<gb, 256, 0, ctx->stream>>>(geo, (const float *)U, ctx->partials, nb,
+		                                           block_order(geo, nb, 256, mesh_order(ctx)));
 	mesh_prof_end(ctx, ph);
 	MESH_LAUNCHED(ctx);
 	return mesh_finish_reduction(ctx, nb, 1, out);
@@ -1285,18 +1282,19 @@ int launch_force_update(mesh_ctx *ctx, Geo const &geo, int prec, const void *U, 
 	{
 		int nb = (int)(geo.V / 64);
 		int gb = mesh_grid_blocks(ctx, nb);
+		const BlockOrder ord = block_order(geo, nb, 64, mesh_order(ctx));
 		auto launch = [&](auto tag, auto l3) {
 			using Rt = decltype(tag);
 			constexpr int l3v = decltype(l3)::value;
 			if (fused && compact)
 				k_force_update_tile<Rt, l3v, true, true><<<gb, 256, 0, ctx->stream>>>(
-				    geo, (const Rt *)U, (Rt *)P, k, nb, mesh_order(ctx), (Rt *)Unext, (Rt)tl, reunit_flag);
+				    geo, (const Rt *)U, (Rt *)P, k, ord, (Rt *)Unext, (Rt)tl, reunit_flag);
 			else if (fused)
 				k_force_update_tile<Rt, l3v, true, false><<<gb, 256, 0, ctx->stream>>>(
-				    geo, (const Rt *)U, (Rt *)P, k, nb, mesh_order(ctx), (Rt *)Unext, (Rt)tl, reunit_flag);
+				    geo, (const Rt *)U, (Rt *)P, k, ord, (Rt *)Unext, (Rt)tl, reunit_flag);
 			else
 				k_force_update_tile<Rt, l3v, false><<<gb, 256, 0, ctx->stream>>>(
-				    geo, (const Rt *)U, (Rt *)P, k, nb, mesh_order(ctx), nullptr, (Rt)0, 0);
+				    geo, (const Rt *)U, (Rt *)P, k, ord, nullptr, (Rt)0, 0);
 		};
 		using I16 = std::integral_constant<int, 16>;
 		using I32 = std::integral_constant<int, 32>;
@@ -1311,29 +1309,30 @@ int launch_force_update(mesh_ctx *ctx, Geo const &geo, int prec, const void *U, 
 		int nb = nblk(geo.V, 256);
 		int gb = mesh_grid_blocks(ctx, nb);
 		if (prec == MESH_F64)
-			k_force_update_site<double><<<gb, 256, 0, ctx->stream>>>(geo, (const double *)U, (double *)P, k, nb,
-			                                                          ctx->xcd_remap);
+			k_force_update_site<double><<<gb, 256, 0, ctx->stream>>>(geo, (const double *)U, (double *)P, k,
+			                                                          block_order(geo, nb, 256, ctx->xcd_remap));
 		else
 			k_force_update_site<float><<<gb, 256, 0, ctx->stream>>>(geo, (const float *)U, (float *)P, k,
-			                                                         nb, ctx->xcd_remap);
+			                                                         block_order(geo, nb, 256, ctx->xcd_remap));
 		fused = false;
 	}
 	else
 	{
 		int nb = nblk(geo.V, SB);
 		int gb = mesh_grid_blocks(ctx, nb);
+		const BlockOrder ord = block_order(geo, nb, SB, mesh_order(ctx));
 		auto launch = [&](auto tag, auto path) {
 			using Rt = decltype(tag);
 			constexpr int PT = decltype(path)::value;
 			if (fused && compact)
 				k_force_update<Rt, true, true, PT><<<gb, 256, 0, ctx->stream>>>(
-				    geo, (const Rt *)U, (Rt *)P, k, nb, mesh_order(ctx), (Rt *)Unext, (Rt)tl, reunit_flag);
+				    geo, (const Rt *)U, (Rt *)P, k, ord, (Rt *)Unext, (Rt)tl, reunit_flag);
 			else if (fused)
 				k_force_update<Rt, true, false, PT><<<gb, 256, 0, ctx->stream>>>(
-				    geo, (const Rt *)U, (Rt *)P, k, nb, mesh_order(ctx), (Rt *)Unext, (Rt)tl, reunit_flag);
+				    geo, (const Rt *)U, (Rt *)P, k, ord, (Rt *)Unext, (Rt)tl, reunit_flag);
 			else
 				k_force_update<Rt, false, false, PT><<<gb, 256, 0, ctx->stream>>>(
-				    geo, (const Rt *)U, (Rt *)P, k, nb, mesh_order(ctx), nullptr, (Rt)0, 0);
+				    geo, (const Rt *)U, (Rt *)P, k, ord, nullptr, (Rt)0, 0);
 		};
 		auto by_path = [&](auto tag) {
 			switch (staple_path(geo))
@@ -1471,6 +1470,7 @@ int delta_h(mesh_ctx *ctx, Geo const &geo, int prec, const void *Uo, const void 
 		return rc;
 	int gb = mesh_grid_blocks(ctx, nb);
 	double c3 = beta / 3.0;
+	const BlockOrder ord = block_order(geo, nb, sbk, mesh_order(ctx));
 	int ph = mesh_prof_begin(ctx, PROF_DELTA_H);
 	auto launch = [&](auto tag, auto pc) {
 		using Rt = decltype(tag);
@@ -1479,10 +1479,10 @@ int delta_h(mesh_ctx *ctx, Geo const &geo, int prec, const void *Uo, const void 
 			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb);
 		else if (MESH_DH_SPLIT)
 			k_delta_h_split<Rt, decltype(pc)::value><<<gb, 256, 0, ctx->stream>>>(
-			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb, mesh_order(ctx));
+			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb, ord);
 		else
 			k_delta_h<Rt, decltype(pc)::value><<<gb, 256, 0, ctx->stream>>>(
-			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb, mesh_order(ctx));
+			    geo, (const Rt *)Uo, (const Rt *)Un, (const Rt *)P, Ko, c3, ctx->partials, nb, ord);
 	};
 	using PC1 = std::true_type;
 	using PC0 = std::false_type;
@@ -1984,9 +1984,11 @@ int mesh_su3_plaquette_noalloc(mesh_ctx *ctx, const mesh_grid *g, int prec, cons
 		return mesh_fail(ctx, MESH_E_STATE, "plaquette_noalloc: scratch address not resolved");
 	const int gb = mesh_grid_blocks(ctx, nb);
 	if (prec == MESH_F64)
-		k_plaq<double><<<gb, 256, 0, ctx->stream>>>(s.geo, (const double *)U, ctx->scratch, nb, mesh_order(ctx));
+		k_plaq<double><<<gb, 256, 0, ctx->stream>>>(s.geo, (const double *)U, ctx->scratch, nb,
+		                                            block_order(s.geo, nb, 256, mesh_order(ctx)));
 	else
-		k_plaq<float><<<gb, 256, 0, ctx->stream>>>(s.geo, (const float *)U, ctx->scratch, nb, mesh_order(ctx));
+		k_plaq<float><<<gb, 256, 0, ctx->stream>>>(s.geo, (const float *)U, ctx->scratch, nb,
+		                                           block_order(s.geo, nb, 256, mesh_order(ctx)));
 	MESH_LAUNCHED(ctx);
 	if (int rc = mesh_reduce_to_device(ctx, ctx->scratch, nb, out_dev))
 		return rc;

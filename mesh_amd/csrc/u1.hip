@@ -314,6 +314,7 @@ struct U1NGeo
 {
 	int nd, V;       // dimensions, sites
 	int L[4], st[4]; // extents, row-major strides (dimension 0 slowest)
+	mesh_dev::FastDiv by[4], by_V; // division by L, V
 };
 
 __device__ __forceinline__ int n_fwd(U1NGeo const &g, int x, int mu)
@@ -355,7 +356,7 @@ template <int ND> struct Nb
 #pragma unroll
 		for (int mu = ND - 1; mu >= 0; --mu)
 		{
-			const int rest = mu ? (int)((unsigned)r / (unsigned)g.L[mu]) : 0, c = r - rest * g.L[mu], st = g.st[mu];
+			const int rest = mu ? (int)g.by[mu]((unsigned)r) : 0, c = r - rest * g.L[mu], st = g.st[mu];
 			r = rest;
 			f[mu] = c + 1 == g.L[mu] ? x - c * st : x + st;
 			b[mu] = c == 0 ? x + (g.L[mu] - 1) * st : x - st;
@@ -373,7 +374,7 @@ __global__ __launch_bounds__(256) void k_u1n_start(U1NGeo g, int batch, const fl
 	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (long)batch * g.V)
 		return;
-	const int c = (int)((unsigned)i / (unsigned)g.V), x = (int)(i - (long)c * g.V);
+	const int c = (int)g.by_V((unsigned)i), x = (int)(i - (long)c * g.V);
 	const long o = (long)c * ND * g.V;
 	const float *t = th + o;
 	const Nb<ND> nb(g, x);
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(256) void k_u1n_step(U1NGeo g, int batch, const flo
 	long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= (long)batch * g.V)
 		return;
-	const int c = (int)((unsigned)i / (unsigned)g.V), x = (int)(i - (long)c * g.V);
+	const int c = (int)g.by_V((unsigned)i), x = (int)(i - (long)c * g.V);
 	const long o = (long)c * ND * g.V;
 	const float *t = in + o;
 	const Nb<ND> nb(g, x);
@@ -595,11 +596,13 @@ int u1n_setup(mesh_ctx *ctx, const mesh_grid *g, int batch, U1NGeo *ug)
 		return mesh_fail(ctx, MESH_E_SIZE, "U(1) batch x links exceeds 2^31");
 	ug->nd = g->nd;
 	ug->V = (int)V;
+	ug->by_V = mesh_dev::FastDiv((uint32_t)V);
 	int s = 1;
 	for (int i = g->nd - 1; i >= 0; --i)
 	{
 		ug->L[i] = g->dims[i];
 		ug->st[i] = s;
+		ug->by[i] = mesh_dev::FastDiv((uint32_t)g->dims[i]);
 		s *= g->dims[i];
 	}
 	for (int i = g->nd; i < 4; ++i)

@@ -25,7 +25,7 @@ int main()
 					site[block_slot(l)] = b0 + l;
 				for (int h = 0; h < 4; ++h)
 				{
-					site[64 + h] = halo_site(L3, b0, n, h);
+					site[64 + h] = halo_site(L3, FastDiv(L3), b0, n, h);
 					bad += site[64 + h] < 0 || site[64 + h] >= V;
 				}
 				for (int l = 0; l < n; ++l, ++count)

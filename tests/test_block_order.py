@@ -1,4 +1,4 @@
-"""The block orders of the stencil kernels (mesh_internal.h ordered_block_of):
+"""The block orders of the stencil kernels (mesh_internal.h block_order):
 each is a permutation of the blocks on every geometry it accepts.  Host only:
 the check is compiled with hipcc for the host."""
 import os
