@@ -125,19 +125,7 @@ inline int mesh_order(mesh_ctx *ctx) { return ctx->xcd_remap | (ctx->rb_tile << 
 
 namespace mesh_dev {
 
-// Workgroups are dispatched round-robin over the 8 XCDs of an MI355X.  With
-// remapping, XCD k processes the contiguous logical block range
-// [k*chunk, (k+1)*chunk), so lattice neighbours a few blocks apart share
-// that XCD's L2.
-__device__ __forceinline__ int logical_block(int nb, int remap)
-{
-	int b = blockIdx.x;
-	if (!remap)
-		return b;
-	int chunk = (nb + 7) >> 3;
-	return (b & 7) * chunk + (b >> 3);
-}
-
+// Workgroups are dispatched round-robin over the 8 XCDs of an MI355X.
 // Block order of the stencil kernels (sbk consecutive sites per workgroup,
 // i.e. one "row-block" rb of the x2/x3 plane), argument order | (T << 4):
 //   0: linear;  1: XCD-contiguous linear;

@@ -370,6 +370,116 @@ __global__ __launch_bounds__(256) void k_su2_force_link_rows(G2 g, const R *__re
 	stq(Unext, g, mu, x, un);
 }
 
+// A wavefront's access to the FP64 quaternions of one direction, all lanes
+// active, lane l at the l-th site of a block in the order site().  A quaternion is
+// 32 bytes, two loads, and with a lane a site each load takes half of every line
+// of a 2 KB span.  Here lanes 2k and 2k + 1 take sites k and 32 + k of the block,
+// in each of the two loads a pair reads one of its sites whole (neighbours of
+// consecutive sites are consecutive, a load spans 1 KB), and the lanes exchange
+// halves in registers.
+struct PairLanes
+{
+	typedef double half __attribute__((ext_vector_type(2)));
+	const int h; // which half of a quaternion the lane loads and stores
+	__device__ explicit PairLanes(int lane) : h(lane & 1) {}
+	static __device__ __forceinline__ int site(int lane) { return (lane & 1) << 5 | lane >> 1; }
+
+	// the other lane's value
+	static __device__ __forceinline__ int swap(int v) { return __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true); }
+	static __device__ __forceinline__ half swap(half v)
+	{
+		typedef int words __attribute__((ext_vector_type(4)));
+		const words w = __builtin_bit_cast(words, v);
+		return __builtin_bit_cast(half, words{swap(w.x), swap(w.y), swap(w.z), swap(w.w)});
+	}
+	// halves (of the pair's first site, of its second) <-> (first, second half) of the lane's own site
+	__device__ __forceinline__ void exchange(half &a, half &b) const
+	{
+		const half r = swap(h ? a : b);
+		a = h ? r : a;
+		b = h ? b : r;
+	}
+	__device__ __forceinline__ qt<double> load(const double *__restrict__ p, int x) const
+	{
+		const int y = swap(x);
+		half a = *reinterpret_cast<const half *>(p + 4u * (unsigned)(h ? y : x) + 2 * h);
+		half b = *reinterpret_cast<const half *>(p + 4u * (unsigned)(h ? x : y) + 2 * h);
+		exchange(a, b);
+		return {a.x, a.y, b.x, b.y};
+	}
+	__device__ __forceinline__ void store(double *__restrict__ p, int x, qt<double> const &q) const
+	{
+		const int y = swap(x);
+		half a = {q.w, q.x}, b = {q.y, q.z};
+		exchange(a, b);
+		*reinterpret_cast<half *>(p + 4u * (unsigned)(h ? y : x) + 2 * h) = a;
+		*reinterpret_cast<half *>(p + 4u * (unsigned)(h ? x : y) + 2 * h) = b;
+	}
+};
+
+// FP64 lattices whose U, P and U' (12 links of 32 bytes a site) exceed the 256 MB
+// last cache: there the step is held by its traffic and whole lines pay (fused
+// step 32^4 and 64 x 32 x 32 x 16 185 -> 176 us);
+// below it the exchange's instructions cost more (24 x 24 x 24 x 32, 170 MB,
+// 57 -> 59..61; 16^4 13.7 -> 14.5)
+inline bool pair_lanes(G2 const &g, int prec) { return prec == MESH_F64 && g.V * 12 * 32 > (256L << 20); }
+
+// k_su2_force_link_rows through PairLanes: the same products in the same order
+__global__ __launch_bounds__(256) void k_su2_force_link_pairs(G2 g, const double *__restrict__ U,
+                                                              double *__restrict__ P, double k,
+                                                              double *__restrict__ Unext, double t, int reunit,
+                                                              BlockOrder ord)
+{
+	using half = PairLanes::half;
+	__shared__ half own[4][2][64]; // halves apart: lanes at consecutive 16 bytes
+	const int lb = ord.at(blockIdx.x);
+	if (lb < 0)
+		return;
+	const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+	const PairLanes wv(lane);
+	const int o = PairLanes::site(lane), x = lb * 64 + o;
+	auto field = [&](auto *p, int f) { return p + 4 * (long)f * g.stride; };
+	{
+		const qt<double> q = wv.load(field(U, mu), x);
+		own[mu][0][o] = half{q.w, q.x};
+		own[mu][1][o] = half{q.y, q.z};
+	}
+	__syncthreads();
+	auto O = [&](int d, int s) {
+		const half a = own[d][0][s], b = own[d][1][s];
+		return qt<double>{a.x, a.y, b.x, b.y};
+	};
+	auto G = [&](int f, long y) { return wv.load(field(U, f), (int)y); };
+	const int L3 = g.L[3], c3 = o & (L3 - 1), o0 = o - c3;
+	const int sp = o0 + (c3 + 1 == L3 ? 0 : c3 + 1), sm = o0 + (c3 == 0 ? L3 - 1 : c3 - 1);
+	qt<double> S = {0.0, 0.0, 0.0, 0.0};
+	int c[4];
+	coords2(g, x, c);
+	const long xpm = shc(g, x, mu, mu == 0 ? c[0] : (mu == 1 ? c[1] : (mu == 2 ? c[2] : c[3])), 1);
+#pragma unroll
+	for (int nu = 0; nu < 4; ++nu)
+	{
+		if (nu == mu)
+			continue;
+		const long xpn = shc(g, x, nu, c[nu], 1), xmn = shc(g, x, nu, c[nu], -1), xpmmn = shc(g, xpm, nu, c[nu], -1);
+		const qt<double> a = mu == 3 ? O(nu, sp) : G(nu, xpm); // U_nu(x+mu)
+		const qt<double> b = nu == 3 ? O(mu, sp) : G(mu, xpn); // U_mu(x+nu)
+		qt<double> up = qmul(qmul(a, qconj(b)), qconj(O(nu, o)));
+		const qt<double> d = nu == 3 ? O(mu, sm) : G(mu, xmn); // U_mu(x-nu)
+		const qt<double> e = nu == 3 ? O(nu, sm) : G(nu, xmn); // U_nu(x-nu)
+		qt<double> lo = qmul(qmul(qconj(G(nu, xpmmn)), qconj(d)), e);
+		S = qadd(qadd(S, up), lo);
+	}
+	const qt<double> u = O(mu, o), M = qmul(u, S), p = wv.load(field(P, mu), x);
+	const qt<double> pn = {p.w, fma(-k, M.x, p.x), fma(-k, M.y, p.y), fma(-k, M.z, p.z)};
+	wv.store(field(P, mu), x, pn);
+	const qt<double> D = q_expm1(pn.x * t, pn.y * t, pn.z * t);
+	qt<double> un = qadd(u, qmul(D, u));
+	if (reunit)
+		un = q_reunit(un);
+	wv.store(field(Unext, mu), x, un);
+}
+
 // Uout = exp(t project_on_algebra(P)) Uin, as Uin + (exp - 1) Uin (+ reunitarisation)
 template <class R>
 __global__ __launch_bounds__(256) void k_su2_link_update(G2 g, int nf, R *Uout, const R *Uin, const R *__restrict__ P,
@@ -733,9 +843,14 @@ int launch_force_link(mesh_ctx *ctx, G2 const &g, int prec, const void *U, void 
 		using R = decltype(tag);
 		if (rows)
 		{
-			const int nb = (int)(g.V / 64);
-			k_su2_force_link_rows<R><<<mesh_grid_blocks(ctx, nb), 256, 0, ctx->stream>>>(
-			    g, as<R>(U), as<R>(P), k, as<R>(Unext), (R)t, reunit, block_order(g, nb, 64, mesh_order(ctx)));
+			const int nb = (int)(g.V / 64), gb = mesh_grid_blocks(ctx, nb);
+			const BlockOrder ord = block_order(g, nb, 64, mesh_order(ctx));
+			if (pair_lanes(g, prec))
+				k_su2_force_link_pairs<<<gb, 256, 0, ctx->stream>>>(g, as<double>(U), as<double>(P), k,
+				                                                    as<double>(Unext), t, reunit, ord);
+			else
+				k_su2_force_link_rows<R><<<gb, 256, 0, ctx->stream>>>(g, as<R>(U), as<R>(P), k, as<R>(Unext), (R)t,
+				                                                      reunit, ord);
 		}
 		else
 			k_su2_force_link<R><<<nblk(g.V * g.nd), 256, 0, ctx->stream>>>(g, as<R>(U), as<R>(P), k,

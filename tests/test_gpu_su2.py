@@ -149,6 +149,24 @@ def test_su2_fused_trajectory_same_bits(ctx, prec, nsub):
     np.testing.assert_array_equal(res[0][1], res[1][1])
 
 
+@pytest.mark.parametrize("sh", [(72, 72, 72, 2), (14, 31, 27, 64), (27, 30, 27, 32), (21, 26, 40, 32)])
+def test_su2_fused_large_same_bits(ctx, sh):
+    """FP64 fields beyond 256 MB (699051 sites on) pair their lanes in the fused
+    step, one below takes a lane a site: the unfused trajectory's bits"""
+    from conftest import options
+
+    d = gauge.makeDeltas("2mn", 0.5, 1)
+    res = []
+    for fuse in (0, 1):
+        h = S2.Hmc(mesh_amd.Grid(sh), F64, seed=33, ctx=ctx)
+        h.randomizeGaugeField()
+        with options(ctx, fuse_md=fuse):
+            r = h.runHmcUpdate(2.1, d, metropolis=False)
+        res.append((r["dH"], h.U.download()))
+    assert res[0][0] == res[1][0]
+    np.testing.assert_array_equal(res[0][1], res[1][1])
+
+
 def test_su2_misaligned_field_refused(ctx):
     g = mesh_amd.Grid([4, 4])
     f = S2.SU2Field(g, None, F64, ctx)
