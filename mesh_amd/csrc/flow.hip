@@ -155,7 +155,7 @@ __device__ __forceinline__ void layer_apply(FGeo const &g, float *th, int mu, in
 			const float tp = plaqf(g, th, y0, y1), u = wrapf(tp - p.t);
 			float v, Gp;
 			if (INV)
-				v = ncpq_inverse(p, u, Gp);
+				v = ncpq_inverse<false>(p, u, Gp);
 			else
 				ncpq_eval(p, u, v, Gp);
 			if ((l & 3) == 0)

@@ -546,12 +546,15 @@ __device__ __forceinline__ float quad_max(float v)
 // are uniform over it).  g is a convex combination of the increasing maps
 // g_k, so the root lies between the smallest and the largest closed-form
 // component inverse g_k^-1(target) = 2 atan2(sin(target/2), s_k cos(target/2))
-// (widened by a few ulps against their rounding); Newton starts from their
-// w-weighted mean and continues as ncp_inverse.  It also stops once
-// |g(u) - target| is at the rounding level of g (2.5e-7 max(1, |target|)):
-// where g' is small the residual is noise and further steps would only wander
-// inside the noise band (u is then as accurate as the output determines it).
-__device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float &Gp)
+// (widened by a few ulps against their rounding).  Newton starts from their
+// w-weighted mean; every evaluation moves one end of the bracket to the iterate,
+// a step that leaves the bracket is replaced by its midpoint, and a step or a
+// bracket below 2e-7 max(1, |u|) (an FP32 ulp of u is up to 2.4e-7) ends it, or 40
+// evaluations.  NEAR: it also stops at |g(u) - target| <= 2.5e-7 max(1, |target|).
+// Where |target| is well below 1 that is above g's rounding: on maps whose s_k are
+// all small u can be off by 5e-4 (s_k = e^-7.5) where the iteration reaches 5e-7,
+// so only the plaquette flow, which has always used it, does.
+template <bool NEAR> __device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float &Gp)
 {
 	float st, ct;
 	sincos1(0.5f * target, st, ct);
@@ -566,7 +569,7 @@ __device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float
 		ncpq_eval(p, u, G, Gp);
 		fresh = true;
 		float f = G - target;
-		if (fabsf(f) <= 2.5e-7f * fmaxf(1.f, fabsf(target)))
+		if (NEAR ? fabsf(f) <= 2.5e-7f * fmaxf(1.f, fabsf(target)) : f == 0.f)
 			break;
 		if (f < 0.f)
 			lo = u;

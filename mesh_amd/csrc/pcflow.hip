@@ -176,7 +176,7 @@ __device__ __forceinline__ void layer_apply(PCGeo const &g, LaneLoops const &ll,
 			const float a = FM::wrapf(phi[xs] - p.t);
 			float v, Gp;
 			if (INV)
-				v = FM::ncpq_inverse(p, a, Gp);
+				v = FM::ncpq_inverse<true>(p, a, Gp);
 			else
 				FM::ncpq_eval(p, a, v, Gp);
 			if ((l & 3) == 0)

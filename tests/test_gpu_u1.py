@@ -242,6 +242,50 @@ def test_flow_inverse_roundtrip(ctx):
     np.testing.assert_allclose(inv[:, 1], fwd[:, 1], rtol=1e-6)
 
 
+def _mixture_inverse(s, w, T):
+    """v and log g'(v) with g(v) = T in float64, g(v) = sum_k w_k 2 atan(s_k tan(v / 2)), by bisection"""
+    lo, hi = np.full_like(T, -np.pi), np.full_like(T, np.pi)
+
+    def g(v):
+        c, sn = np.cos(0.5 * v)[..., None], np.sin(0.5 * v)[..., None]
+        return (w * 2 * np.arctan2(s * sn, c)).sum(-1), np.log((w * s / (c * c + s * s * sn * sn)).sum(-1))
+
+    for _ in range(80):
+        mid = 0.5 * (lo + hi)
+        below = g(mid)[0] < T
+        lo, hi = np.where(below, mid, lo), np.where(below, hi, mid)
+    return 0.5 * (lo + hi), g(0.5 * (lo + hi))[1]
+
+
+def test_flow_inverse_of_small_slopes(ctx):
+    """one layer whose map has slopes s_k of 5e-4 .. 2e-3 whatever the context,
+    inverted at links that make the plaquettes exact in FP32: the moved link is
+    then v = g^-1(theta_P) itself.  Bound: the iteration's last step and v's own
+    rounding, 2e-7 + 1.2e-7 relative to max(1, |v|) <= 2.5, and four roundings of
+    g, 4 2^-24 g / g' with g / g' <= sin v <= 1: 1.1e-6."""
+    L, B = 8, 16
+    y = np.array([-7.5, -7.2, -6.8, -6.2, 0.3, 0.0, -0.2, 0.1, 1.0, 0.0], np.float32)
+    p = np.zeros(U.NP_LAYER, np.float32)
+    p[-U.NO:] = y
+    f = U1.Flow(L, L, ctx, layers=1)
+    f.set_params(p)
+    s, w = np.exp(y[:4].astype(np.float64)), np.exp(y[4:8].astype(np.float64))
+    w /= w.sum()
+    v = np.random.default_rng(7).uniform(-2.5, 2.5, (B, L, 2))
+    T = (w * 2 * np.arctan(s * np.tan(0.5 * v[..., None]))).sum(-1).astype(np.float32)
+    th = np.zeros((B, 2, L, L), np.float32)
+    th[:, 0, :, ::4] = T  # the first layer's active plaquettes: theta_0 of every fourth column
+    ens = U1.U1Ensemble(L, L, B, ctx)
+    ens.set_angles(th)
+    z = U1.Buffer(B * 2 * L * L, np.float32, ctx)
+    out = f.logq(ens, z_out=z).download().reshape(B, 2)
+    ref, lg = _mixture_inverse(s, w, T.astype(np.float64))
+    got = z.download().reshape(th.shape)
+    assert np.abs(got[:, 0, :, ::4] - ref).max() < 1.1e-6
+    # d log g' / dv = tan(v / 2) <= 3 there, over 16 links, and the logs' own rounding
+    np.testing.assert_allclose(out[:, 0], U.log_prior(L, L) - lg.sum((1, 2)), atol=16 * (3 * 1.1e-6 + 1e-6))
+
+
 def test_flow_gradient_against_autograd(ctx):
     """mesh_flow_gradient against torch float64 autograd of
     mean(beta S(f(z)) - log det f'(z)) on the same prior draws."""
