@@ -491,6 +491,32 @@ def test_pflow_edges(ctx, L0, L1, scale):
         assert out[c, 1] == pytest.approx(S, rel=1e-5)
 
 
+def test_pflow_inverse_of_steep_and_shallow(ctx):
+    """a map whose slope changes by e^10 within a degree of v = 0, at links that
+    make the plaquettes exact in FP32 (one link of a 2 x 2 lattice moved: plaquettes
+    a, -a, 0): log q against bisection in float64, over targets g(v) of v = -2.6 ..
+    2.6.  The iteration run to its end has an error of 1.5e-7 rms and 8e-7 at most a
+    plaquette (the parameters' and g's roundings); the bounds are four times that,
+    over three plaquettes and log q's offset."""
+    y = np.array([-4.6, -3.05, -2.35, -4.65, -5.25, 5.55, -5.7, 3.95, -1.1, 0.3, -4.5, -0.4, 6.1, -1.55, -0.4, -0.9,
+                  1.0, 0.0], np.float32)
+    s, w = np.exp(y[:8].astype(np.float64)), np.exp(y[8:16].astype(np.float64))
+    w /= w.sum()
+    v = np.linspace(-2.6, 2.6, 512)
+    T = (w * 2 * np.arctan(s * np.tan(0.5 * v[:, None]))).sum(-1).astype(np.float32)
+    th = np.zeros((len(T), 2, 2, 2), np.float32)
+    th[:, 0, 0, 0] = T
+    f = U1.PlaqFlow(2, 2, ctx)
+    f.set_params(y)
+    ens = U1.U1Ensemble(2, 2, len(T), ctx)
+    ens.set_angles(th)
+    out = f.logq(ens).download().reshape(-1, 2)
+    T = T.astype(np.float64)
+    err = out[:, 0] - U.log_prior(2, 2) + sum(_mixture_inverse(s, w, a)[1] for a in (T, -T, 0 * T))
+    assert np.sqrt(np.mean(err ** 2)) < 3 * 6e-7
+    assert np.abs(err).max() < 3 * 3.2e-6
+
+
 def test_pflow_propose(ctx):
     """mesh_pflow_propose: the states' (log q, S/beta) are mesh_pflow_logq's
     bit for bit, the proposals mesh_pflow_sample's, and the proposals' log q
