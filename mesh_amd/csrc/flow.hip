@@ -99,6 +99,8 @@ __device__ __forceinline__ int updated_link(FGeo const &g, int mu, int y0, int y
 // rows: the cosine (q even) or sine of frozen neighbour 2 s + q / 2.
 __device__ __forceinline__ int feature_row(int q, int s) { return 4 * s + q; }
 
+// ANY: the links may be the caller's, not wrapped.
+template <bool ANY = false>
 __device__ __forceinline__ void features(FGeo const &g, const float *t, int mu, int a, int r, float (&x)[NI / 4])
 {
 	const int q = (threadIdx.x >> 4) & 3;
@@ -110,7 +112,8 @@ __device__ __forceinline__ void features(FGeo const &g, const float *t, int mu, 
 		int z0, z1;
 		frozen_corner(mu, 2 * s + (q >> 1), y0, y1, z0, z1);
 		float sn, cs;
-		sincos1(plaqf(g, t, z0, z1), sn, cs);
+		const float p = plaqf(g, t, z0, z1);
+		ANY ? sincos_any(p, sn, cs) : sincos1(p, sn, cs);
 		x[s] = (q & 1) ? sn : cs;
 	}
 }
@@ -142,7 +145,7 @@ __device__ __forceinline__ void layer_apply(FGeo const &g, float *th, int mu, in
 	for (int tix = w; tix < ntile; tix += THREADS / 64)
 	{
 		float x[NI / 4];
-		features(g, th, mu, a, min(tix * 16 + (l & 15), g.NA - 1), x);
+		features<INV>(g, th, mu, a, min(tix * 16 + (l & 15), g.NA - 1), x);
 		f4 h1[4], h2[4];
 		put_outputs(y, mlp_rows<NI, false>(sh.lw, x, [&](int s) { return feature_row(q, s); }, h1, h2));
 		wave_sync();

@@ -286,12 +286,12 @@ __device__ __forceinline__ void pc_inverse(PCGeo const &g, int nl, const float *
 	{
 		const int x0 = x / g.L1, x1 = x - x0 * g.L1;
 		const float tp = plaqp(g, th, x0, x1);
-		v[1] += 1.0 - cos1((double)tp);
+		v[1] += 1.0 - cos_any((double)tp);
 		phi[x] = x < g.V - 1 ? FM::wrapf(tp) : 0.f;
 	}
 	__syncthreads(); // the links are read; cs takes their place
 	for (int x = threadIdx.x; x < g.V; x += NT)
-		cs[x] = sincos2(phi[x]);
+		sincos_any(phi[x], cs[x].y, cs[x].x);
 	for (int layer = nl - 1; layer >= 0; --layer)
 	{
 		__syncthreads();

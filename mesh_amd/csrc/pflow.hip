@@ -277,7 +277,7 @@ __device__ void pflow_logq(PGeo const &g, const float *__restrict__ params, cons
 	{
 		int x0 = x / g.L1, x1 = x - x0 * g.L1;
 		float tp = plaqp(g, t, x0, x1);
-		v[1] += 1.0 - cos1((double)tp);
+		v[1] += 1.0 - cos_any((double)tp);
 		if (x < g.V - 1)
 		{
 			float Gp;

@@ -1,5 +1,6 @@
 // Sine, cosine, arctangent and quotient for the ranges that the U(1) kernels
-// meet: angles of a few turns at most and finite, non-zero quotients.
+// meet: angles of a few turns at most and finite, non-zero quotients (the functions
+// named any: those of a caller's links, which need not be wrapped).
 //
 // These kernels are held by vector instructions, and the library's functions
 // carry the reduction of huge arguments, infinities and zeros: sincosf and
@@ -65,6 +66,15 @@ TD void sincos1(float x, float &sn, float &cs)
 	sn = flip(odd ? c : s, (unsigned)i >> 1 & 1);
 	cs = flip(odd ? s : c, (unsigned)(i + 1) >> 1 & 1);
 }
+// sin and cos of any x: a caller's angle may be anything, and beyond some 10^7 the
+// reduction above leaves no angle at all
+TD void sincos_any(float x, float &sn, float &cs)
+{
+	if (fabsf(x) < 32768.f)
+		sincos1(x, sn, cs);
+	else
+		sn = sinf(x), cs = cosf(x);
+}
 // atan2(y, x) for finite arguments, the larger of them a normal number whose
 // reciprocal is one too
 TD float atan2_1(float y, float x)
@@ -87,7 +97,7 @@ TD float atan2_1(float y, float x)
 	return copysignf(k + t, y);
 }
 
-// cos for |x| up to a few turns, FP64
+// cos for |x| < 10^9, FP64
 TD double cos1(double x)
 {
 	const double q = rint(x * 0.63661977236758134308);
@@ -112,6 +122,8 @@ TD double cos1(double x)
 	const double v = i & 1 ? s : c;
 	return (i + 1) & 2 ? -v : v;
 }
+// cos of any x, FP64
+TD double cos_any(double x) { return fabs(x) < 1e9 ? cos1(x) : cos(x); }
 
 #undef TD
 

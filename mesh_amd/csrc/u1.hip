@@ -223,7 +223,7 @@ __global__ __launch_bounds__(1024) void k_u1_hmc(U1Geo g, float *th, const doubl
 		if ((int)(threadIdx.x + k * blockDim.x) >= g.V)
 			break;
 		const double kin = (double)q0[k] * q0[k] + (double)q1[k] * q1[k];
-		v[2] += beta * (1.0 - cos1((double)angle(k))) + kin;
+		v[2] += beta * (1.0 - cos_any((double)angle(k))) + kin;
 	}
 	// every wave has read the start angles before the first link step moves them
 	__syncthreads();
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(1024) void k_u1_hmc(U1Geo g, float *th, const doubl
 		if ((int)(threadIdx.x + k * blockDim.x) >= g.V)
 			break;
 		const double kin = (double)q0[k] * q0[k] + (double)q1[k] * q1[k];
-		const double sn = 1.0 - cos1((double)angle(k));
+		const double sn = 1.0 - cos_any((double)angle(k));
 		v[0] += beta * sn + kin;
 		v[1] += sn;
 	}
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(256) void k_u1n_start(U1NGeo g, int batch, const fl
 		for (int nu = mu + 1; nu < ND; ++nu)
 		{
 			const float p = tx[mu] + t[nu * g.V + nb.f[mu]] - t[mu * g.V + nb.f[nu]] - tx[nu];
-			e += beta * (1.0 - cos1((double)p));
+			e += beta * (1.0 - cos_any((double)p));
 		}
 #pragma unroll
 	for (int mu = 0; mu < ND; ++mu)
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(256) void k_u1n_energy(U1NGeo g, int nbk, const flo
 			{
 				const float p =
 				    t[mu * g.V + x] + t[nu * g.V + nb.f[mu]] - t[mu * g.V + nb.f[nu]] - t[nu * g.V + x];
-				sn += 1.0 - cos1((double)p);
+				sn += 1.0 - cos_any((double)p);
 			}
 #pragma unroll
 		for (int mu = 0; mu < ND; ++mu)

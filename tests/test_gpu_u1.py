@@ -517,6 +517,36 @@ def test_pflow_inverse_of_steep_and_shallow(ctx):
     assert np.abs(err).max() < 3 * 3.2e-6
 
 
+def _plaq32(th):
+    """plaquette angles summed in FP32, left to right as the kernels do"""
+    return ((th[:, 0] + np.roll(th[:, 1], -1, axis=1)) - np.roll(th[:, 0], -1, axis=2)) - th[:, 1]
+
+
+@pytest.mark.parametrize("mag", [3e3, 3e7, 3e10, 1e30])
+@pytest.mark.parametrize("L0,L1", [(8, 8), (68, 64)])
+def test_u1_angles_of_many_turns(ctx, L0, L1, mag):
+    """links need not be wrapped: the actions that HMC and the flows report are those
+    of the angles they are given, however large (the cosine of the FP32 plaquette sums
+    in float64; a sum of L0 L1 terms in another order)"""
+    B, beta = 2, 1.0
+    th = (np.random.default_rng(71).uniform(-1, 1, (B, 2, L0, L1)) * mag).astype(np.float32)
+    S = (1 - np.cos(_plaq32(th).astype(np.float64))).sum((1, 2))
+    tol = dict(rtol=1e-12, atol=1e-9)
+    ens = U1.U1Ensemble(L0, L1, B, ctx)
+    if L0 * L1 <= 4096:
+        for f in (U1.Flow(L0, L1, ctx), U1.PlaqFlow(L0, L1, ctx), U1.PlaqCouplingFlow(L0, L1, ctx)):
+            ens.set_angles(th)
+            out = f.logq(ens).download().reshape(B, 2)
+            np.testing.assert_allclose(out[:, 1], S, **tol)
+            assert np.isfinite(out[:, 0]).all()
+    # a trajectory of one link step of no length: only the wrapping moves the angles
+    ens.set_angles(th)
+    r = ens.hmc(beta, [0.0], 72, 0, metropolis=False)
+    new = (1 - np.cos(_plaq32(ens.angles()).astype(np.float64))).sum((1, 2))
+    np.testing.assert_allclose(r["S"], new, **tol)
+    np.testing.assert_allclose(r["dH"], beta * (new - S), rtol=1e-10, atol=1e-8)
+
+
 def test_pflow_propose(ctx):
     """mesh_pflow_propose: the states' (log q, S/beta) are mesh_pflow_logq's
     bit for bit, the proposals mesh_pflow_sample's, and the proposals' log q
