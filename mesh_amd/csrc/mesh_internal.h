@@ -143,18 +143,16 @@ namespace mesh_dev {
 //      not divide L0.
 // Where a plane is no whole number of blocks, or the extents allow neither,
 // orders 3 and 4 give XCD k the k-th eighth of the blocks in memory order, about
-// L0/8 slices of x0, walked side by side (slice fastest, then the position in
-// the slice), so the x0-neighbours of a workgroup are the launches before and
-// after it, to within a block -- if a slice has more than 128 blocks: below
-// that an XCD has the x0-neighbours in flight in memory order as well
-// (18x15x20x22, 103 blocks: 83 us a fused step in memory order, 85 so; 36^4,
-// 729 blocks: 1109 and 1053 us; 44^4 2536 and 2344; 40^4, whose planes of 25
-// blocks take tiles of 5 in order 3, 1740 and 1485).
+// L0/8 slices of x0, and walk it as the kernel asks (Walk): in memory order, with
+// the slices side by side (slice fastest, then the position in the slice, so the
+// x0-neighbours of a workgroup are the launches before and after it, to within a
+// block), or, where planes are whole blocks, in order 2.
 // Returns the memory-order block index (-1: padding workgroup).  The order
 // only permutes workgroups; every site's arithmetic is unchanged.  GEO: any
 // geometry with nd and L[4] (the SU(3) and SU(2) ones).
 // the row-blocks of a tile of orders 3 and 4: the divisor of nb2 (row-blocks of
-// a plane) nearest below or just above the one asked for
+// a plane) nearest below or just above the one asked for (fused step FP64 40^4, whose
+// planes of 25 blocks take 5: 1740 us in memory order, 1485)
 inline int tile_of(int nb2, int t)
 {
 	if (nb2 % t == 0)
@@ -225,7 +223,46 @@ struct BlockOrder
 	}
 };
 
-template <class GEO> inline BlockOrder block_order(GEO const &g, int nb, int sbk, int arg)
+// how orders 3 and 4 walk a lattice that allows neither: slices side by side if a
+// slice has at least `side` blocks and an XCD `slices` of them; else order 2 if
+// `cache` and planes are whole blocks, else memory order
+struct Walk
+{
+	int side = 129, slices = 1;
+	bool cache = false;
+};
+// (measured on lattices with and without whole planes, a slice of 60 to 1,700
+// blocks, an XCD of less than one to six slices)
+//
+// SU(3) fused step.  FP64: side by side from 300 blocks a slice (28^4, 343 blocks:
+// 396 -> 383 us; 36^4, 729: 1121 -> 1059; 44^4 2558 -> 2355; 26^4, 274: 299 -> 304;
+// 30x24^3, 216: 245 -> 250); below that, or with fewer than two slices an XCD, order 2
+// if a block holds two rows or more (18x16^3 46.6 -> 44.0 us, 18x8x32x32 89.2 -> 84.4,
+// 30x32x32x16 285 -> 273, 6x32^3 114.8 -> 111.4; 22x16x16x64, whose blocks are single
+// rows, 208 -> 216 us, and 18x24^3, whose rows cross the blocks, 147 -> 153).  FP32,
+// with four workgroups a CU and half the bytes, has a slice's neighbours in its L2 for
+// longer: side by side from 600 blocks and four slices (36^4 657 -> 633 us, 38^4 976
+// -> 921; 34^4, 614, even; 28^4, 343: 223 -> 226; 18x36^3, two slices: 297 -> 309),
+// order 2 nowhere (18x32^3 197 -> 200 us, 6x32^3 67.5 -> 71.1).
+template <class GEO> inline Walk fused_walk(GEO const &g, bool f64)
+{
+	if (!f64)
+		return {601, 4, false};
+	return {301, 2, g.L[3] <= 32 && 64 % g.L[3] == 0};
+}
+// SU(3) Delta H (blocks of 128 sites).  FP64 reads two fields and leaves its slices
+// in memory order (side by side 36^4 974 -> 1038 us, 38^4 1288 -> 1345); order 2 with
+// fewer than three slices an XCD (6x32^3 127 -> 120 us, 18x32x32x16 181 -> 173;
+// 30x32^3 561 -> 597).  FP32 walks them side by side (36^4 541 -> 513 us, 44^4 1177
+// -> 1119, 30x32^3 311 -> 290).
+template <class GEO> inline Walk delta_h_walk(GEO const &g, bool f64)
+{
+	if (!f64)
+		return {};
+	return {1 << 30, 1, g.L[0] < 24 && g.L[3] <= 32 && 64 % g.L[3] == 0};
+}
+
+template <class GEO> inline BlockOrder block_order(GEO const &g, int nb, int sbk, int arg, Walk walk = {})
 {
 	BlockOrder o;
 	const int order = arg & 15;
@@ -249,16 +286,18 @@ template <class GEO> inline BlockOrder block_order(GEO const &g, int nb, int sbk
 		return o;
 	}
 	o.chunk = (nb + 7) >> 3;
-	o.kind = order == 2 && planes ? BlockOrder::CACHE : BlockOrder::CHUNK;
-	if (o.kind == BlockOrder::CACHE)
+	o.kind = BlockOrder::CHUNK;
+	const int slice = g.nd == 4 ? nb / g.L[0] : 0;
+	if (order >= 3 && slice >= walk.side && o.chunk >= walk.slices * slice)
 	{
+		o.S = slice;
+		o.by_a = FastDiv(o.S);
+	}
+	else if (planes && (order == 2 || (order >= 3 && walk.cache)))
+	{
+		o.kind = BlockOrder::CACHE;
 		o.X = g.L[0];
 		o.by_a = FastDiv(g.L[0]), o.by_b = FastDiv(g.L[1]);
-	}
-	else if (order >= 3 && g.nd == 4 && nb / g.L[0] > 128)
-	{
-		o.S = nb / g.L[0];
-		o.by_a = FastDiv(o.S);
 	}
 	return o;
 }

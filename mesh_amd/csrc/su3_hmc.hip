@@ -1320,7 +1320,7 @@ int launch_force_update(mesh_ctx *ctx, Geo const &geo, int prec, const void *U, 
 	{
 		int nb = nblk(geo.V, SB);
 		int gb = mesh_grid_blocks(ctx, nb);
-		const BlockOrder ord = block_order(geo, nb, SB, mesh_order(ctx));
+		const BlockOrder ord = block_order(geo, nb, SB, mesh_order(ctx), fused_walk(geo, prec == MESH_F64));
 		auto launch = [&](auto tag, auto path) {
 			using Rt = decltype(tag);
 			constexpr int PT = decltype(path)::value;
@@ -1473,7 +1473,7 @@ int delta_h(mesh_ctx *ctx, Geo const &geo, int prec, const void *Uo, const void 
 	// FP64: half the tile, its two fields being twice the bytes in the L2 (32^4 575
 	// -> 529 us, 48^4 3030 -> 2820, 40^4 and 24^4 even; FP32 48^4 1503 -> 1554)
 	const int tile = prec == MESH_F64 && ctx->rb_tile > 1 ? ctx->rb_tile / 2 : ctx->rb_tile;
-	const BlockOrder ord = block_order(geo, nb, sbk, ctx->xcd_remap | (tile << 4));
+	const BlockOrder ord = block_order(geo, nb, sbk, ctx->xcd_remap | (tile << 4), delta_h_walk(geo, prec == MESH_F64));
 	int ph = mesh_prof_begin(ctx, PROF_DELTA_H);
 	auto launch = [&](auto tag, auto pc) {
 		using Rt = decltype(tag);
