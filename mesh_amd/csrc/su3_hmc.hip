@@ -24,11 +24,20 @@ using namespace mesh_dev;
 #define MESH_PIPE_F64 1
 #endif
 // The global operands of the shared upper-staple factors loaded before the
-// staging barrier (share_fetch; same bits) instead of after it: in FP64 on the
-// rows path, 32^4 568.5 -> 566.5 us.  With the halo slots it loses (FP64 36^4
-// 1045 -> 1087, 48^4 3047 -> 3162), and in FP32 the four workgroups of a CU cover
-// the latency (32^4 341.7 -> 343.2).
-template <class R, bool ROWS> constexpr bool share_prefetch() { return ROWS && std::is_same<R, double>::value; }
+// staging barrier on the rows path (share_fetch; same bits) instead of after it,
+// FP32 / FP64: in FP64 32^4 568.5 -> 566.5 us; in FP32 the four workgroups of a CU
+// cover the latency (32^4 341.7 -> 343.2).  With the halo slots it loses (FP64 36^4
+// 1045 -> 1087, 48^4 3047 -> 3162) and is never done.
+#ifndef MESH_SHARE_PREFETCH
+#define MESH_SHARE_PREFETCH 0
+#endif
+#ifndef MESH_SHARE_PREFETCH_F64
+#define MESH_SHARE_PREFETCH_F64 1
+#endif
+template <class R, bool ROWS> constexpr bool share_prefetch()
+{
+	return ROWS && (std::is_same<R, double>::value ? MESH_SHARE_PREFETCH_F64 : MESH_SHARE_PREFETCH) != 0;
+}
 // waves per SIMD the force kernels are compiled for (0: the compiler's choice)
 #ifndef MESH_FORCE_WAVES
 #define MESH_FORCE_WAVES 0
@@ -117,7 +126,7 @@ constexpr long DH_PLANES_V = 64 * 256;
 #else
 #define DH_OCC
 #endif
-// staples with the direction as a compile-time constant (4-d lattices)
+// fused tile variant: the direction as a compile-time constant
 #ifndef MESH_STATIC_MU
 #define MESH_STATIC_MU 1
 #endif
@@ -830,9 +839,8 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 		// stage the block's links, then the staples read them from LDS
 		constexpr bool RW = PATH == STAPLE_ROWS;
 		constexpr int SH = share_mode<R>(), NS = RW ? 64 : 68;
-		static_assert(SH > 0, "the staged kernels share the planes' upper factors");
 		__shared__ vec2_t<R> own[4][9][NS];
-		__shared__ vec2_t<R> sh[shared_planes(SH)][9][64];
+		__shared__ vec2_t<R> sh[SH > 0 ? shared_planes(SH) : 1][9][64];
 		const long b0 = (long)lb * SB;
 		const int n = RW || g.V - b0 >= SB ? SB : (int)(g.V - b0);
 		if (n < SB)
@@ -871,7 +879,7 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 #define MESH_STAPLE(M)                                                                             \
 	S = PIPE ? staple_pipe<M, RW, SH>(g, U, x, c, own, at, lane, sh)                               \
 	         : staple_4d_own<M, RW, SH>(g, U, x, c, own, at, lane, sh)
-		if constexpr (PF)
+		if constexpr (SH > 0 && PF)
 			MESH_BY_DIRECTION(MESH_FETCH)
 		{
 			const vec2_t<R> *p = reinterpret_cast<const vec2_t<R> *>(U) + site_off(g, mu, x);
@@ -887,10 +895,13 @@ __attribute__((amdgpu_waves_per_eu(force_min_waves<R, PATH>(), force_max_waves<R
 				    U)[site_off(g, d, halo_site(g.L[3], g.by[3], b0, n, h)) + k * plane_step(g)];
 			}
 		__syncthreads();
-		if constexpr (!PF)
-			MESH_BY_DIRECTION(MESH_FETCH)
-		MESH_BY_DIRECTION(MESH_SHARE)
-		__syncthreads();
+		if constexpr (SH > 0)
+		{
+			if constexpr (!PF)
+				MESH_BY_DIRECTION(MESH_FETCH)
+			MESH_BY_DIRECTION(MESH_SHARE)
+			__syncthreads();
+		}
 		MESH_BY_DIRECTION(MESH_STAPLE)
 #undef MESH_FETCH
 #undef MESH_SHARE
