@@ -89,6 +89,12 @@ template <int NI> struct alignas(16) LWP
 	float w1[NI * WS], b1[NH], w2[NH * WS], b2[NH], w3[NH * W3S], b3[16];
 };
 
+// two floats of memory that is aligned for one
+struct __attribute__((packed, aligned(4))) Pair
+{
+	float x, y;
+};
+
 // One layer's parameters held in registers (two floats a lane per chunk, from
 // 4-byte aligned memory) so that the next layer's global loads overlap the
 // current layer's work.  store() writes the LDS image (the pad columns of
@@ -101,10 +107,6 @@ template <int NI, int THREADS> struct WeightRegsP
 	              "pairs of parameters");
 	static constexpr int NC = Y::NP / 2;
 	static constexpr int PER = (NC + THREADS - 1) / THREADS;
-	struct __attribute__((packed, aligned(4))) Pair
-	{
-		float x, y;
-	};
 	Pair v[PER];
 
 	__device__ void load(const float *__restrict__ p)

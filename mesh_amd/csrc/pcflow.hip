@@ -436,8 +436,8 @@ __global__ __launch_bounds__(THREADS) void k_pc_backward(PCGeo g, int nl, const 
 				e[k] = fmaf(x[2 * k], dx[(2 * k + 1) / 4][(2 * k + 1) & 3], -x[2 * k + 1] * dx[2 * k / 4][(2 * k) & 3]);
 			const float from_next = __shfl(e[3] + e[4], (l + 16) & 63, 64);
 			if (r < NA)
-				*reinterpret_cast<float2 *>(dr + r * 8 + 2 * ll.q) =
-				    make_float2(e[0] + e[2] + e[3] + e[4], e[1] + e[2] + e[4] + from_next);
+				*reinterpret_cast<FM::Pair *>(dr + r * 8 + 2 * ll.q) = // (the caller's workspace)
+				    FM::Pair{e[0] + e[2] + e[3] + e[4], e[1] + e[2] + e[4] + from_next};
 		}
 		__syncthreads();
 		FM::store_grad<NI>(gr, row, part + (long)layer * NP_LAYER);

@@ -3,6 +3,7 @@ float64 oracle: identity initialisation, samples and log q of the forward
 map, log q of given configurations by the inverse, gauge invariance, the
 reverse-KL gradient against autograd, and training against the exact
 free-energy bound with MH chains reproducing the exact torus <cos theta_P>."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -269,6 +270,20 @@ def test_pcflow_gradient_tile_edges(ctx, L0, L1, B, nl):
     for layer in range(nl):
         sl = slice(layer * U.PC_NP_LAYER, (layer + 1) * U.PC_NP_LAYER)
         assert np.linalg.norm(g[sl] - gr[sl]) <= 2e-3 * np.linalg.norm(gr[sl]) + 1e-6, layer
+
+
+def test_pcflow_gradient_workspace_offset(ctx):
+    """the workspace holds floats and needs no more than their alignment: the same
+    gradient bit for bit from one that starts 4 bytes into an allocation"""
+    L0, L1, B = 8, 10, 3
+    f = U1.PlaqCouplingFlow(L0, L1, ctx)
+    f.set_params(_params(33, 0.2))
+    f.gradient(B, 2.0, 34, 1)
+    ref = f.grad.download()
+    ws, out = U1.Buffer(f._workspace(B).n + 16, np.uint8, ctx), U1.Buffer(2 * B, np.float64, ctx)
+    ctx.call("mesh_pcflow_gradient", f.grid.ref, B, f.layers, f.params.ptr, C.c_uint64(34), C.c_uint32(1),
+             C.c_double(2.0), C.c_void_p(ws.ptr.value + 4), f.grad.ptr, out.ptr)
+    np.testing.assert_array_equal(f.grad.download(), ref)
 
 
 def test_pcflow_deeper_stack(ctx):
