@@ -230,6 +230,8 @@ int mesh_ctx_create(mesh_ctx **out, int device)
 	if (hipHostMalloc(&ctx->red_host, RED_MAX_Q * sizeof(double), hipHostMallocMapped) != hipSuccess ||
 	    hipHostGetDevicePointer((void **)&ctx->red_out, ctx->red_host, 0) != hipSuccess)
 	{
+		if (ctx->red_host)
+			(void)hipHostFree(ctx->red_host);
 		(void)hipStreamDestroy(ctx->stream);
 		delete ctx;
 		return MESH_E_ALLOC;

@@ -84,6 +84,27 @@ def test_context_creation_without_gpu_fails_cleanly():
     assert not h.value
 
 
+def test_failed_context_creation_gives_everything_back(tmp_path):
+    """pinned memory without a device address: no context, no stream or pinned memory left
+    (in a process of its own, on a stand-in for the runtime)"""
+    import subprocess
+    import sys
+
+    so = str(tmp_path / "failing_runtime.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-Wall", os.path.join(ROOT, "tests", "failing_runtime.c"), "-o", so],
+                   check=True, timeout=60)
+    code = f"""
+import ctypes as C
+r = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
+L = C.CDLL({_lib.LIB_PATH!r})
+h = C.c_void_p()
+rc = L.mesh_ctx_create(C.byref(h), 0)
+print(rc, h.value, C.c_int.in_dll(r, "live_streams").value, C.c_int.in_dll(r, "live_pinned").value)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.stdout.split() == [str(_lib.MESH_E_ALLOC), "None", "0", "0"], r.stdout + r.stderr
+
+
 def test_cpp_programs_built_and_reject_bad_options():
     import subprocess
 
