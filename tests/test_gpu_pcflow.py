@@ -119,6 +119,37 @@ def test_pcflow_tile_edges(ctx, L0, L1):
     np.testing.assert_allclose(inv[:, 0], out[:, 0], atol=tol)
 
 
+def _to_16_bits(p):
+    """weights rounded to 16 bits of mantissa, two BF16 numbers' worth"""
+    b = p.view(np.uint32).astype(np.uint64)
+    return (((b + 0x80) >> 8) << 8).astype(np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("L0,L1", [(8, 8), (10, 50), (32, 32)])
+def test_pcflow_products_hold_32_bits(ctx, L0, L1):
+    """the products of numbers split in three keep FP32's precision: over eight layers
+    the median error of a plaquette is a few ulps of an angle (measured 2.2e-7 ..
+    3.4e-7; the largest, 5e-6 .. 4e-5, sits where the map is steep and says little), the
+    bound three times that, forward and inverse; the oracle with weights of 16 bits is
+    at 4e-6 and more, so a lost third part or product does not pass"""
+    torch = pytest.importorskip("torch")
+    B, seed, step, V = 2, 17, 3, L0 * L1
+    z = np.stack([U.pcflow_draws(seed, step, c, L0, L1)[0] for c in range(B)]).astype(np.float64)
+    for k in (18, 19):
+        p = _params(k, 0.2)
+        f = U1.PlaqCouplingFlow(L0, L1, ctx)
+        f.set_params(p)
+        ens = U1.U1Ensemble(L0, L1, B, ctx)
+        f.sample(ens, seed, step)
+        ref, low = (U.pcflow_forward(torch.tensor(w.astype(np.float64)), torch.tensor(z), L0, L1)[0].numpy()
+                    for w in (p, _to_16_bits(p)))
+        assert np.median(_wrapdiff(_free_plaquettes(ens.angles()), ref)) < 1e-6
+        assert np.median(_wrapdiff(low, ref)) > 4e-6
+        z_out = U1.Buffer(B * V, np.float32, ctx)
+        f.logq(ens, z_out=z_out)
+        assert np.median(_wrapdiff(z_out.download().reshape(B, V)[:, :-1], z)) < 1e-6
+
+
 @pytest.mark.parametrize("L0,L1", [(4, 128), (24, 24), (26, 64), (28, 60)])
 def test_pcflow_width_by_batch(ctx, L0, L1):
     """more workgroups than CUs run on 256 threads up to 1664 plaquettes: the
