@@ -6,9 +6,10 @@
 //   h(a) = g(wrap(a - t)) + t,  g(u) = sum_k w_k 2 atan(s_k tan(u / 2))
 // (a mixture of NK = 4 non-compact projections; s_k = exp(clamp(y_k, -8, 8)),
 // w = softmax(y_{4..7}), t = atan2(y_9, y_8)).  The dense layers run on FP32
-// MFMA (v_mfma_f32_16x16x4_f32) in 16-row tiles, one tile per wavefront, with
-// the activations in registers; the backward pass forms the weight gradients
-// as MFMA products over the rows of four tiles.
+// MFMA (v_mfma_f32_16x16x4_f32), or on BF16 MFMA with every number split in three,
+// in 16-row tiles, one tile per wavefront, with the activations in registers; the
+// backward pass forms the weight gradients as MFMA products over the rows of four
+// tiles.
 //
 // Parameters of one layer, in order: W1 [NI][64], b1 [64], W2 [64][64],
 // b2 [64], W3 [64][10], b3 [10].
@@ -271,9 +272,10 @@ __device__ __forceinline__ f4 mlp_rows(LWP<NI> const &lw, const float (&x)[NI / 
 // with signs hold all 24), and of the nine products of two such sums the six
 // that reach FP32's rounding are formed and accumulated in FP32: the three
 // left out are below 2^-24 of the product.  Against 64 bits, 32 seeds of 64
-// chains: links of a 32^2 proposal 7.2e-7 on FP32 MFMA, 7.2e-7 here, its log q
-// 2.9e-9 and 3.3e-9 (1.4e-8 with layers and tails in separate passes).
-// 32^2 propose, 256 chains: 209 -> 159 us; 64^2: 872 -> 615.
+// chains of a 32^2 proposal round: links 7.0e-7, log q 1.3e-9 of its value (FP32
+// MFMA on tiles in LDS with the library's trigonometry: 8.3e-7 and 8.1e-9).  A round
+// of 256 chains of 32^2: 224 -> 178 us with weights of order one, 209 -> 160 with the
+// initial ones and 5% noise.
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -599,7 +601,11 @@ template <bool NEAR> __device__ __forceinline__ float ncpq_inverse(NCPq const &p
 // Adjoints of L = A (g(u) + t) - log g'(u), u = wrap(a - t), for one active
 // variable a with MLP outputs y[16] on its quad: overwrites y with dL/dy
 // (through s, w and t; the columns from NO on zero) and returns dL/da in every
-// lane of the quad.  live = false: a row without a variable, dL/dy = 0.
+// lane of the quad.  live = false: a row without a variable, dL/dy = 0.  (The
+// direction (y_8, y_9) passes dL/dt / r, r its length: a variable that the MLP leaves
+// with r of order 1e-3 carries most of a gradient's error, whatever the products'
+// rounding.  80 inputs, plaquette flow 16^2 against 64 bits: median 2.4e-7, 95% below
+// 4.0e-7, largest 1.8e-5.)
 __device__ __forceinline__ float ncpq_adjoint(NCPq const &p, float *y, float u, float A, bool live)
 {
 	const int k = threadIdx.x & 3;

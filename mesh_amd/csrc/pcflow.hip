@@ -55,8 +55,8 @@ constexpr int THREADS = 256; // of the backward kernel
 // of the eight wavefronts has a tile in a layer (V / 4 >= 8 * 16), unless the
 // launch has more workgroups than CUs and two of 256 threads fit a CU's LDS
 // (V <= PAIR_V): those run side by side without each other's barriers.  256
-// chains: sample 32^2 103 us on 256 threads, 90 on 512, 64^2 342 and 282; propose
-// (512 workgroups) 32^2 161 and 179, 64^2 772 and 617.
+// chains, initial weights with 5% noise: sample 32^2 103 us on 256 threads, 90 on 512,
+// 64^2 342 and 282; propose (512 workgroups) 32^2 161 and 179, 64^2 772 and 617.
 constexpr int WIDE_V = 512, PAIR_V = 1664;
 constexpr bool FAST = true; // tanh_fast in every kernel of this flow
 constexpr uint32_t TAG_PCFZ = 0x5043465au; // prior, holonomies, gauge
