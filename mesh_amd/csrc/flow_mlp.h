@@ -557,7 +557,7 @@ __device__ __forceinline__ float quad_max(float v)
 // evaluations.  NEAR: it also stops at |g(u) - target| <= 2.5e-7 max(1, |target|).
 // Where |target| is well below 1 that is above g's rounding: on maps whose s_k are
 // all small u can be off by 5e-4 (s_k = e^-7.5) where the iteration reaches 5e-7,
-// so only the plaquette flow, which has always used it, does.
+// so only the plaquette coupling flow, which has always used it, does.
 template <bool NEAR> __device__ __forceinline__ float ncpq_inverse(NCPq const &p, float target, float &Gp)
 {
 	float st, ct;
